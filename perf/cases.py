@@ -38,6 +38,7 @@ import lattice_amd as la  # noqa: E402
 
 PHI0, DPHI0 = 1.0093430384226378929425913902459, -0.7137133070120812430962278466136
 G2 = 2.5e5
+G2_COARSE = 2e4  # a coupling whose coarse leapfrog step (8 dt) is stable: the corrector's range
 DX = 10.0 / 256
 AMP = 1e-4  # fluctuation amplitude of fields and momenta
 U_MPL = 1.0  # reduced Planck mass of the tensor source
@@ -209,7 +210,7 @@ def _lattice(case):
                       stencil=la.STENCIL_27PT if case.get("lap") == "fd27" else la.STENCIL_7PT,
                       time_var=la.CONFORMAL if phi4 else la.COSMIC,
                       model=la.MODEL_PHI4 if phi4 else la.MODEL_TWOFIELD,
-                      model_params=(1.0,) if phi4 else (1.0, G2), gw=case["kind"] == "gw", gw_mpl=U_MPL)
+                      model_params=(1.0,) if phi4 else (1.0, case.get("g2", G2)), gw=case["kind"] == "gw", gw_mpl=U_MPL)
 
 
 def _classes(case):
@@ -230,7 +231,7 @@ def _member_case(case, n):
 
 
 def _cube(case):
-    return dict(case, nx=case["n"], ny=case["n"], nz=case["n"], model="twofield")
+    return dict(case, nx=case["n"], ny=case["n"], nz=case["n"], model="twofield", g2=G2_COARSE)
 
 
 def _layers(seed):
