@@ -37,7 +37,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short bf16;
 
-// round-to-nearest-even FP32 -> BF16 (finite inputs)
+// round-to-nearest-even FP32 -> BF16 (finite inputs).  The compiler's own
+// conversion of this instruction set gives another result for about one in
+// 1e4 activations, so host and device share the integer form.
 __host__ __device__ inline bf16 to_bf16(float f)
 {
     unsigned u = __builtin_bit_cast(unsigned, f);
@@ -69,19 +71,149 @@ enum { CONV_SILU = 0,  // Z = acc + b (BF16), Y = silu(Z) (BF16)
        CONV_LINEAR = 1, // Yf = acc + b (FP32)
        CONV_DSILU = 2 };  // Y = acc * silu'(Zin) (BF16): data gradient through the activation
 
-// Neighbour of site (x, y, z) for tap t = (dz+1)*9 + (dy+1)*3 + (dx+1).
-__device__ inline size_t nbr_site(int x, int y, int z, int t, int n)
+// Epilogue of one 16-site x 16-channel tile: the lane holds D[co0 + e][site s],
+// e = 0..3, co0 = 16 mt + 4 (lane / 16) < COUT.  Z may be null (inference: only the backward
+// pass reads the pre-activations).
+template <int COUT, int MODE>
+__device__ __forceinline__ void conv_store(const f32x4 &acc, size_t s, int co0, const float *__restrict__ bias,
+                                           bf16 *__restrict__ Y, float *__restrict__ Yf, bf16 *__restrict__ Z,
+                                           const bf16x4 &zi)
 {
-    int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-    int xx = x + dx, yy = y + dy, zz = z + dz;
-    xx = xx < 0 ? xx + n : (xx >= n ? xx - n : xx);
-    yy = yy < 0 ? yy + n : (yy >= n ? yy - n : yy);
-    zz = zz < 0 ? zz + n : (zz >= n ? zz - n : zz);
-    return (size_t)xx + (size_t)n * ((size_t)yy + (size_t)n * zz);
+    if constexpr (MODE == CONV_LINEAR) {
+        float4 o;
+        o.x = acc[0] + bias[co0];
+        o.y = acc[1] + bias[co0 + 1];
+        o.z = acc[2] + bias[co0 + 2];
+        o.w = acc[3] + bias[co0 + 3];
+        *reinterpret_cast<float4 *>(Yf + s * COUT + co0) = o;
+    } else if constexpr (MODE == CONV_SILU) {
+        bf16x4 zo, yo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = acc[e] + bias[co0 + e];
+            const bf16 zb = to_bf16(v);
+            zo[e] = (short)zb;
+            yo[e] = (short)to_bf16(silu(from_bf16(zb)));
+        }
+        if (Z) *reinterpret_cast<bf16x4 *>(Z + s * COUT + co0) = zo;
+        *reinterpret_cast<bf16x4 *>(Y + s * COUT + co0) = yo;
+    } else {
+        bf16x4 yo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) yo[e] = (short)to_bf16(acc[e] * dsilu(from_bf16((bf16)zi[e])));
+        *reinterpret_cast<bf16x4 *>(Y + s * COUT + co0) = yo;
+    }
 }
 
-// One wave per 16-site tile; CONV_WAVES waves per workgroup share the LDS
-// copy of the weights; grid-stride over tiles.
+// Convolution with 32 input channels: one K step of the MFMA is one tap.
+// A wave owns 16 sites along x of T consecutive rows y.  Per dz it holds the
+// nine taps' weight fragments in registers (from LDS, stored in fragment
+// order: conflict-free 16-byte reads) and walks the T + 2 input rows; each
+// row's three x-shifted fragments (1 KB contiguous per load, from L1 / L2)
+// feed the output rows above, at and below it, i.e. up to 6 MFMAs per load
+// instead of 2, and no address is computed per tap.  The loads of the next
+// PF rows are in flight meanwhile.  Every output accumulates its taps in
+// the order 0..26.  32 -> 32 channels at 128^3: 465 -> 162 us (716 TFLOP/s; the
+// activations in and out take about 65 us at the copy rate), 32 -> 4: 265 -> 97 us.
+constexpr int CONV32_WAVES = 4;
+template <int COUT, int MODE, int T>
+__global__ __launch_bounds__(64 * CONV32_WAVES, 2) void k_conv32(const bf16 *__restrict__ X, const bf16 *__restrict__ W,
+                                                              const float *__restrict__ bias, bf16 *__restrict__ Y,
+                                                              float *__restrict__ Yf, bf16 *__restrict__ Z,
+                                                              const bf16 *__restrict__ Zin, int n)
+{
+    constexpr int CIN = 32, MT = (COUT + 15) / 16, KP = KPAD(CIN);
+    __shared__ s16x8 ws[27 * MT * 64]; // [tap][mt][lane]
+    for (int q = threadIdx.x; q < 27 * MT * 64; q += 64 * CONV32_WAVES) {
+        const int l = q % 64, mt = q / 64 % MT, t = q / (64 * MT);
+        ws[q] = *reinterpret_cast<const s16x8 *>(W + (mt * 16 + (l & 15)) * KP + t * CIN + 8 * (l >> 4));
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane & 15, kg = lane >> 4;
+    const int ntx = n / 16, nty = n / T, ntask = ntx * nty * n;
+    // each XCD walks one contiguous eighth of the tasks (neighbouring rows and
+    // planes in the same L2)
+    const int G8 = gridDim.x >> 3, C = (ntask + 7) >> 3;
+    const int t0 = (blockIdx.x & 7) * C, t1 = min(t0 + C, ntask);
+    for (int task = t0 + (int)(blockIdx.x >> 3) * CONV32_WAVES + wave; task < t1; task += G8 * CONV32_WAVES) {
+        const int x0 = task % ntx * 16, y0 = task / ntx % nty * T, z = task / (ntx * nty);
+        int xo[3]; // element offset of the lane's fragment in a row, per dx
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+            int x = x0 + j + dx - 1;
+            x = x < 0 ? x + n : (x >= n ? x - n : x);
+            xo[dx] = x * CIN + 8 * kg;
+        }
+        constexpr int NR = T + 2, RING = NR % 5 == 0 ? 5 : 3, PF = RING - 1; // input rows per plane; fragments held
+        static_assert(NR % RING == 0, "the ring starts anew with every plane");
+        auto load_row = [&](int dz, int r, s16x8 (&b)[3]) {
+            int zz = z + dz - 1, y = y0 + r - 1;
+            zz = zz < 0 ? zz + n : (zz >= n ? zz - n : zz);
+            y = y < 0 ? y + n : (y >= n ? y - n : y);
+            const bf16 *row = X + ((size_t)zz * n + y) * n * CIN;
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx) b[dx] = *reinterpret_cast<const s16x8 *>(row + xo[dx]);
+        };
+        f32x4 acc[T][MT];
+#pragma unroll
+        for (int r = 0; r < T; ++r)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[r][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        s16x8 b[RING][3];
+#pragma unroll
+        for (int r = 0; r < PF; ++r) load_row(0, r, b[r]);
+        const size_t s0 = ((size_t)z * n + y0) * n + x0 + j;
+        bf16x4 zi[T][MT];
+#pragma unroll 1
+        for (int dz = 0; dz < 3; ++dz) {
+            s16x8 a[9][MT];
+#pragma unroll
+            for (int t = 0; t < 9; ++t)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) a[t][mt] = ws[((dz * 9 + t) * MT + mt) * 64 + lane];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                // PF rows ahead, into the next plane at the end of this one
+                if (r + PF < NR) load_row(dz, r + PF, b[(r + PF) % RING]);
+                else if (dz < 2) load_row(dz + 1, r + PF - NR, b[(r + PF) % RING]);
+                const s16x8(&c)[3] = b[r % RING];
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy) {
+                    const int ro = r - dy; // output row that sees this input row as tap row dy
+                    if (ro < 0 || ro >= T) continue;
+#pragma unroll
+                    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) acc[ro][mt] = mfma32(a[dy * 3 + dx][mt], c[dx], acc[ro][mt]);
+                }
+            }
+        }
+        if constexpr (MODE == CONV_DSILU) {
+#pragma unroll
+            for (int r = 0; r < T; ++r)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    zi[r][mt] =
+                        *reinterpret_cast<const bf16x4 *>(Zin + (s0 + (size_t)r * n) * COUT + mt * 16 + 4 * kg);
+        }
+#pragma unroll
+        for (int r = 0; r < T; ++r)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int co0 = mt * 16 + 4 * kg;
+                if (co0 >= COUT) continue;
+                conv_store<COUT, MODE>(acc[r][mt], s0 + (size_t)r * n, co0, bias, Y, Yf, Z, zi[r][mt]);
+            }
+    }
+}
+
+// Convolution with 4 or 8 input channels: a K step covers 8 or 4 taps, each lane
+// supplying one tap's 8 channels or two taps' 4.  One wave per 16-site tile
+// (within a row: n is a multiple of 16), CONV_WAVES waves per workgroup share
+// the LDS copy of the weights; grid-stride over tiles.  The lane's tap offsets
+// are the same for every tile and held in registers.  8 -> 32 at 128^3: 150 ->
+// 129 us; bound by the vector instructions of addresses and activations.
 // W: [MT*16][KP] BF16 (rows >= COUT and k >= 27*CIN are zero).
 constexpr int CONV_WAVES = 8;
 template <int CIN, int COUT, int MODE>
@@ -90,215 +222,289 @@ __global__ __launch_bounds__(64 * CONV_WAVES) void k_conv(const bf16 *__restrict
                                               float *__restrict__ Yf, bf16 *__restrict__ Z,
                                               const bf16 *__restrict__ Zin, int n)
 {
+    static_assert(CIN == 4 || CIN == 8, "narrow inputs; 32 channels: k_conv32");
     constexpr int MT = (COUT + 15) / 16;
-    constexpr int KP = KPAD(CIN);
-    __shared__ __attribute__((aligned(16))) bf16 ws[MT * 16 * KP];
-    for (int q = threadIdx.x; q < MT * 16 * KP / 8; q += 64 * CONV_WAVES)
-        reinterpret_cast<s16x8 *>(ws)[q] = reinterpret_cast<const s16x8 *>(W)[q];
+    constexpr int KP = KPAD(CIN), KS = KP / 32;
+    constexpr int TPL = 8 / CIN; // taps per lane and K step
+    __shared__ s16x8 ws[KS * MT * 64]; // [K step][mt][lane]
+    for (int q = threadIdx.x; q < KS * MT * 64; q += 64 * CONV_WAVES) {
+        const int l = q % 64, mt = q / 64 % MT, ks = q / (64 * MT);
+        ws[q] = *reinterpret_cast<const s16x8 *>(W + (mt * 16 + (l & 15)) * KP + ks * 32 + 8 * (l >> 4));
+    }
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, kg = lane >> 4;
-    const size_t nvol = (size_t)n * n * n, ntile = nvol / 16;
-    for (size_t tile = (size_t)blockIdx.x * CONV_WAVES + wave; tile < ntile;
-         tile += (size_t)gridDim.x * CONV_WAVES) {
-        const size_t s = tile * 16 + j;
-        const int x = (int)(s % n), y = (int)((s / n) % n), z = (int)(s / ((size_t)n * n));
+    int dx[KS][TPL], dy[KS][TPL], dz[KS][TPL]; // taps past the 27th: zeroed below
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int u = 0; u < TPL; ++u) {
+            const int t = (ks * 32 + 8 * kg) / CIN + u;
+            dx[ks][u] = t < 27 ? t % 3 - 1 : 0;
+            dy[ks][u] = t < 27 ? (t / 3) % 3 - 1 : 0;
+            dz[ks][u] = t < 27 ? t / 9 - 1 : 0;
+        }
+    const int ntx = n / 16;
+    const int ntile = ntx * n * n; // n <= 1024: below 2^26
+    for (int tile = (int)blockIdx.x * CONV_WAVES + wave; tile < ntile; tile += (int)gridDim.x * CONV_WAVES) {
+        const int x = tile % ntx * 16 + j, y = tile / ntx % n, z = tile / (ntx * n);
+        const size_t s = ((size_t)z * n + y) * n + x;
+        bf16x4 zi[MT];
+        if constexpr (MODE == CONV_DSILU) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                zi[mt] = *reinterpret_cast<const bf16x4 *>(Zin + s * COUT + mt * 16 + 4 * kg);
+        }
+        s16x8 b[KS];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            auto at = [&](int u) {
+                int xx = x + dx[ks][u], yy = y + dy[ks][u], zz = z + dz[ks][u];
+                xx = xx < 0 ? xx + n : (xx >= n ? xx - n : xx);
+                yy = yy < 0 ? yy + n : (yy >= n ? yy - n : yy);
+                zz = zz < 0 ? zz + n : (zz >= n ? zz - n : zz);
+                return X + ((size_t)(zz * n + yy) * n + xx) * CIN;
+            };
+            if constexpr (CIN == 8) {
+                b[ks] = *reinterpret_cast<const s16x8 *>(at(0));
+                if (4 * ks + 3 >= 27 && kg == 3) b[ks] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            } else {
+                const bf16x4 lo = *reinterpret_cast<const bf16x4 *>(at(0));
+                const bf16x4 hi = *reinterpret_cast<const bf16x4 *>(at(1));
+                b[ks] = s16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                if (8 * ks + 2 * kg + 1 >= 27) // the second tap (27, 29, 31), or both, do not exist
+                    b[ks] = 8 * ks + 2 * kg < 27 ? s16x8{lo[0], lo[1], lo[2], lo[3], 0, 0, 0, 0}
+                                                 : s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            }
+        }
         f32x4 acc[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < KP; k0 += 32) {
-            const int k = k0 + 8 * kg;
-            s16x8 b = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if constexpr (CIN % 8 == 0) {
-                const int t = k / CIN, ci = k - t * CIN;
-                if (t < 27) b = *reinterpret_cast<const s16x8 *>(X + nbr_site(x, y, z, t, n) * CIN + ci);
-            } else {
-                static_assert(CIN == 4, "4 or a multiple of 8 input channels");
-                const int t = k / 4; // taps t and t + 1, channels 0..3 of each
-                bf16x4 lo = bf16x4{0, 0, 0, 0}, hi = bf16x4{0, 0, 0, 0};
-                if (t < 27) lo = *reinterpret_cast<const bf16x4 *>(X + nbr_site(x, y, z, t, n) * 4);
-                if (t + 1 < 27) hi = *reinterpret_cast<const bf16x4 *>(X + nbr_site(x, y, z, t + 1, n) * 4);
-                b = s16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            }
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const s16x8 a = *reinterpret_cast<const s16x8 *>(ws + (mt * 16 + j) * KP + k);
-                acc[mt] = mfma32(a, b, acc[mt]);
-            }
-        }
-        // lane holds D[co][site] for co = mt*16 + 4*kg + e, site = tile*16 + j
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[mt] = mfma32(ws[(ks * MT + mt) * 64 + lane], b[ks], acc[mt]);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int co0 = mt * 16 + 4 * kg;
             if (co0 >= COUT) continue;
-            if constexpr (MODE == CONV_LINEAR) {
-                float4 o;
-                o.x = acc[mt][0] + bias[co0];
-                o.y = acc[mt][1] + bias[co0 + 1];
-                o.z = acc[mt][2] + bias[co0 + 2];
-                o.w = acc[mt][3] + bias[co0 + 3];
-                *reinterpret_cast<float4 *>(Yf + s * COUT + co0) = o;
-            } else if constexpr (MODE == CONV_SILU) {
-                bf16x4 zo, yo;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = acc[mt][e] + bias[co0 + e];
-                    const bf16 zb = to_bf16(v);
-                    zo[e] = (short)zb;
-                    yo[e] = (short)to_bf16(silu(from_bf16(zb)));
-                }
-                *reinterpret_cast<bf16x4 *>(Z + s * COUT + co0) = zo;
-                *reinterpret_cast<bf16x4 *>(Y + s * COUT + co0) = yo;
-            } else {
-                const bf16x4 zi = *reinterpret_cast<const bf16x4 *>(Zin + s * COUT + co0);
-                bf16x4 yo;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    yo[e] = (short)to_bf16(acc[mt][e] * dsilu(from_bf16((bf16)zi[e])));
-                *reinterpret_cast<bf16x4 *>(Y + s * COUT + co0) = yo;
-            }
+            conv_store<COUT, MODE>(acc[mt], s, co0, bias, Y, Yf, Z, zi[mt]);
         }
     }
 }
 
-// Weight gradient partials: one per block, nchunks(nvol) of them at most
-// (GCHUNK sites per partial), each [MT*16][KP + 16] FP32 with the bias
-// gradient in column KP.
-constexpr int GCHUNK = 4096;
+// Weight gradient dW[co][tap][ci] = sum_s G[s][co] X[s + tap][ci]: a GEMM over
+// sites (32 per MFMA, A = G^T, B = X).  A task is a chunk of CL sites along x
+// (64, 32 or 16, dividing n) of one plane z, marched over LY rows y.  Per step
+// the block stages X row r of the planes z-1, z, z+1 (one site of halo in x)
+// and G row r + 1 in LDS as they lie in memory (site-major, 16-byte copies,
+// two buffers, the rows of the step after next in flight in registers) and
+// reads them back transposed: ds_read_b64_tr_b16 gives a lane 4 consecutive
+// sites of its channel, two of them the 8 reduction indices that it supplies.
+// Wave (dz, nt) owns the nine (dy, dx) taps of plane dz and the input
+// channels 16 nt ..: one X fragment per dx meets the G rows r + 1, r, r - 1
+// (dy = 0, 1, 2; the older two kept in registers), so a step takes 6 + 4 LDS
+// reads of 512 bytes per 32 sites for 18 MFMAs.  The block sums all its tasks
+// in its accumulators and writes one partial dW (and db in column KP, from
+// G times a matrix of ones) as [MT*16][KP + 16]; k_sum_chunks adds the partials
+// in block order.  At 128^3: 32 x 32 channels 1078 -> 147 us (790 TFLOP/s),
+// 32 x 4 767 -> 97 us, 8 x 32 369 -> 77 us (the form before wrote the tiles
+// channel-major into LDS element by element and read X at odd offsets, one
+// 2-byte read per element).
+constexpr int DW_CLMAX = 64;
+constexpr int DW_BLOCKS = 512; // most partials (2 blocks per CU)
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-// Weight gradient from LDS tiles.  A block of 9 waves walks chunks of CL
-// sites along x (one row segment; CL = 64, 32 or 16, dividing n).  Per chunk
-// the X rows of the 3 x 3 (dy, dz) neighbour rows with one site of halo on
-// each side in x, and the chunk's G, are staged in LDS channel-major
-// (xs[ci][row][x], gs[co][x]), so that the 8 consecutive sites an MFMA lane
-// supplies are 8 consecutive LDS entries.  Wave w takes the tap row (dy, dz)
-// = (w % 3 - 1, w / 3 - 1) and its three dx taps: per 32 sites it loads G
-// once (A = G^T, rows co) and X shifted by dx (B, columns ci) and keeps the
-// 3 x MT x NTL accumulator tiles of its taps in registers across its chunks.
-// The block writes its partial dW (and db in column KP) as [MT*16][KP + 16];
-// the partials are summed in block order by k_sum_chunks.
-constexpr int DW2_WAVES = 9;
-constexpr int DW2_CLMAX = 64;
-constexpr int DW2_RP = DW2_CLMAX + 8;   // LDS row pitch of the X tile (halo + 16-byte multiple)
-constexpr int DW2_BLOCKS = 512;          // persistent blocks (2 per CU)
+__host__ __device__ inline int dw_chunk(int n) { return n % 64 == 0 ? 64 : (n % 32 == 0 ? 32 : 16); }
+// rows per task: as many as leave DW_BLOCKS tasks (each task recomputes two
+// halo rows), at least 8
+__host__ __device__ inline int dw_rows(int n)
+{
+    int ly = n;
+    while (ly % 2 == 0 && ly > 8 && (long long)n * (n / dw_chunk(n)) * (n / ly) < DW_BLOCKS) ly /= 2;
+    return ly;
+}
+__host__ __device__ inline int dw_tasks(int n) { return n * (n / dw_chunk(n)) * (n / dw_rows(n)); }
+static int dw_blocks(int n) { return dw_tasks(n) < DW_BLOCKS ? dw_tasks(n) : DW_BLOCKS; }
+template <int CIN>
+constexpr int dw_waves() { return 3 * ((CIN + 15) / 16); }
 
-__device__ inline int dw2_chunk(int n) { return n % 64 == 0 ? 64 : (n % 32 == 0 ? 32 : 16); }
+// four reduction indices of this lane's channel: within a group of 16 lanes,
+// lane 4 r + c points at channels 4 c .. 4 c + 3 of site r; lane i gets channel i of sites 0..3
+__device__ __forceinline__ s16x4 lds_tr(const bf16 *p)
+{
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(p));
+}
+__device__ __forceinline__ s16x8 join(s16x4 a, s16x4 b) { return s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 
-template <int CIN, int COUT>
-__global__ __launch_bounds__(64 * DW2_WAVES) void k_conv_dw2(const bf16 *__restrict__ G, const bf16 *__restrict__ X,
-                                                             float *__restrict__ part, int n)
+template <int CIN, int COUT, int CL>
+__global__ __launch_bounds__(64 * dw_waves<CIN>(), 2) void k_conv_dw(const bf16 *__restrict__ G, const bf16 *__restrict__ X,
+                                                                  float *__restrict__ part, int n, int LY, int ntask)
 {
     constexpr int MT = (COUT + 15) / 16, NTL = (CIN + 15) / 16;
     constexpr int KP = KPAD(CIN), LD = KP + 16;
-    constexpr int NT = 64 * DW2_WAVES;
-    // channel rows padded to whole 16-row tiles; rows >= CIN / COUT stay zero
-    __shared__ __attribute__((aligned(16))) bf16 xs[NTL * 16][9][DW2_RP];
-    __shared__ __attribute__((aligned(16))) bf16 gs[MT * 16][DW2_CLMAX];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NT = 64 * dw_waves<CIN>();
+    constexpr int KS = (CL + 31) / 32;
+    // staged rows: X [3][CL + 2][CIN], then G [CL][COUT]; 16-byte copies
+    constexpr int XE = 3 * (CL + 2) * CIN, GE = CL * COUT, BUF = XE + GE;
+    constexpr int XI = XE / 8, GI = GE / 8, NI = cdiv(XI + GI, NT);
+    static_assert(XE % 8 == 0 && GE % 8 == 0 && CL % 16 == 0, "16-byte items");
+    __shared__ __attribute__((aligned(16))) bf16 lds[2 * BUF];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, kg = lane >> 4;
-    const int dy = wave % 3 - 1, dz = wave / 3 - 1;
-    const int row = (dz + 1) * 3 + (dy + 1);
-    const int CL = dw2_chunk(n);
-    const int KS = (CL + 31) / 32;
-    const size_t nvol = (size_t)n * n * n;
-    const int nchunk = (int)(nvol / CL);
-    for (int q = threadIdx.x; q < NTL * 16 * 9 * DW2_RP; q += NT) (&xs[0][0][0])[q] = 0;
-    for (int q = threadIdx.x; q < MT * 16 * DW2_CLMAX; q += NT) (&gs[0][0])[q] = 0;
-    f32x4 acc[3][MT][NTL];
+    const int dz = wave % 3, nt = wave / 3;
+    // the lane's part of a transposed read: site 8 kg + 4 h + lr, channels lc ..; a tensor
+    // with fewer channels than 16 is read at its own (columns past the last are not used)
+    const int lr = (lane & 15) >> 2, lc = (lane & 3) * 4;
+    const int xc = CIN < 16 ? lc % CIN : nt * 16 + lc;
+    const bool half = CL == 16 && kg >= 2; // a 16-site chunk fills half of a K step
+    const int sk = half ? 8 * kg - 16 + lr : 8 * kg + lr;
+    f32x4 acc[3][3][MT], accb[MT];
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int mt = 0; mt < MT; ++mt) {
+        accb[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int d = 0; d < 9; ++d) acc[d / 3][d % 3][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const s16x8 zero8 = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    const short one = (short)0x3f80; // 1.0 in BF16
+    const s16x8 ones = s16x8{one, one, one, one, one, one, one, one};
+    const int ntx = n / CL, nly = n / LY;
+    for (int task = blockIdx.x; task < ntask; task += gridDim.x) {
+        const int x0 = task % ntx * CL, y0 = task / ntx % nly * LY, z = task / (ntx * nly);
+        // the thread's staged items: row-independent element offsets
+        size_t off[NI];
+        auto isx = [&](int i) { return (int)threadIdx.x + i * NT < XI; };
+        auto ok = [&](int i) { return (int)threadIdx.x + i * NT < XI + GI; };
 #pragma unroll
-            for (int nt = 0; nt < NTL; ++nt) acc[d][mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float db = 0.f; // bias gradient of channel co = threadIdx.x (< COUT)
-    __syncthreads();
-    for (int ch = blockIdx.x; ch < nchunk; ch += gridDim.x) {
-        const size_t s0 = (size_t)ch * CL;
-        const int x0 = (int)(s0 % n), y = (int)((s0 / n) % n), z = (int)(s0 / ((size_t)n * n));
-        // stage X: 9 rows x (CL + 2) sites x CIN channels, 4 channels (8 bytes) per item
-        constexpr int C4 = CIN / 4;
-        for (int q = threadIdx.x; q < 9 * (CL + 2) * C4; q += NT) {
-            const int c4 = q % C4, rest = q / C4;
-            const int xi = rest % (CL + 2), r = rest / (CL + 2);
-            int xx = x0 + xi - 1, yy = y + r % 3 - 1, zz = z + r / 3 - 1;
-            xx = xx < 0 ? xx + n : (xx >= n ? xx - n : xx);
-            yy = yy < 0 ? yy + n : (yy >= n ? yy - n : yy);
-            zz = zz < 0 ? zz + n : (zz >= n ? zz - n : zz);
-            const size_t site = (size_t)xx + (size_t)n * ((size_t)yy + (size_t)n * zz);
-            const bf16x4 v = *reinterpret_cast<const bf16x4 *>(X + site * CIN + 4 * c4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) xs[4 * c4 + e][r][xi] = (bf16)v[e];
-        }
-        // stage G: CL sites x COUT channels
-        constexpr int O4 = COUT / 4;
-        for (int q = threadIdx.x; q < CL * O4; q += NT) {
-            const int o4 = q % O4, xi = q / O4;
-            const bf16x4 v = *reinterpret_cast<const bf16x4 *>(G + (s0 + xi) * COUT + 4 * o4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) gs[4 * o4 + e][xi] = (bf16)v[e];
-        }
-        __syncthreads();
-        if (threadIdx.x < COUT) {
-            for (int xi = 0; xi < CL; ++xi) db += from_bf16(gs[threadIdx.x][xi]);
-        }
-        for (int ks = 0; ks < KS; ++ks) {
-            // first of the lane's 8 sites within the chunk; at CL = 16 the upper
-            // half of the K step holds no sites and supplies zeros
-            const int xk = 32 * ks + 8 * kg;
-            s16x8 a[MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                a[mt] = xk < CL ? *reinterpret_cast<const s16x8 *>(&gs[mt * 16 + j][xk]) : s16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-#pragma unroll
-                for (int nt = 0; nt < NTL; ++nt) {
-                    s16x8 b;
-                    const bf16 *src = &xs[nt * 16 + j][row][xk + d]; // site x0 + xk + q + (d - 1), halo at 0
-#pragma unroll
-                    for (int qq = 0; qq < 8; ++qq) b[qq] = xk < CL ? (short)src[qq] : (short)0;
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) acc[d][mt][nt] = mfma32(a[mt], b, acc[d][mt][nt]);
-                }
+        for (int i = 0; i < NI; ++i) {
+            const int q = threadIdx.x + i * NT;
+            if (isx(i)) {
+                constexpr int C8 = CIN / 8;
+                const int c = q % C8, rest = q / C8, xi = rest % (CL + 2), p = rest / (CL + 2);
+                int x = x0 + xi - 1, zz = z + p - 1;
+                x = x < 0 ? x + n : (x >= n ? x - n : x);
+                zz = zz < 0 ? zz + n : (zz >= n ? zz - n : zz);
+                off[i] = ((size_t)zz * n * n + x) * CIN + 8 * c;
+            } else {
+                off[i] = ((size_t)z * n * n + x0) * COUT + 8 * (size_t)(q - XI);
             }
         }
+        // step s: X row y0 - 1 + s, G row y0 + s (zero past the task's rows)
+        s16x8 v[NI];
+        auto fetch = [&](int s) {
+            int yx = y0 - 1 + s;
+            yx = yx < 0 ? yx + n : (yx >= n ? yx - n : yx);
+            const size_t rx = (size_t)yx * n * CIN, rg = (size_t)(y0 + s) * n * COUT;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                v[i] = zero8;
+                if (isx(i)) v[i] = *reinterpret_cast<const s16x8 *>(X + off[i] + rx);
+                else if (ok(i) && s < LY) v[i] = *reinterpret_cast<const s16x8 *>(G + off[i] + rg);
+            }
+        };
+        auto stage = [&](int s) {
+            bf16 *b = lds + (s & 1) * BUF;
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                if (ok(i)) *reinterpret_cast<s16x8 *>(b + 8 * ((size_t)threadIdx.x + i * NT)) = v[i];
+        };
+        s16x8 g[3][KS][MT]; // G rows r + 1, r, r - 1 in rotation
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) g[u][ks][mt] = zero8;
+        auto step = [&](int s, s16x8 (&gn)[KS][MT], const s16x8 (&g1)[KS][MT], const s16x8 (&g2)[KS][MT]) {
+            if (s + 1 < LY + 2) stage(s + 1);
+            if (s + 2 < LY + 2) fetch(s + 2);
+            const bf16 *xb = lds + (s & 1) * BUF + dz * (CL + 2) * CIN, *gb = lds + (s & 1) * BUF + XE;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const bf16 *p = gb + (32 * ks + sk) * COUT + (COUT < 16 ? lc % COUT : mt * 16 + lc);
+                    gn[ks][mt] = join(lds_tr(p), lds_tr(p + 4 * COUT));
+                    if (half) gn[ks][mt] = zero8;
+                    if (wave == 0) accb[mt] = mfma32(gn[ks][mt], ones, accb[mt]);
+                }
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx) {
+                    const bf16 *p = xb + (32 * ks + sk + dx) * CIN + xc;
+                    const s16x8 b = join(lds_tr(p), lds_tr(p + 4 * CIN));
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) {
+                        acc[0][dx][mt] = mfma32(gn[ks][mt], b, acc[0][dx][mt]);
+                        acc[1][dx][mt] = mfma32(g1[ks][mt], b, acc[1][dx][mt]);
+                        acc[2][dx][mt] = mfma32(g2[ks][mt], b, acc[2][dx][mt]);
+                    }
+                }
+            }
+            __syncthreads();
+        };
+        fetch(0);
+        stage(0);
+        fetch(1);
         __syncthreads();
+        int s = 0;
+        for (; s + 2 < LY + 2; s += 3) {
+            step(s, g[0], g[1], g[2]);
+            step(s + 1, g[2], g[0], g[1]);
+            step(s + 2, g[1], g[2], g[0]);
+        }
+        if (s < LY + 2) step(s, g[0], g[1], g[2]);
+        if (s + 1 < LY + 2) step(s + 1, g[2], g[0], g[1]);
     }
-    // D[row co = mt*16 + 4*kg + e][col ci = nt*16 + j] of tap t = (dz+1)*9 + (dy+1)*3 + d
+    // D[row co = mt*16 + 4*kg + e][col ci = nt*16 + j] of tap t = dz*9 + dy*3 + dx
     float *dst = part + (size_t)blockIdx.x * (MT * 16) * LD;
+    const int ci = nt * 16 + j;
+    if (ci < CIN) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const int t = (dz + 1) * 9 + (dy + 1) * 3 + d;
+        for (int d = 0; d < 9; ++d)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NTL; ++nt) {
-                const int ci = nt * 16 + j;
-                if (ci >= CIN) continue;
+            for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int co = mt * 16 + 4 * kg + e;
-                    dst[(size_t)co * LD + t * CIN + ci] = co < COUT ? acc[d][mt][nt][e] : 0.f;
+                    dst[(size_t)co * LD + (dz * 9 + d) * CIN + ci] = co < COUT ? acc[d / 3][d % 3][mt][e] : 0.f;
                 }
-            }
     }
     // padding columns 27 CIN .. KP-1 and the bias block KP .. KP+15
     for (int q = threadIdx.x; q < MT * 16 * (LD - 27 * CIN); q += NT) {
         const int co = q / (LD - 27 * CIN), k = 27 * CIN + q % (LD - 27 * CIN);
         if (!(k == KP && co < COUT)) dst[(size_t)co * LD + k] = 0.f;
     }
-    if (threadIdx.x < COUT) dst[(size_t)threadIdx.x * LD + KP] = db;
+    if (wave == 0 && j == 0) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int co = mt * 16 + 4 * kg + e;
+                if (co < COUT) dst[(size_t)co * LD + KP] = accb[mt][e];
+            }
+    }
 }
 
-// out[q] = sum over chunks (in order) of part[chunk][q]
-__global__ __launch_bounds__(256) void k_sum_chunks(const float *__restrict__ part, int nchunk, int nq,
-                                                    float *__restrict__ out)
+// out[q] = sum over chunks of part[chunk][q]: SUM_LANES threads per q take
+// every SUM_LANES-th chunk, in order, and are added in order (512 chunks of a
+// 32 x 32 layer: 129 us with one thread per q, 8.7 us).
+constexpr int SUM_LANES = 8, SUM_Q = 32;
+__global__ __launch_bounds__(SUM_LANES *SUM_Q) void k_sum_chunks(const float *__restrict__ part, int nchunk, int nq,
+                                                                 float *__restrict__ out)
 {
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= nq) return;
+    __shared__ float red[SUM_LANES][SUM_Q];
+    const int lq = threadIdx.x % SUM_Q, lane = threadIdx.x / SUM_Q;
+    const int q = blockIdx.x * SUM_Q + lq;
     float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * nq + q];
+    if (q < nq)
+#pragma unroll 8
+        for (int c = lane; c < nchunk; c += SUM_LANES) s += part[(size_t)c * nq + q];
+    red[lane][lq] = s;
+    __syncthreads();
+    if (lane || q >= nq) return;
+#pragma unroll
+    for (int l = 1; l < SUM_LANES; ++l) s += red[l][lq];
     out[q] = s;
 }
 
@@ -437,8 +643,6 @@ static void free_buffers(Net &net)
     net.n = 0;
 }
 
-static size_t nchunks(size_t nvol) { return (nvol + GCHUNK - 1) / GCHUNK; }
-
 static int ensure_buffers(Net &net, const Ctx &c)
 {
     if (net.n == c.nx) return 0;
@@ -460,7 +664,7 @@ static int ensure_buffers(Net &net, const Ctx &c)
         const size_t q = (size_t)net.L[l].mp * (net.L[l].kp + 16);
         maxpart = q > maxpart ? q : maxpart;
     }
-    rc |= alloc(net, &net.part, maxpart * nchunks(nv), "dW partials");
+    rc |= alloc(net, &net.part, maxpart * dw_blocks(c.nx), "dW partials");
     rc |= alloc(net, &net.lossp, 1024, "loss partials");
     rc |= alloc(net, &net.cm, CM_SLOTS, "channel statistics");
     rc |= alloc(net, &net.cpart, 4 * CM_BLOCKS, "channel-mean partials");
@@ -535,13 +739,18 @@ __global__ __launch_bounds__(256) void k_chsum(const double *__restrict__ f, con
 
 // out[c] = sum / nvol, or with root the standard deviation sqrt(sum / nvol)
 // (root 1: 1 where it is 0, so a channel without fluctuations is left
-// unscaled; root 2: the RMS as it is)
+// unscaled; root 2: the RMS as it is).  One wave: lane 4 b + c takes every 16th partial of
+// channel c, in order, and the 16 are added by shuffles (4 threads walking all
+// 512 partials took 62 us of load latency; now 4.4 us).
 __global__ __launch_bounds__(64) void k_chmean(const double *__restrict__ part, int nb, size_t nvol, int root,
                                                double *__restrict__ out)
 {
+    double t = 0;
+#pragma unroll 8
+    for (int q = threadIdx.x; q < 4 * nb; q += 64) t += part[q];
+#pragma unroll
+    for (int m = 4; m < 64; m <<= 1) t += __shfl_xor(t, m, 64);
     if (threadIdx.x < 4) {
-        double t = 0;
-        for (int b = 0; b < nb; ++b) t += part[b * 4 + threadIdx.x];
         t /= (double)nvol;
         if (root) {
             t = sqrt(t);
@@ -635,40 +844,62 @@ __global__ __launch_bounds__(256) void k_apply(double *__restrict__ f, double *_
 }
 
 // ---------------------------------------------------------------- network passes
+// Rows per wave of the 32-channel convolution: 8, or 4 where 8 would leave
+// SIMDs idle (fewer wave tasks than the device's 4 x 256 SIMDs: n <= 48).
+// Per launch, 32 -> 32, T = 8 / 4: 16^3 16.0 / 11.2 us, 32^3 16.7 / 12.2, 48^3
+// 20.1 / 18.9; 64^3 and 96^3 together 67.7 / 75.2.
 template <int CIN, int COUT, int MODE>
 static void conv(Net &net, const bf16 *X, const bf16 *W, const float *bias, bf16 *Y, float *Yf, bf16 *Z,
                  const bf16 *Zin)
 {
     const size_t ntile = (size_t)net.n * net.n * net.n / 16;
-    size_t g = (ntile + CONV_WAVES - 1) / CONV_WAVES;
-    if (g > 4096) g = 4096;
-    hipLaunchKernelGGL((k_conv<CIN, COUT, MODE>), dim3((unsigned)g), dim3(64 * CONV_WAVES), 0, net.stream, X, W, bias,
-                       Y, Yf, Z, Zin, net.n);
+    if constexpr (CIN == 32) {
+        const bool wide = ntile / 8 >= 1024;
+        size_t g = (ntile / (wide ? 8 : 4) + CONV32_WAVES - 1) / CONV32_WAVES;
+        g = g > 512 ? 512 : (g + 7) / 8 * 8;
+        if (wide)
+            hipLaunchKernelGGL((k_conv32<COUT, MODE, 8>), dim3((unsigned)g), dim3(64 * CONV32_WAVES), 0, net.stream,
+                               X, W, bias, Y, Yf, Z, Zin, net.n);
+        else
+            hipLaunchKernelGGL((k_conv32<COUT, MODE, 4>), dim3((unsigned)g), dim3(64 * CONV32_WAVES), 0, net.stream,
+                               X, W, bias, Y, Yf, Z, Zin, net.n);
+    } else {
+        size_t g = (ntile + CONV_WAVES - 1) / CONV_WAVES;
+        if (g > 4096) g = 4096;
+        hipLaunchKernelGGL((k_conv<CIN, COUT, MODE>), dim3((unsigned)g), dim3(64 * CONV_WAVES), 0, net.stream, X, W,
+                           bias, Y, Yf, Z, Zin, net.n);
+    }
 }
 
-static void forward(Net &net)
+// train: keep the pre-activations for the backward pass
+static void forward(Net &net, bool train)
 {
-    conv<NIN, WID, CONV_SILU>(net, net.x0, net.L[0].wb, net.L[0].b, net.a[0], nullptr, net.z[0], nullptr);
-    conv<WID, WID, CONV_SILU>(net, net.a[0], net.L[1].wb, net.L[1].b, net.a[1], nullptr, net.z[1], nullptr);
-    conv<WID, WID, CONV_SILU>(net, net.a[1], net.L[2].wb, net.L[2].b, net.a[2], nullptr, net.z[2], nullptr);
+    bf16 *z[3];
+    for (int q = 0; q < 3; ++q) z[q] = train ? net.z[q] : nullptr;
+    conv<NIN, WID, CONV_SILU>(net, net.x0, net.L[0].wb, net.L[0].b, net.a[0], nullptr, z[0], nullptr);
+    conv<WID, WID, CONV_SILU>(net, net.a[0], net.L[1].wb, net.L[1].b, net.a[1], nullptr, z[1], nullptr);
+    conv<WID, WID, CONV_SILU>(net, net.a[1], net.L[2].wb, net.L[2].b, net.a[2], nullptr, z[2], nullptr);
     conv<WID, 4, CONV_LINEAR>(net, net.a[2], net.L[3].wb, net.L[3].b, nullptr, net.y, nullptr, nullptr);
 }
 
 template <int CIN, int COUT>
 static void weight_grad(Net &net, Layer &l, const bf16 *G, const bf16 *X)
 {
-    const size_t nv = (size_t)net.n * net.n * net.n;
-    const int MT = (COUT + 15) / 16, CT = KPAD(CIN) / 16 + 1;
-    // one partial per block: at most the nchunks(nv) partials net.part holds
-    size_t nch = nchunks(nv);
-    if (nch > DW2_BLOCKS) nch = DW2_BLOCKS;
-    (void)MT;
-    (void)CT;
-    hipLaunchKernelGGL((k_conv_dw2<CIN, COUT>), dim3((unsigned)nch), dim3(64 * DW2_WAVES), 0, net.stream, G, X,
-                       net.part, net.n);
+    const int nb = dw_blocks(net.n), ly = dw_rows(net.n), nt = dw_tasks(net.n);
+    const dim3 blk(64 * dw_waves<CIN>());
+    switch (dw_chunk(net.n)) {
+    case 64:
+        hipLaunchKernelGGL((k_conv_dw<CIN, COUT, 64>), dim3(nb), blk, 0, net.stream, G, X, net.part, net.n, ly, nt);
+        break;
+    case 32:
+        hipLaunchKernelGGL((k_conv_dw<CIN, COUT, 32>), dim3(nb), blk, 0, net.stream, G, X, net.part, net.n, ly, nt);
+        break;
+    default:
+        hipLaunchKernelGGL((k_conv_dw<CIN, COUT, 16>), dim3(nb), blk, 0, net.stream, G, X, net.part, net.n, ly, nt);
+    }
     const int nq = l.mp * (l.kp + 16);
-    hipLaunchKernelGGL(k_sum_chunks, dim3((nq + 255) / 256), dim3(256), 0, net.stream, net.part, (int)nch, nq,
-                       l.grad);
+    hipLaunchKernelGGL(k_sum_chunks, dim3((nq + SUM_Q - 1) / SUM_Q), dim3(SUM_LANES * SUM_Q), 0, net.stream, net.part,
+                       nb, nq, l.grad);
 }
 
 // output gradient G4 and the loss partials for the current y / tgt
@@ -939,7 +1170,7 @@ int lat_corrector_infer(lat_corrector *h, lat_ctx *ctx, float *out)
     int rc = check_ctx(net, c);
     if (rc) return rc;
     pack(net, c, c.fld, c.fldp);
-    forward(net);
+    forward(net, false);
     LAT_HIP(&c, hipMemcpyAsync(out, net.y, sizeof(float) * 4 * c.nvol, hipMemcpyDeviceToHost, c.stream));
     LAT_HIP(&c, hipStreamSynchronize(c.stream));
     return 0;
@@ -959,7 +1190,7 @@ int lat_corrector_gradients(lat_corrector *h, lat_ctx *ctx, const float *target,
     if (rc) return rc;
     LAT_HIP(&c, hipMemcpyAsync(net.tgt, target, sizeof(float) * 4 * c.nvol, hipMemcpyHostToDevice, c.stream));
     pack(net, c, c.fld, c.fldp);
-    forward(net);
+    forward(net, true);
     backward(net);
     std::vector<float> lp(1024);
     LAT_HIP(&c, hipMemcpyAsync(lp.data(), net.lossp, sizeof(float) * 1024, hipMemcpyDeviceToHost, c.stream));
@@ -1038,7 +1269,7 @@ int lat_corrector_train(lat_corrector *h, lat_ctx *ctx, double dt, int coarse_fa
         hipLaunchKernelGGL(k_target, dim3(grid_sites(c.nvol)), dim3(256), 0, c.stream, (const double *)c.fld,
                            (const double *)c.fldp, (const double *)net.coarse_f, (const double *)net.coarse_p,
                            c.nvol, (const double *)net.cm, d4(net.ratio), net.tgt);
-        forward(net);
+        forward(net, true);
         loss_grad(net);
         std::vector<float> lp(1024);
         LAT_HIP(&c, hipMemcpyAsync(lp.data(), net.lossp, sizeof(float) * 1024, hipMemcpyDeviceToHost, c.stream));
@@ -1081,7 +1312,7 @@ int lat_corrector_step(lat_corrector *h, lat_ctx *ctx, double dt, int coarse_fac
         if ((rc = save_state(net, c))) return rc;
         if ((rc = lat_symp(ctx, 2, coarse_factor * dt, 1))) return rc;
         pack(net, c, c.fld, c.fldp);
-        forward(net);
+        forward(net, false);
         channel_means(net, c, nullptr, nullptr, nullptr, nullptr, net.y, 2);
         hipLaunchKernelGGL(k_apply, dim3(grid_sites(c.nvol)), dim3(256), 0, c.stream, (double *)c.fld,
                            (double *)c.fldp, net.y, c.nvol, (const double *)net.cm, d4(net.ratio));
@@ -1165,7 +1396,7 @@ int lat_corrector_step_judged(lat_corrector *h, lat_ctx *ctx, double dt, int coa
             LAT_HIP(&c, hipMemcpyAsync(net.leap_p, c.fldp, bytes, hipMemcpyDeviceToDevice, c.stream));
         }
         pack(net, c, c.fld, c.fldp);
-        forward(net);
+        forward(net, false);
         channel_means(net, c, nullptr, nullptr, nullptr, nullptr, net.y, 2);
         hipLaunchKernelGGL(k_apply, dim3(grid_sites(c.nvol)), dim3(256), 0, c.stream, (double *)c.fld,
                            (double *)c.fldp, net.y, c.nvol, (const double *)net.cm, d4(net.ratio));

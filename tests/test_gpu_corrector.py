@@ -132,6 +132,37 @@ def test_corrector_gradients_match_torch(gpu):
         assert cos > 0.998, li
 
 
+@pytest.mark.parametrize("n", [32, 48, 64])
+def test_corrector_layers_at_other_sizes(gpu, n):
+    """Forward and gradients where the kernels split the lattice differently:
+    chunks of 16, 32 and 64 sites, 4 and 8 rows per wave, tasks of 8 to 12 rows
+    (rows per task other than a power of two at 48).  Bounds as at 16^3."""
+    print("case corrector sizes", n, flush=True)
+    L = 10.0
+    rng = np.random.default_rng(n)
+    fld, fldp = state(n, L, 6)
+    layers = random_layers(rng, scale=0.5)
+    target = (rng.standard_normal((n, n, n, 4)) * 0.5).astype(np.float32)
+    with gpu.Lattice(n, nfld=2, length=L, model_params=(1.0, 1e4)) as lat, gpu.Corrector(3) as corr:
+        lat.set_state(fld, fldp, 1.0, 0.0)
+        for li, (w, b) in enumerate(layers):
+            corr.set_layer(li, w, b)
+        corr.set_norm(np.ones(4))
+        infer = corr.infer(lat)
+        loss, grads = corr.gradients(lat, target)
+    out, params = torch_forward(packed_input(fld, fldp, 1e4), layers)
+    tl = ((out - torch.from_numpy(target)) ** 2).mean()
+    tl.backward()
+    ref = out.detach().numpy()
+    assert np.linalg.norm(infer - ref) < 2e-2 * np.linalg.norm(ref)
+    assert abs(loss - tl.item()) < 1e-2 * tl.item()
+    for li, ((W, B), (gw, gb)) in enumerate(zip(params, grads)):
+        cout, _, cin = gw.shape
+        ref_w = W.grad.numpy().transpose(0, 2, 3, 4, 1).reshape(cout, 27, cin)
+        assert np.linalg.norm(gw - ref_w) < 5e-2 * np.linalg.norm(ref_w), li
+        assert np.linalg.norm(gb - B.grad.numpy()) < 5e-2 * np.linalg.norm(B.grad.numpy()), li
+
+
 def test_corrector_training_and_fallback(gpu):
     """Training on integrator pairs lowers the loss; a zero threshold makes
     every step fall back to the plain integrator, reproducing Yoshida-4."""
