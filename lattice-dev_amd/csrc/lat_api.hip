@@ -234,16 +234,21 @@ static int state_force(Ctx &c, bool drift, int epi)
         }
     }
     if (c.cfg.laplacian == LAT_LAP_STENCIL) {
-        if (drift) {
+        const bool fuse = drift && c.fd_fuse;
+        if (drift && !fuse) {
             int rc = launch_drift<T>(c);
             if (rc) return rc;
         }
         int g;
         {
             StageTimer st(c, LAT_ST_STENCIL);
-            g = launch_stencil<T>(c, epi);
+            g = epi == EPI_KICK ? launch_fd_kick<T>(c, fuse) : launch_fd_reduce<T>(c);
         }
         if (g < 0) return g;
+        if (fuse) {
+            std::swap(c.fld, c.fld2);
+            std::swap(c.fldp, c.fldp2);
+        }
         if (gw) {
             int rc = gw_kick<T>(c, drift);
             if (rc) return rc;
@@ -352,8 +357,38 @@ static int build_symp(const Ctx &c, std::vector<Op> &ops, int order, double dt, 
 // drifts' and grav steps' scalar parts, and computes the next kick's
 // coefficients; the drifts' field updates are fused into the next x-R2C sweep
 // (spectral) or run as one drift sweep (stencil, end of sequence).
+// Finite-difference contexts with second state arrays take drift and kick in
+// one sweep that swaps the state's arrays.  The state is in its own arrays
+// between calls (views, lat_device_state and captured graphs hold their
+// addresses), so an odd number of such kicks runs the first one as a drift
+// sweep and a kick in place.
+struct FdHome {
+    Ctx &c;
+    void *const f, *const p;
+    explicit FdHome(Ctx &cc) : c(cc), f(cc.fld), p(cc.fldp) {}
+    ~FdHome() // (an error in between)
+    {
+        c.fd_fuse = false;
+        if (c.fld != f) std::swap(c.fld, c.fld2);
+        if (c.fldp != p) std::swap(c.fldp, c.fldp2);
+    }
+};
+
 static int run_ops(Ctx &c, const std::vector<Op> &ops)
 {
+    FdHome home(c);
+    bool unfused = false; // one kick is left to run unfused
+    if (c.fld2) {
+        int nd = 0;
+        for (const Op &op : ops) {
+            if (op.type == OP_KICK) {
+                if (nd > 0) unfused = !unfused;
+                nd = 0;
+            } else if (op.type == OP_DRIFT) {
+                nd = nd == 2 ? 1 : nd + 1; // (two at most are pending, see below)
+            }
+        }
+    }
     int npart = 0;
     if (!get_ke_valid(c)) {
         npart = c.prec == LAT_F64 ? launch_reduce_state<double>(c) : launch_reduce_state<float>(c);
@@ -387,7 +422,10 @@ static int run_ops(Ctx &c, const std::vector<Op> &ops)
             so.h[so.n++] = op.h;
             int rc = launch_scalar(c, so, npart);
             if (rc) return rc;
+            c.fd_fuse = c.fld2 && ndrift > 0 && !unfused;
+            if (ndrift > 0) unfused = false;
             int g = force(c, ndrift > 0, EPI_KICK);
+            c.fd_fuse = false;
             if (g < 0) return g;
             npart = g;
             ndrift = 0;
@@ -650,6 +688,20 @@ static int create_ctx(const lat_config *cfg, int B, const double *mparams, lat_c
         rc |= ensure(c, &c.gwp, es * 6 * c.nvol, "hipMalloc gwp");
         if (cfg->laplacian == LAT_LAP_SPECTRAL) rc |= ensure(c, &c.gwsrc, es * 2 * c.nvol, "hipMalloc gwsrc");
     }
+    if (cfg->laplacian == LAT_LAP_STENCIL && !c.gw) {
+        // second state arrays of the fused drift + kick sweep, where they
+        // leave half of the device's memory free; without them the drift is
+        // a sweep of its own
+        const size_t bytes = es * B * c.ms.f;
+        size_t fr = 0, tot = 0;
+        if (hipMemGetInfo(&fr, &tot) == hipSuccess && fr > 2 * bytes + tot / 2 &&
+            hipMalloc(&c.fld2, bytes) == hipSuccess && hipMalloc(&c.fldp2, bytes) != hipSuccess) {
+            (void)hipFree(c.fld2);
+            c.fld2 = nullptr;
+        }
+        (void)hipGetLastError();
+        if (!c.fld2) c.fldp2 = nullptr;
+    }
     rc |= ensure(c, (void **)&c.dsc, sizeof(DevScalars) * B, "hipMalloc dsc");
     rc |= ensure(c, (void **)&c.partials, sizeof(double) * MAX_GRID * NRED * B, "hipMalloc partials");
     if (rc) { lat_destroy(h); return -3; }
@@ -768,7 +820,7 @@ void lat_destroy(lat_ctx *h)
     }
     (void)hipSetDevice(c.device);
     if (c.stream) (void)hipStreamSynchronize(c.stream);
-    void *ptrs[] = {c.fld, c.fldp, c.Fk, c.Fk2, c.io64, (c.Fk64 != c.Fk) ? c.Fk64 : nullptr, c.dsc, c.partials,
+    void *ptrs[] = {c.fld, c.fldp, c.fld2, c.fldp2, c.Fk, c.Fk2, c.io64, (c.Fk64 != c.Fk) ? c.Fk64 : nullptr, c.dsc, c.partials,
                     c.spec_part, c.spec_out, c.twx64, c.twy64, c.twz64, c.twx32, c.twy32, c.twz32,
                     c.gwu, c.gwp, c.gwsrc, c.gwk, c.lap, c.disc_part};
     for (void *p : ptrs)

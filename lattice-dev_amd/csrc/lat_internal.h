@@ -18,6 +18,12 @@ constexpr int MAX_GRID = 8192; // most reduction partials (blocks) per member of
 constexpr int GRID_CAP = 4096; // default cap of grid-stride launches
 constexpr int NRED = 8;        // reduction channels per partial
 
+// 16-byte vector of reals (4 floats or 2 doubles) for vector loads/stores.
+template <typename T>
+struct alignas(16) Vec16 {
+    T e[16 / sizeof(T)];
+};
+
 // Reduction channels written by the sweep kernels (FP64 partial per block).
 // FP64 form: sums of the full fields.  Mixed form: sums of the fluctuations
 // (GE uses dphi, PE is the sum of V(phi) - V(mean)).
@@ -117,6 +123,11 @@ struct Ctx {
     int device;
 
     void *fld, *fldp;       // nfld * nvol of T (state)
+    // second state arrays of a finite-difference context (nullptr: none): the
+    // fused drift + kick sweeps write the new state there and run_ops swaps
+    // the two, an even number of times per call
+    void *fld2 = nullptr, *fldp2 = nullptr;
+    bool fd_fuse = false;   // the kick being run takes the fused sweep
     void *Fk;               // nfld * nk of cpx<T>
     void *Fk2;              // nk of cpx<T>, spectra second operand
     double *io64;           // nvol doubles: host-interface staging (FP64)
@@ -218,8 +229,11 @@ template <typename T>
 int launch_gw_stencil_kick(Ctx &c);    // FD: pi_u += hA (stencil lap u + gw_coup S)
 template <typename T>
 int launch_reduce_state(Ctx &c);        // partials: PE, KE, means (no Laplacian)
+// FD kick; drift: the pending drifts first, phi' and pi' into fld2 and fldp2
 template <typename T>
-int launch_stencil(Ctx &c, int epi);    // FD Laplacian + kick / reduce epilogue
+int launch_fd_kick(Ctx &c, bool drift);
+template <typename T>
+int launch_fd_reduce(Ctx &c);           // FD Laplacian and reductions of the state
 int launch_scalar(Ctx &c, const ScalarOps &ops, int npart);
 int grid_for(int tiles, int cap = GRID_CAP);
 

@@ -254,8 +254,6 @@ int launch_reduce_state(Ctx &c)
 // wrap_fields, hamiltonian_conformal.f90:309-330); the a-dependence of the
 // reference's b-coefficients (hamiltonian_conformal.f90:177-179,
 // hamiltonian_cosmic.f90:185-187) lives in the kick coefficients hA.
-// EPI_KICK: pi += hA lap - hB V', reduce GE, PE, KE'.  EPI_REDUCE: reduce only.
-// EPI_STORE: write lap_raw of field 0 into out.
 struct StencilC {
     double c0, c1, c2, c3, elap;
 };
@@ -321,11 +319,12 @@ __device__ __forceinline__ double grad2_site(const T *__restrict__ fld, size_t n
     return v;
 }
 
-template <typename T, int EPI>
-__global__ __launch_bounds__(TPB) void k_stencil(const T *__restrict__ fld, T *__restrict__ fldp, T *__restrict__ out,
-                                                 int nx, int ny, int nz, int nf, StencilC sc, ModelDev md,
-                                                 const DevScalars *__restrict__ dsc, double *__restrict__ partials,
-                                                 size_t ms)
+// Reductions of the state with the Laplacian and the GRAD2 form, any stencil.
+template <typename T>
+__global__ __launch_bounds__(TPB) void k_reduce27(const T *__restrict__ fld, const T *__restrict__ fldp, int nx, int ny,
+                                                  int nz, int nf, StencilC sc, ModelDev md,
+                                                  const DevScalars *__restrict__ dsc, double *__restrict__ partials,
+                                                  size_t ms)
 {
     fld += blockIdx.y * ms;
     fldp += blockIdx.y * ms;
@@ -337,20 +336,9 @@ __global__ __launch_bounds__(TPB) void k_stencil(const T *__restrict__ fld, T *_
     const size_t nvol = (size_t)nx * ny * nz;
     const T c0 = T(sc.c0), c1 = T(sc.c1), c2 = T(sc.c2), c3 = T(sc.c3), el = T(sc.elap);
     const bool has2 = sc.c2 != 0.0, has3 = sc.c3 != 0.0;
-    T hA = 0, hB = 0;
-    if constexpr (EPI == EPI_KICK) {
-        hA = T(dsc->hA);
-        hB = T(dsc->hB);
-    }
-    float pb32[2] = {0, 0};
     double pb64[2] = {0, 0};
-    T mu[2] = {0, 0};
     if constexpr (sizeof(T) == 4) {
-        for (int l = 0; l < 2; ++l) {
-            pb64[l] = dsc->mean_phi[l];
-            pb32[l] = float(pb64[l]);
-            if constexpr (EPI == EPI_KICK) mu[l] = T(dsc->mu[l]);
-        }
+        for (int l = 0; l < 2; ++l) pb64[l] = dsc->mean_phi[l];
     }
     double acc[NRED] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (size_t s = blockIdx.x * (size_t)TPB + threadIdx.x; s < nvol; s += (size_t)gridDim.x * TPB) {
@@ -361,39 +349,25 @@ __global__ __launch_bounds__(TPB) void k_stencil(const T *__restrict__ fld, T *_
         const int jm = j == 0 ? ny - 1 : j - 1, jp = j == ny - 1 ? 0 : j + 1;
         const int km = k == 0 ? nz - 1 : k - 1, kp = k == nz - 1 ? 0 : k + 1;
         const int xs[3] = {im, i, ip}, ys[3] = {jm, j, jp}, zs[3] = {km, k, kp};
-        T lap[2] = {0, 0}, phi[2] = {0, 0};
+        T phi[2] = {0, 0};
         for (int l = 0; l < nf; ++l) {
             T f0;
             const T v = stencil_sum(fld + (size_t)l * nvol, xs, ys, zs, nx, ny, c0, c1, c2, c3, has2, has3, &f0);
-            lap[l] = v * el;
             phi[l] = f0;
+            const T p = fldp[(size_t)l * nvol + s];
+            acc[RC_GE] -= double(f0) * double(v * el);
+            acc[RC_KE] += double(p) * double(p);
+            acc[RC_S1 + l] += double(p);
         }
-        if constexpr (EPI == EPI_STORE) {
-            for (int l = 0; l < nf; ++l) out[(size_t)l * nvol + s] = lap[l];
-        } else {
-            T dv[2] = {0, 0};
-            if constexpr (EPI == EPI_KICK) site_dv(md, pb32, phi, dv);
-            acc[RC_PE] += site_v(md, pb64, phi);
-            for (int l = 0; l < nf; ++l) {
-                T p = fldp[(size_t)l * nvol + s];
-                if constexpr (EPI == EPI_KICK) {
-                    p = p + (hA * lap[l] - hB * dv[l]);
-                    if constexpr (sizeof(T) == 4) p = p - mu[l];
-                    fldp[(size_t)l * nvol + s] = p;
-                }
-                acc[RC_GE] -= double(phi[l]) * double(lap[l]);
-                acc[RC_KE] += double(p) * double(p);
-                acc[RC_S1 + l] += double(p);
-            }
-            acc[RC_M1] += double(phi[0]);
-            acc[RC_M2] += double(phi[1]);
-            if constexpr (EPI == EPI_REDUCE) acc[RC_X] += grad2_site(fld, nvol, nf, xs, ys, zs, nx, ny, sc);
-        }
+        acc[RC_PE] += site_v(md, pb64, phi);
+        acc[RC_M1] += double(phi[0]);
+        acc[RC_M2] += double(phi[1]);
+        acc[RC_X] += grad2_site(fld, nvol, nf, xs, ys, zs, nx, ny, sc);
     }
-    if constexpr (EPI != EPI_STORE) block_reduce_store2<NRED>(acc, partials + (size_t)blockIdx.x * NRED);
+    block_reduce_store2<NRED>(acc, partials + (size_t)blockIdx.x * NRED);
 }
 
-// 7-point stencil (c2 = c3 = 0) + kick / reduce, marching along z: a
+// The same reductions for the 7-point stencil (c2 = c3 = 0), marching along z: a
 // TXV x TYV block (64 x 4) owns an (x, y) tile and a chunk of KCV (32)
 // planes; each thread keeps its column's values at k-1, k, k+1 in registers,
 // so per site it loads the new k+1 value and the four in-plane neighbours
@@ -402,9 +376,9 @@ __global__ __launch_bounds__(TPB) void k_stencil(const T *__restrict__ fld, T *_
 // same as there.
 constexpr int ST7_TX = 64, ST7_TY = 4, ST7_KC = 32;
 
-template <typename T, int EPI, int TXV = ST7_TX, int TYV = ST7_TY, int KCV = ST7_KC>
-__global__ __launch_bounds__(TPB) void k_stencil7(const T *__restrict__ fld, T *__restrict__ fldp, int nx, int ny,
-                                                  int nz, int nf, StencilC sc, ModelDev md,
+template <typename T, int TXV = ST7_TX, int TYV = ST7_TY, int KCV = ST7_KC>
+__global__ __launch_bounds__(TPB) void k_reduce7(const T *__restrict__ fld, const T *__restrict__ fldp, int nx, int ny,
+                                                 int nz, int nf, StencilC sc, ModelDev md,
                                                   const DevScalars *__restrict__ dsc, double *__restrict__ partials,
                                                   size_t ms)
 {
@@ -418,20 +392,9 @@ __global__ __launch_bounds__(TPB) void k_stencil7(const T *__restrict__ fld, T *
     md.p2 = dsc->mp[2];
     const size_t nvol = (size_t)nx * ny * nz, plane = (size_t)nx * ny;
     const T c0 = T(sc.c0), c1 = T(sc.c1), el = T(sc.elap);
-    T hA = 0, hB = 0;
-    if constexpr (EPI == EPI_KICK) {
-        hA = T(dsc->hA);
-        hB = T(dsc->hB);
-    }
-    float pb32[2] = {0, 0};
     double pb64[2] = {0, 0};
-    T mu[2] = {0, 0};
     if constexpr (sizeof(T) == 4) {
-        for (int l = 0; l < 2; ++l) {
-            pb64[l] = dsc->mean_phi[l];
-            pb32[l] = float(pb64[l]);
-            if constexpr (EPI == EPI_KICK) mu[l] = T(dsc->mu[l]);
-        }
+        for (int l = 0; l < 2; ++l) pb64[l] = dsc->mean_phi[l];
     }
     double acc[NRED] = {0, 0, 0, 0, 0, 0, 0, 0};
     const int ntx = (nx + TXV - 1) / TXV, nty = (ny + TYV - 1) / TYV, nkc = (nz + KCV - 1) / KCV;
@@ -473,7 +436,6 @@ __global__ __launch_bounds__(TPB) void k_stencil7(const T *__restrict__ fld, T *
         }
         load_plane(k0, nb, nxt, pp);
         for (int k = k0; k < k1; ++k) {
-            const size_t pk = plane * (size_t)k;
             T nb2[2][4] = {}, nxt2[2] = {0, 0}, pp2[2] = {0, 0};
             if (k + 1 < k1) load_plane(k + 1, nb2, nxt2, pp2);
             T lap[2] = {0, 0}, phi[2] = {0, 0};
@@ -484,24 +446,16 @@ __global__ __launch_bounds__(TPB) void k_stencil7(const T *__restrict__ fld, T *
                 lap[l] = (c0 * cur[l] + c1 * r1) * el;
                 phi[l] = cur[l];
             }
-            const size_t s = col + pk;
-            T dv[2] = {0, 0};
-            if constexpr (EPI == EPI_KICK) site_dv(md, pb32, phi, dv);
             acc[RC_PE] += site_v(md, pb64, phi);
             for (int l = 0; l < nf; ++l) {
-                T p = pp[l];
-                if constexpr (EPI == EPI_KICK) {
-                    p = p + (hA * lap[l] - hB * dv[l]);
-                    if constexpr (sizeof(T) == 4) p = p - mu[l];
-                    fldp[(size_t)l * nvol + s] = p;
-                }
+                const T p = pp[l];
                 acc[RC_GE] -= double(phi[l]) * double(lap[l]);
                 acc[RC_KE] += double(p) * double(p);
                 acc[RC_S1 + l] += double(p);
             }
             acc[RC_M1] += double(phi[0]);
             acc[RC_M2] += double(phi[1]);
-            if constexpr (EPI == EPI_REDUCE) {
+            {
                 // STENCIL(c, GRAD2) with c2 = c3 = 0, neighbours in RANK1 order
                 // (x-, x+, y-, y+, z-, z+), each summed over the fields
                 auto d2 = [&](T v0, T v1) {
@@ -531,37 +485,303 @@ __global__ __launch_bounds__(TPB) void k_stencil7(const T *__restrict__ fld, T *
     block_reduce_store2<NRED>(acc, partials + (size_t)blockIdx.x * NRED);
 }
 
+// Finite-difference kick, marching along z: pi += hA lap - hB V', reduce GE, PE,
+// KE'.  With DRIFT the pending drifts come first, phi' = phi + dc pi, and the
+// kick takes the Laplacian of phi': the sites and the halo of each plane are
+// drifted as they are loaded, so one sweep moves four arrays per field (phi,
+// pi in; phi', pi' out) where a drift sweep and a kick move six.  Neighbouring
+// blocks read each other's old phi and pi, so phi' and pi' go to other arrays
+// (fo, po), which run_ops swaps with the state's; without DRIFT phi is only
+// read and pi is kicked in place (po = p).
+//
+// A block owns a tile of LX 16-byte vectors by TY rows and a chunk of KC
+// planes, one vector of 4 (FP32) or 2 (FP64) sites per thread.  Per plane a
+// thread loads its vector (and the tile's edge threads the halo), one plane
+// ahead; the drifted plane goes to LDS (two buffers, one barrier per plane);
+// the thread forms the sums F of the four faces and, for the 27-point
+// stencil, D of the four corners around each site within the plane.  A
+// site's sums are then r1 = F(k) + C(k-1) + C(k+1), r2 = D(k) + F(k-1) + F(k+1),
+// r3 = D(k-1) + D(k+1): every plane is read once, and 8 neighbours per site come from
+// LDS instead of 26 from memory.  Per kick with its drift (drift sweep +
+// grid-stride or register-marching kick before), three lattices in turn: 256^3
+// mixed 7-point 190 -> 139 us, 27-point 397 -> 147 us, FP64 7-point 341 -> 239 us,
+// 512^3 mixed 1.51 -> 1.11 ms (4.0 TB/s of the four arrays), 64^3 FP64 24 -> 9 us.
+// Two waves per SIMD by registers (FP32, two fields); a cap at 170 registers spills
+// (512^3: 1.9 ms) and loading each plane when its turn comes costs 7 %.
+template <typename T, int NF, bool DRIFT, bool WIDE>
+__global__ __launch_bounds__(TPB) void k_fd_kick(const T *f, const T *p, T *fo, T *po, int nx, int ny, int nz,
+                                                 StencilC sc, ModelDev md, const DevScalars *__restrict__ dsc,
+                                                 double *__restrict__ partials, size_t ms, int LX, int TY, int KC)
+{
+    constexpr int VW = 16 / sizeof(T);
+    using VT = Vec16<T>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char fd_lds[];
+    f += blockIdx.y * ms;
+    p += blockIdx.y * ms;
+    if constexpr (DRIFT) fo += blockIdx.y * ms;
+    po += blockIdx.y * ms;
+    dsc += blockIdx.y;
+    partials += (size_t)blockIdx.y * MAX_GRID * NRED;
+    md.p0 = dsc->mp[0];
+    md.p1 = dsc->mp[1];
+    md.p2 = dsc->mp[2];
+    const size_t nvol = (size_t)nx * ny * nz;
+    const T c0 = T(sc.c0), c1 = T(sc.c1), c2 = T(sc.c2), c3 = T(sc.c3), el = T(sc.elap);
+    const T hA = T(dsc->hA), hB = T(dsc->hB);
+    float pb32[2] = {0, 0};
+    double pb64[2] = {0, 0};
+    T mu[2] = {0, 0}, nu[2] = {0, 0};
+    if constexpr (sizeof(T) == 4) {
+        for (int l = 0; l < 2; ++l) {
+            pb64[l] = dsc->mean_phi[l];
+            pb32[l] = float(pb64[l]);
+            mu[l] = T(dsc->mu[l]);
+            nu[l] = T(dsc->nu[l]);
+        }
+    }
+    const int nd = DRIFT ? dsc->nd : 0;
+    const T dc0 = T(dsc->dc[0]), dc1 = T(dsc->dc[1]);
+    // the drift sweep's arithmetic (launch_drift)
+    auto drift = [&](T x, T q, int l) {
+        if constexpr (DRIFT) {
+            x = x + dc0 * q;
+            if (nd > 1) x = x + dc1 * q;
+            if constexpr (sizeof(T) == 4) x = x - nu[l];
+        }
+        return x;
+    };
+    const int TX = LX * VW, ntx = nx / TX, nty = (ny + TY - 1) / TY, nkc = (nz + KC - 1) / KC;
+    const int items = ntx * nty * nkc;
+    // LDS plane: interior at column VW, one halo column either side; rows -1 .. TY
+    const int pitch = TX + 2 * VW, psize = (TY + 2) * pitch;
+    T *const buf = reinterpret_cast<T *>(fd_lds);
+    const int tid = threadIdx.x;
+    const int lx = tid % LX, ty = tid / LX;
+    const bool active = ty < TY;
+    const bool hv = tid < 2 * LX; // halo row -1 (tid < LX) or TY
+    const int hvr = tid < LX ? -1 : TY;
+    const int hs = TPB - 1 - tid; // halo column cell: row hs / 2 - 1, side hs % 2
+    const bool hsok = hs < 2 * (TY + 2);
+    const int hsr = hs / 2 - 1, hsc = hs % 2;
+    auto wrap = [](int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); };
+    double acc[NRED] = {0, 0, 0, 0, 0, 0, 0, 0};
+    // each XCD (block index mod 8) takes a contiguous eighth of the items, so
+    // neighbouring tiles share an L2
+    const int C8 = (items + 7) >> 3, i1 = min(((int)(blockIdx.x & 7) + 1) * C8, items);
+    for (int it = (int)(blockIdx.x & 7) * C8 + (int)(blockIdx.x >> 3); it < i1; it += gridDim.x >> 3) {
+        const int xt = it % ntx, rest = it / ntx, yt = rest % nty, kc = rest / nty;
+        const int x0 = xt * TX, y0 = yt * TY, k0 = kc * KC, k1 = min(k0 + KC, nz);
+        const bool valid = active && y0 + ty < ny;
+        // row-plane offsets within a plane: own vector, halo vector, halo cell
+        const size_t oo = (size_t)wrap(y0 + ty, ny) * nx + x0 + lx * VW;
+        const size_t ov = (size_t)wrap(y0 + hvr, ny) * nx + x0 + lx * VW;
+        const size_t os = (size_t)wrap(y0 + hsr, ny) * nx + (hsc ? wrap(x0 + TX, nx) : wrap(x0 - 1, nx));
+        VT rf[NF], rp[NF], vf[NF], vp[NF];
+        T sf[NF], sp[NF];
+        auto issue = [&](int k) {
+            const size_t zo = (size_t)wrap(k, nz) * nx * ny;
+#pragma unroll
+            for (int l = 0; l < NF; ++l) {
+                const size_t o = l * nvol + zo;
+                if (active) {
+                    rf[l] = *reinterpret_cast<const VT *>(f + o + oo);
+                    rp[l] = *reinterpret_cast<const VT *>(p + o + oo);
+                }
+                if (hv) {
+                    vf[l] = *reinterpret_cast<const VT *>(f + o + ov);
+                    if constexpr (DRIFT) vp[l] = *reinterpret_cast<const VT *>(p + o + ov);
+                }
+                if (hsok) {
+                    sf[l] = f[o + os];
+                    if constexpr (DRIFT) sp[l] = p[o + os];
+                }
+            }
+        };
+        VT C[NF], F[NF], D[NF], r1[NF], r2[NF], r3[NF], pc[NF]; // plane k - 1
+        issue(k0 - 1);
+        for (int k = k0 - 1; k <= k1; ++k) {
+            VT Cn[NF], pn[NF];
+            T *const b = buf + ((k - k0) & 1) * NF * psize;
+#pragma unroll
+            for (int l = 0; l < NF; ++l) {
+                T *const bl = b + l * psize;
+                if (active) {
+#pragma unroll
+                    for (int e = 0; e < VW; ++e) Cn[l].e[e] = drift(rf[l].e[e], rp[l].e[e], l);
+                    pn[l] = rp[l];
+                    *reinterpret_cast<VT *>(bl + (ty + 1) * pitch + VW + lx * VW) = Cn[l];
+                }
+                if (hv) {
+                    VT v;
+#pragma unroll
+                    for (int e = 0; e < VW; ++e) v.e[e] = drift(vf[l].e[e], DRIFT ? vp[l].e[e] : T(0), l);
+                    *reinterpret_cast<VT *>(bl + (hvr + 1) * pitch + VW + lx * VW) = v;
+                }
+                if (hsok) bl[(hsr + 1) * pitch + (hsc ? VW + TX : VW - 1)] = drift(sf[l], DRIFT ? sp[l] : T(0), l);
+            }
+            if (k < k1) issue(k + 1);
+            lds_sync();
+            VT Fn[NF], Dn[NF];
+            if (active && (WIDE || (k >= k0 && k < k1))) {
+#pragma unroll
+                for (int l = 0; l < NF; ++l) {
+                    const T *q = b + l * psize + (ty + 1) * pitch + VW + lx * VW;
+                    const VT up = *reinterpret_cast<const VT *>(q - pitch), dn = *reinterpret_cast<const VT *>(q + pitch);
+                    const T xl = q[-1], xr = q[VW];
+#pragma unroll
+                    for (int e = 0; e < VW; ++e)
+                        Fn[l].e[e] = (e ? Cn[l].e[e - 1] : xl) + (e < VW - 1 ? Cn[l].e[e + 1] : xr) + up.e[e] + dn.e[e];
+                    if constexpr (WIDE) {
+                        const T ul = q[-pitch - 1], ur = q[-pitch + VW], dl = q[pitch - 1], dr = q[pitch + VW];
+#pragma unroll
+                        for (int e = 0; e < VW; ++e)
+                            Dn[l].e[e] = (e ? up.e[e - 1] : ul) + (e < VW - 1 ? up.e[e + 1] : ur) +
+                                         (e ? dn.e[e - 1] : dl) + (e < VW - 1 ? dn.e[e + 1] : dr);
+                    }
+                }
+            }
+            if (valid && k > k0) { // plane k - 1 is complete
+                const size_t site = (size_t)(k - 1) * nx * ny + oo;
+#pragma unroll
+                for (int e = 0; e < VW; ++e) {
+                    T lap[NF], phi[2] = {0, 0}, dv[2] = {0, 0};
+#pragma unroll
+                    for (int l = 0; l < NF; ++l) {
+                        T v = c0 * C[l].e[e] + c1 * (r1[l].e[e] + Cn[l].e[e]);
+                        if constexpr (WIDE) {
+                            v = v + c2 * (r2[l].e[e] + Fn[l].e[e]);
+                            v = v + c3 * (r3[l].e[e] + Dn[l].e[e]);
+                        }
+                        lap[l] = v * el;
+                        phi[l] = C[l].e[e];
+                    }
+                    site_dv(md, pb32, phi, dv);
+                    acc[RC_PE] += site_v(md, pb64, phi);
+#pragma unroll
+                    for (int l = 0; l < NF; ++l) {
+                        T q = pc[l].e[e];
+                        q = q + (hA * lap[l] - hB * dv[l]);
+                        if constexpr (sizeof(T) == 4) q = q - mu[l];
+                        pc[l].e[e] = q;
+                        acc[RC_GE] -= double(phi[l]) * double(lap[l]);
+                        acc[RC_KE] += double(q) * double(q);
+                        acc[RC_S1 + l] += double(q);
+                        acc[RC_M1 + l] += double(phi[l]);
+                    }
+                }
+#pragma unroll
+                for (int l = 0; l < NF; ++l) {
+                    *reinterpret_cast<VT *>(po + l * nvol + site) = pc[l];
+                    if constexpr (DRIFT) *reinterpret_cast<VT *>(fo + l * nvol + site) = C[l];
+                }
+            }
+#pragma unroll
+            for (int l = 0; l < NF; ++l) {
+#pragma unroll
+                for (int e = 0; e < VW; ++e) {
+                    r1[l].e[e] = Fn[l].e[e] + C[l].e[e];
+                    if constexpr (WIDE) {
+                        r2[l].e[e] = Dn[l].e[e] + F[l].e[e];
+                        r3[l].e[e] = D[l].e[e];
+                    }
+                }
+                C[l] = Cn[l];
+                F[l] = Fn[l];
+                D[l] = Dn[l];
+                pc[l] = pn[l];
+            }
+        }
+        lds_sync(); // the next item writes the buffers anew
+    }
+    block_reduce_store2<NRED>(acc, partials + (size_t)blockIdx.x * NRED);
+}
+
+// Tile of the kick: as many vectors along x as divide the row, up to 64 sites
+// (neighbouring lanes read neighbouring vectors; a row's tiles are equal, so no
+// lane is masked along x); as many rows as 256 threads hold, spread evenly
+// over ny; planes per chunk: 32 (two of 34 loaded planes are halo), halved down
+// to 4 until there are 2 blocks per CU (256^3 mixed, per kick with three lattices
+// in turn: 139 us; until 1 / 4 / 8 per CU: 140, 147,
+// 161 us; 192 x 96 x 128 FP64 27-point: 48 us, 45, 56, 56).  The shape depends on the lattice only,
+// so batch members run exactly as single contexts.
+struct FdShape {
+    int LX, TY, KC, items;
+    size_t lds;
+};
 template <typename T>
-int launch_stencil(Ctx &c, int epi)
+static FdShape fd_shape(const Ctx &c)
+{
+    constexpr int VW = 16 / sizeof(T);
+    FdShape s{};
+    const int nv = c.nx / VW;
+    for (int d = 1; d <= 64 / VW; ++d)
+        if (nv % d == 0) s.LX = d;
+    int ty = TPB / s.LX;
+    if (ty > 64) ty = 64;
+    if (ty > c.ny) ty = c.ny;
+    const int nty = (c.ny + ty - 1) / ty;
+    s.TY = (c.ny + nty - 1) / nty;
+    const int tiles = nv / s.LX * nty;
+    s.KC = 32;
+    while (s.KC > 4 && tiles * ((c.nz + s.KC - 1) / s.KC) < 512) s.KC /= 2;
+    s.items = tiles * ((c.nz + s.KC - 1) / s.KC);
+    s.lds = sizeof(T) * 2 * c.nfld * (s.TY + 2) * (s.LX * VW + 2 * VW);
+    return s;
+}
+
+template <typename T, int NF, bool DRIFT>
+static int fd_kick_go(Ctx &c, T *fo, T *po)
+{
+    const double *cs = c.cfg.stencil;
+    const StencilC sc{cs[0], cs[1], cs[2], cs[3], 1.0 / (c.dx * c.dx) / cs[4]};
+    const ModelDev md{c.cfg.model, c.nfld, c.cfg.model_params[0], c.cfg.model_params[1]};
+    const FdShape s = fd_shape<T>(c);
+    // a multiple of 8, for the tile order; blocks past the last item add nothing
+    const int g = s.items > MAX_GRID ? MAX_GRID : (s.items + 7) & ~7;
+    if (cs[2] == 0.0 && cs[3] == 0.0)
+        hipLaunchKernelGGL((k_fd_kick<T, NF, DRIFT, false>), dim3(g, c.B), dim3(TPB), s.lds, c.stream,
+                           (const T *)c.fld, (const T *)c.fldp, fo, po, c.nx, c.ny, c.nz, sc, md, c.dsc, c.partials,
+                           c.ms.f, s.LX, s.TY, s.KC);
+    else
+        hipLaunchKernelGGL((k_fd_kick<T, NF, DRIFT, true>), dim3(g, c.B), dim3(TPB), s.lds, c.stream,
+                           (const T *)c.fld, (const T *)c.fldp, fo, po, c.nx, c.ny, c.nz, sc, md, c.dsc, c.partials,
+                           c.ms.f, s.LX, s.TY, s.KC);
+    LAT_HIP(&c, hipGetLastError());
+    return g;
+}
+
+template <typename T>
+int launch_fd_kick(Ctx &c, bool drift)
+{
+    if (drift)
+        return c.nfld == 2 ? fd_kick_go<T, 2, true>(c, (T *)c.fld2, (T *)c.fldp2)
+                           : fd_kick_go<T, 1, true>(c, (T *)c.fld2, (T *)c.fldp2);
+    return c.nfld == 2 ? fd_kick_go<T, 2, false>(c, nullptr, (T *)c.fldp)
+                       : fd_kick_go<T, 1, false>(c, nullptr, (T *)c.fldp);
+}
+
+// Reduction of the state with the finite-difference Laplacian (EPI_REDUCE);
+// returns the number of partials.
+template <typename T>
+int launch_fd_reduce(Ctx &c)
 {
     const double *cs = c.cfg.stencil;
     StencilC sc{cs[0], cs[1], cs[2], cs[3], 1.0 / (c.dx * c.dx) / cs[4]};
     ModelDev md{c.cfg.model, c.nfld, c.cfg.model_params[0], c.cfg.model_params[1]};
-    size_t blocks = (c.nvol + TPB - 1) / TPB;
-    int g = grid_for(blocks > (size_t)MAX_GRID ? MAX_GRID : (int)blocks);
-    T *fld = (T *)c.fld, *fldp = (T *)c.fldp;
-    if (cs[2] == 0.0 && cs[3] == 0.0 && (epi == EPI_KICK || epi == EPI_REDUCE)) {
+    const T *fld = (const T *)c.fld, *fldp = (const T *)c.fldp;
+    int g;
+    if (cs[2] == 0.0 && cs[3] == 0.0) {
         const int items = ((c.nx + ST7_TX - 1) / ST7_TX) * ((c.ny + ST7_TY - 1) / ST7_TY) *
                           ((c.nz + ST7_KC - 1) / ST7_KC);
         g = grid_for(items > MAX_GRID ? MAX_GRID : items);
-        if (epi == EPI_KICK)
-            hipLaunchKernelGGL((k_stencil7<T, EPI_KICK>), dim3(g, c.B), dim3(TPB), 0, c.stream, fld, fldp, c.nx,
-                               c.ny, c.nz, c.nfld, sc, md, c.dsc, c.partials, c.ms.f);
-        else
-            hipLaunchKernelGGL((k_stencil7<T, EPI_REDUCE>), dim3(g, c.B), dim3(TPB), 0, c.stream, fld, fldp, c.nx,
-                               c.ny, c.nz, c.nfld, sc, md, c.dsc, c.partials, c.ms.f);
-        LAT_HIP(&c, hipGetLastError());
-        return g;
+        hipLaunchKernelGGL((k_reduce7<T>), dim3(g, c.B), dim3(TPB), 0, c.stream, fld, fldp, c.nx, c.ny, c.nz, c.nfld,
+                           sc, md, c.dsc, c.partials, c.ms.f);
+    } else {
+        const size_t blocks = (c.nvol + TPB - 1) / TPB;
+        g = grid_for(blocks > (size_t)MAX_GRID ? MAX_GRID : (int)blocks);
+        hipLaunchKernelGGL((k_reduce27<T>), dim3(g, c.B), dim3(TPB), 0, c.stream, fld, fldp, c.nx, c.ny, c.nz, c.nfld,
+                           sc, md, c.dsc, c.partials, c.ms.f);
     }
-    if (epi == EPI_KICK)
-        hipLaunchKernelGGL((k_stencil<T, EPI_KICK>), dim3(g, c.B), dim3(TPB), 0, c.stream, fld, fldp, (T *)nullptr,
-                           c.nx, c.ny, c.nz, c.nfld, sc, md, c.dsc, c.partials, c.ms.f);
-    else if (epi == EPI_REDUCE)
-        hipLaunchKernelGGL((k_stencil<T, EPI_REDUCE>), dim3(g, c.B), dim3(TPB), 0, c.stream, fld, fldp,
-                           (T *)nullptr, c.nx, c.ny, c.nz, c.nfld, sc, md, c.dsc, c.partials, c.ms.f);
-    else
-        hipLaunchKernelGGL((k_stencil<T, EPI_STORE>), dim3(g), dim3(TPB), 0, c.stream, fld, fldp, (T *)c.io64, c.nx,
-                           c.ny, c.nz, 1, sc, md, c.dsc, c.partials, (size_t)0);
     LAT_HIP(&c, hipGetLastError());
     return g;
 }
@@ -875,8 +1095,10 @@ template int launch_drift<double>(Ctx &);
 template int launch_drift<float>(Ctx &);
 template int launch_reduce_state<double>(Ctx &);
 template int launch_reduce_state<float>(Ctx &);
-template int launch_stencil<double>(Ctx &, int);
-template int launch_stencil<float>(Ctx &, int);
+template int launch_fd_kick<double>(Ctx &, bool);
+template int launch_fd_kick<float>(Ctx &, bool);
+template int launch_fd_reduce<double>(Ctx &);
+template int launch_fd_reduce<float>(Ctx &);
 template int launch_gw_source<double>(Ctx &, int, int, double *);
 template int launch_gw_source<float>(Ctx &, int, int, float *);
 template int launch_gw_stencil_kick<double>(Ctx &);

@@ -79,12 +79,6 @@ __device__ __forceinline__ int kspace_row(int row)
     }
 }
 
-// 16-byte vector of reals (4 floats or 2 doubles) for vector loads/stores.
-template <typename T>
-struct alignas(16) Vec16 {
-    T e[16 / sizeof(T)];
-};
-
 // ---------------------------------------------------------------- block reduction
 template <int NCH>
 __device__ __forceinline__ void block_reduce_store(double (&v)[NCH], double *out)

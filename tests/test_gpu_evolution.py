@@ -108,6 +108,63 @@ def test_single_splits_match_oracle(gpu, case):
     assert abs(g[3] - o[3]) < 1e-12 * abs(o[3])
 
 
+FD_SHAPES = [(8, 8, 64), (16, 48, 8), (96, 32, 8), (192, 8, 16), (64, 192, 8), (128, 16, 96)]
+
+
+@pytest.mark.parametrize("shape", FD_SHAPES)
+@pytest.mark.parametrize("stencil", [(-6.0, 1.0, 0.0, 0.0, 1.0), (-128.0, 14.0, 3.0, 1.0, 30.0)])
+def test_fd_tiles_match_oracle(gpu, shape, stencil):
+    """Finite-difference kicks on boxes whose rows, planes and chunks leave
+    partial tiles (nx, ny, nz from 8 to 192), an even and an odd number of kicks
+    per call (the odd one runs its first kick unfused)."""
+    print("case fd tiles", shape, stencil, flush=True)
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx + ny + nz)
+    fld = 1e-3 * rng.standard_normal((2, nz, ny, nx))
+    fldp = 1e-3 * rng.standard_normal((2, nz, ny, nx))
+    fld[0] += PHI0_C
+    fldp[0] += DPHI0_C
+    g, o = run_pair(gpu, shape, 0.05 * nx, 2, O.COSMIC, O.MODEL_TWOFIELD, (1.0, 2.5e5), O.LAP_STENCIL, stencil,
+                    fld, fldp, [("symp", (2, 1e-3, 2)), ("symp", (2, 1e-3, 3)), ("symp", (4, 1e-3, 1))])
+    assert rel(g[0], o[0]) < 1e-12 and rel(g[1], o[1]) < 1e-12
+    assert abs(g[2] - o[2]) < 1e-13 * abs(o[2]) and abs(g[3] - o[3]) < 1e-11 * abs(o[3])
+    for k in ("rho", "ke", "pe", "ge"):
+        assert abs(g[4][k] - o[4][k]) <= 1e-11 * abs(o[4][k]), k
+
+
+@pytest.mark.parametrize("members", [None, 3])
+@pytest.mark.parametrize("precision,tol", [("f64", 1e-13), ("mixed", 2e-6)])
+def test_fd_fused_kicks_match_single_steps(gpu, precision, tol, members):
+    """One call of four leapfrog steps (fused drift + kick sweeps) against four
+    calls of one step (a drift sweep and a kick each), single and batched: the
+    same fluctuations to a few roundings per step."""
+    print("case fd fused", precision, members, flush=True)
+    n, L, dt = (48, 32, 16), 2.4, 1e-3
+    rng = np.random.default_rng(3)
+    fld = 1e-3 * rng.standard_normal((2, 16, 32, 48))
+    fldp = 1e-3 * rng.standard_normal((2, 16, 32, 48))
+    fld[0] += PHI0_C
+    fldp[0] += DPHI0_C
+    kw = dict(nfld=2, length=L, laplacian=gpu.LAP_STENCIL, precision=gpu.F64 if precision == "f64" else gpu.MIXED)
+    got = []
+    for calls in ((4,), (1, 1, 1, 1)):
+        with gpu.Lattice(n, members=None if members is None else [(1.0, 2.5e5)] * members, **kw) as lat:
+            views = [lat] if members is None else [lat.member(m) for m in range(members)]
+            for v in views:
+                v.set_state(fld, fldp, 1.0, 0.0)
+                v.calc_metric()
+            for k in calls:
+                lat.symp2(dt, k)
+            got.append(views[-1].get_state())
+            if members is not None:
+                for v in views:
+                    v.close()
+    for a, b in zip(got[0][:2], got[1][:2]):
+        for l in range(2):
+            assert np.linalg.norm(a[l] - b[l]) < tol * np.linalg.norm(b[l] - b[l].mean())
+    assert abs(got[0][2] - got[1][2]) < 1e-13 * abs(got[1][2])
+
+
 def test_state_roundtrip_ghost_layout(gpu):
     """AoS ghosted fld(nfld,0:nx+1,...) in, periodic ghosts out (wrap_fields)."""
     n = 8
