@@ -181,6 +181,8 @@ int  lat_synchronize(lat_ctx *ctx);
  * f (host, n1*n2*n3 doubles) is overwritten in place with its Laplacian.  The
  * reference's Fk scratch and FFTW plans are owned by the context. */
 int  lat_laplacian_3d(lat_ctx *ctx, int n1, int n2, int n3, double *f, double dk);
+/* The same operator into another host array: f is only read (lap may be f). */
+int  lat_laplacian_3d_to(lat_ctx *ctx, int n1, int n2, int n3, const double *f, double *lap, double dk);
 
 /* Replaces gradient_squared_3d_spectral,
  * Pseudospec/mpi_dev/fftw_mod_mpi.f90:279-327 (correct-sign form). */

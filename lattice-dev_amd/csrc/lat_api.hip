@@ -1,10 +1,12 @@
 // lat_api.hip -- C ABI (include/lattice_c.h): context, state transfer, the
 // drop-in operators, and the device-resident symplectic executor.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <thread>
 #include <vector>
 
 #include "lat_internal.h"
@@ -64,15 +66,181 @@ static int sync(Ctx &c)
     return 0;
 }
 
+// ---------------------------------------------------------------- host copies
+static int stage_ring(Ctx &c)
+{
+    HostStage &h = *c.stage;
+    if (h.ring) return 0;
+    for (hipEvent_t &e : h.ev)
+        if (!e) LAT_HIP(&c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    LAT_HIP(&c, hipHostMalloc((void **)&h.ring, HostStage::SLOT * HostStage::SLOTS, hipHostMallocDefault));
+    return 0;
+}
+
+static void stage_free(HostStage *h)
+{
+    if (!h) return;
+    if (h->small) (void)hipHostFree(h->small);
+    if (h->ring) (void)hipHostFree(h->ring);
+    for (hipEvent_t e : h->ev)
+        if (e) (void)hipEventDestroy(e);
+    delete h;
+}
+
+// Chunks of whole rows, or of one row's bytes, of at most one slot.
+namespace {
+struct Chunks {
+    size_t width, rows, per; // rows per chunk; 0: the row is cut into slots
+    size_t count;
+    Chunks(size_t w, size_t r) : width(w), rows(r), per(w <= HostStage::SLOT ? HostStage::SLOT / w : 0)
+    {
+        count = per ? (r + per - 1) / per : r * ((w + HostStage::SLOT - 1) / HostStage::SLOT);
+    }
+    // device byte offset (rows dpitch apart), host byte offset, row bytes, rows
+    void at(size_t i, size_t dpitch, size_t &doff, size_t &hoff, size_t &w, size_t &n) const
+    {
+        if (per) {
+            const size_t r0 = i * per;
+            n = std::min(per, rows - r0);
+            w = width;
+            doff = r0 * dpitch;
+            hoff = r0 * width;
+        } else {
+            const size_t cuts = (width + HostStage::SLOT - 1) / HostStage::SLOT, r = i / cuts, b = (i % cuts) * HostStage::SLOT;
+            n = 1;
+            w = std::min(HostStage::SLOT, width - b);
+            doff = r * dpitch + b;
+            hoff = r * width + b;
+        }
+    }
+};
+} // namespace
+
+// Rows of w 16-byte elements, dp / sp elements apart, between the device and
+// pinned host memory.  A kernel instead of the copy engine: the engine's
+// copies of 1 MB in a stream start about 12 us apart.
+constexpr int STAGE_GRID = 128;
+__global__ __launch_bounds__(256) void k_stage(uint4 *__restrict__ dst, const uint4 *__restrict__ src, size_t w,
+                                               size_t dp, size_t sp, size_t n)
+{
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const size_t r = i / w, e = i - r * w;
+        dst[r * dp + e] = src[r * sp + e];
+    }
+}
+
+// Both directions: thread t of T copies the chunks t, t + T, ... through its
+// two slots, the DMA of one slot running while the CPU fills or drains the other.
+static int stage_copy(Ctx &c, bool to_host, char *dev, size_t dpitch, char *host, size_t width, size_t rows)
+{
+    if (!width || !rows) return 0;
+    int rc = stage_ring(c);
+    if (rc) return rc;
+    HostStage &h = *c.stage;
+    const Chunks ck(width, rows);
+    // a thread costs about 20 us to start: from 8 chunks on
+    const size_t T = ck.count >= 8 ? HostStage::THREADS : 1;
+    std::atomic<int> err{(int)hipSuccess};
+    auto work = [&](size_t t) {
+        auto check = [&](hipError_t e) {
+            if (e != hipSuccess) err.store((int)e);
+            return e == hipSuccess;
+        };
+        if (!check(hipSetDevice(c.device))) return;
+        auto slot_of = [&](size_t i) { return (int)(2 * t + (i / T) % 2); };
+        auto send = [&](size_t i) { // the chunk's DMA, and its event
+            size_t doff, hoff, w, n;
+            ck.at(i, dpitch, doff, hoff, w, n);
+            const int q = slot_of(i);
+            char *slot = h.ring + (size_t)q * HostStage::SLOT;
+            if (to_host)
+                hipLaunchKernelGGL(k_stage, dim3(STAGE_GRID), dim3(256), 0, c.stream, (uint4 *)slot,
+                                   (const uint4 *)(dev + doff), w / 16, w / 16, dpitch / 16, w * n / 16);
+            else
+                hipLaunchKernelGGL(k_stage, dim3(STAGE_GRID), dim3(256), 0, c.stream, (uint4 *)(dev + doff),
+                                   (const uint4 *)slot, w / 16, dpitch / 16, w / 16, w * n / 16);
+            if (!check(hipGetLastError()) || !check(hipEventRecord(h.ev[q], c.stream))) return false;
+            h.used[q] = true;
+            return true;
+        };
+        auto settle = [&](int q) { // the slot's last DMA is over
+            if (!h.used[q]) return true;
+            h.used[q] = false;
+            return check(hipEventSynchronize(h.ev[q]));
+        };
+        for (int q = 2 * (int)t; q < 2 * (int)t + 2; ++q)
+            if (!settle(q)) return; // of an earlier call
+        if (to_host && t < ck.count && !send(t)) return;
+        for (size_t i = t; i < ck.count && err.load() == (int)hipSuccess; i += T) {
+            size_t doff, hoff, w, n;
+            ck.at(i, dpitch, doff, hoff, w, n);
+            const int q = slot_of(i);
+            char *slot = h.ring + (size_t)q * HostStage::SLOT;
+            if (to_host) {
+                if (i + T < ck.count && !send(i + T)) return;
+                if (!settle(q)) return;
+                memcpy(host + hoff, slot, w * n);
+            } else {
+                if (!settle(q)) return;
+                memcpy(slot, host + hoff, w * n);
+                if (!send(i)) return;
+            }
+        }
+    };
+    std::vector<std::thread> th;
+    size_t started = 1;
+    try {
+        th.reserve(T - 1);
+        for (; started < T; ++started) th.emplace_back(work, started);
+    } catch (...) { // no further thread: this one copies the rest
+    }
+    work(0);
+    for (size_t t = started; t < T; ++t) work(t);
+    for (std::thread &x : th) x.join();
+    const hipError_t e = (hipError_t)err.load();
+    return e == hipSuccess ? 0 : hip_fail(&c, e, to_host ? "copy to the host" : "copy to the device");
+}
+
+int copy_to_device(Ctx &c, void *dev, size_t dpitch, const void *host, size_t width, size_t rows)
+{
+    return stage_copy(c, false, (char *)dev, dpitch, (char *)const_cast<void *>(host), width, rows);
+}
+
+int copy_to_host(Ctx &c, void *host, const void *dev, size_t dpitch, size_t width, size_t rows)
+{
+    return stage_copy(c, true, (char *)const_cast<void *>(dev), dpitch, (char *)host, width, rows);
+}
+
+// The binned channels (spec_out) into the small area, and from there after a
+// synchronisation.
+static int spec_fetch(Ctx &c, size_t n)
+{
+    if (sizeof(double) * n > HostStage::SMALL - HostStage::SPEC) {
+        c.last_error = "spectrum larger than the staging area";
+        return -2;
+    }
+    LAT_HIP(&c, hipMemcpyAsync(c.stage->small + HostStage::SPEC, c.spec_out, sizeof(double) * n, hipMemcpyDeviceToHost,
+                               c.stream));
+    return 0;
+}
+
+static void spec_read(Ctx &c, std::vector<double> &raw)
+{
+    memcpy(raw.data(), c.stage->small + HostStage::SPEC, sizeof(double) * raw.size());
+}
+
 static int pull_scalars(Ctx &c)
 {
-    LAT_HIP(&c, hipMemcpyAsync(&c.host_sc, c.dsc, sizeof(DevScalars), hipMemcpyDeviceToHost, c.stream));
-    return sync(c);
+    LAT_HIP(&c, hipMemcpyAsync(c.stage->small, c.dsc, sizeof(DevScalars), hipMemcpyDeviceToHost, c.stream));
+    int rc = sync(c);
+    if (!rc) memcpy(&c.host_sc, c.stage->small, sizeof(DevScalars));
+    return rc;
 }
 
 static int push_scalars(Ctx &c)
 {
-    LAT_HIP(&c, hipMemcpyAsync(c.dsc, &c.host_sc, sizeof(DevScalars), hipMemcpyHostToDevice, c.stream));
+    memcpy(c.stage->small, &c.host_sc, sizeof(DevScalars));
+    LAT_HIP(&c, hipMemcpyAsync(c.dsc, c.stage->small, sizeof(DevScalars), hipMemcpyHostToDevice, c.stream));
     return sync(c);
 }
 
@@ -530,7 +698,7 @@ static int host_r2c(Ctx &c, const double *f_host)
 {
     int rc = ensure_io(c);
     if (rc) return rc;
-    LAT_HIP(&c, hipMemcpyAsync(c.io64, f_host, sizeof(double) * c.nvol, hipMemcpyHostToDevice, c.stream));
+    if ((rc = copy_to_device(c, c.io64, f_host, sizeof(double) * c.nvol))) return rc;
     cpx<double> *F = (cpx<double> *)c.Fk64;
     if ((rc = launch_x_r2c<double>(c, c.twx64, c.io64, nullptr, F, 0))) return rc;
     if ((rc = launch_col<double>(c, c.twy64, F, 1, 0, 1))) return rc;
@@ -539,16 +707,12 @@ static int host_r2c(Ctx &c, const double *f_host)
 
 static int fk_to_host(Ctx &c, const cpx<double> *F, double *Fk_host)
 {
-    LAT_HIP(&c, hipMemcpy2DAsync(Fk_host, sizeof(cpx<double>) * c.nxh, F, sizeof(cpx<double>) * c.P,
-                                 sizeof(cpx<double>) * c.nxh, (size_t)c.ny * c.nz, hipMemcpyDeviceToHost, c.stream));
-    return 0;
+    return copy_to_host(c, Fk_host, F, sizeof(cpx<double>) * c.P, sizeof(cpx<double>) * c.nxh, (size_t)c.ny * c.nz);
 }
 
 static int fk_from_host(Ctx &c, cpx<double> *F, const double *Fk_host)
 {
-    LAT_HIP(&c, hipMemcpy2DAsync(F, sizeof(cpx<double>) * c.P, Fk_host, sizeof(cpx<double>) * c.nxh,
-                                 sizeof(cpx<double>) * c.nxh, (size_t)c.ny * c.nz, hipMemcpyHostToDevice, c.stream));
-    return 0;
+    return copy_to_device(c, F, sizeof(cpx<double>) * c.P, Fk_host, sizeof(cpx<double>) * c.nxh, (size_t)c.ny * c.nz);
 }
 
 // derivative multiply: G = i k_axis dk * F / nvol (signed wavenumbers)
@@ -581,31 +745,23 @@ __global__ void k_sq_acc(const double *__restrict__ d, double *__restrict__ acc,
 template <typename T>
 static int upload_fields(Ctx &c, void *dst, const double *soa, size_t n)
 {
-    // the copy runs on the null stream, which does not order against the
-    // context's non-blocking stream: drain it first
-    int rc = sync(c);
-    if (rc) return rc;
     if (sizeof(T) == 8) {
-        LAT_HIP(&c, hipMemcpy(dst, soa, sizeof(double) * n, hipMemcpyHostToDevice));
-        return 0;
+        const int rc = copy_to_device(c, dst, soa, sizeof(double) * n);
+        return rc ? rc : sync(c);
     }
     std::vector<float> tmp(n);
     for (size_t i = 0; i < n; ++i) tmp[i] = (float)soa[i];
-    LAT_HIP(&c, hipMemcpy(dst, tmp.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-    return 0;
+    const int rc = copy_to_device(c, dst, tmp.data(), sizeof(float) * n);
+    return rc ? rc : sync(c);
 }
 
 template <typename T>
 static int download_fields(Ctx &c, double *soa, const void *src, size_t n)
 {
-    int rc = sync(c);
-    if (rc) return rc;
-    if (sizeof(T) == 8) {
-        LAT_HIP(&c, hipMemcpy(soa, src, sizeof(double) * n, hipMemcpyDeviceToHost));
-        return 0;
-    }
+    if (sizeof(T) == 8) return copy_to_host(c, soa, src, sizeof(double) * n);
     std::vector<float> tmp(n);
-    LAT_HIP(&c, hipMemcpy(tmp.data(), src, sizeof(float) * n, hipMemcpyDeviceToHost));
+    const int rc = copy_to_host(c, tmp.data(), src, sizeof(float) * n);
+    if (rc) return rc;
     for (size_t i = 0; i < n; ++i) soa[i] = tmp[i];
     return 0;
 }
@@ -676,6 +832,11 @@ static int create_ctx(const lat_config *cfg, int B, const double *mparams, lat_c
     int rc = 0;
     hipError_t e = hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
     if (e != hipSuccess) { delete h; return -3; }
+    c.stage = new HostStage();
+    if (hipHostMalloc((void **)&c.stage->small, HostStage::SMALL, hipHostMallocDefault) != hipSuccess) {
+        lat_destroy(h);
+        return -3;
+    }
     const size_t es = elem_size(c);
     rc |= ensure(c, &c.fld, es * B * c.ms.f, "hipMalloc fld");
     rc |= ensure(c, &c.fldp, es * B * c.ms.f, "hipMalloc fldp");
@@ -775,6 +936,7 @@ int lat_member(lat_ctx *h, int m, lat_ctx **out)
     w.parent = &c;
     w.nx = c.nx; w.ny = c.ny; w.nz = c.nz; w.nxh = c.nxh; w.P = c.P;
     w.nvol = c.nvol; w.nk = c.nk; w.dx = c.dx; w.dk = c.dk; w.prec = c.prec; w.nfld = c.nfld;
+    w.stage = c.stage;
     w.stream = c.stream;
     w.device = c.device;
     w.cus = c.cus;
@@ -827,6 +989,7 @@ void lat_destroy(lat_ctx *h)
         if (p) (void)hipFree(p);
     for (hipEvent_t e : c.prof.pool) (void)hipEventDestroy(e);
     if (c.stream && c.owns_stream) (void)hipStreamDestroy(c.stream);
+    stage_free(c.stage);
     delete h;
 }
 
@@ -852,8 +1015,7 @@ int lat_fft_r2c_3d(lat_ctx *h, const double *f, double *Fk)
     if (!f || !Fk) return -1;
     int rc = host_r2c(c, f);
     if (rc) return rc;
-    if ((rc = fk_to_host(c, (const cpx<double> *)c.Fk64, Fk))) return rc;
-    return sync(c);
+    return fk_to_host(c, (const cpx<double> *)c.Fk64, Fk);
 }
 
 int lat_fft_c2r_3d(lat_ctx *h, const double *Fk, double *f)
@@ -869,15 +1031,19 @@ int lat_fft_c2r_3d(lat_ctx *h, const double *Fk, double *f)
     if ((rc = launch_col<double>(c, c.twy64, F, 1, 1, 1))) return rc;
     rc = launch_x_c2r<double>(c, c.twx64, F, 1, EPI_STORE, c.io64, nullptr, nullptr);
     if (rc < 0) return rc;
-    LAT_HIP(&c, hipMemcpyAsync(f, c.io64, sizeof(double) * c.nvol, hipMemcpyDeviceToHost, c.stream));
-    return sync(c);
+    return copy_to_host(c, f, c.io64, sizeof(double) * c.nvol);
 }
 
 int lat_laplacian_3d(lat_ctx *h, int n1, int n2, int n3, double *f, double dk)
 {
+    return lat_laplacian_3d_to(h, n1, n2, n3, f, f, dk);
+}
+
+int lat_laplacian_3d_to(lat_ctx *h, int n1, int n2, int n3, const double *f, double *lap, double dk)
+{
     CTX_OR_FAIL(h);
     ONE_MEMBER(c);
-    if (!f) return -1;
+    if (!f || !lap) return -1;
     if (n1 != c.nx || n2 != c.ny || n3 != c.nz) {
         c.last_error = "lattice size differs from the context";
         return -2;
@@ -885,7 +1051,7 @@ int lat_laplacian_3d(lat_ctx *h, int n1, int n2, int n3, double *f, double dk)
     int rc = ensure_io(c);
     if (rc) return rc;
     cpx<double> *F = (cpx<double> *)c.Fk64;
-    LAT_HIP(&c, hipMemcpyAsync(c.io64, f, sizeof(double) * c.nvol, hipMemcpyHostToDevice, c.stream));
+    if ((rc = copy_to_device(c, c.io64, f, sizeof(double) * c.nvol))) return rc;
     if ((rc = launch_x_r2c<double>(c, c.twx64, c.io64, nullptr, F, 0))) return rc;
     if ((rc = launch_col<double>(c, c.twy64, F, 1, 0, 1))) return rc;
     const double saved = c.dk;
@@ -896,8 +1062,7 @@ int lat_laplacian_3d(lat_ctx *h, int n1, int n2, int n3, double *f, double dk)
     if ((rc = launch_col<double>(c, c.twy64, F, 1, 1, 1))) return rc;
     rc = launch_x_c2r<double>(c, c.twx64, F, 1, EPI_STORE, c.io64, nullptr, nullptr);
     if (rc < 0) return rc;
-    LAT_HIP(&c, hipMemcpyAsync(f, c.io64, sizeof(double) * c.nvol, hipMemcpyDeviceToHost, c.stream));
-    return sync(c);
+    return copy_to_host(c, lap, c.io64, sizeof(double) * c.nvol);
 }
 
 int lat_gradient_squared_3d(lat_ctx *h, const double *f, double *grad2, double dk)
@@ -922,8 +1087,7 @@ int lat_gradient_squared_3d(lat_ctx *h, const double *f, double *grad2, double d
         hipLaunchKernelGGL(k_sq_acc, dim3(4096), dim3(256), 0, c.stream, c.io64, acc, c.nvol, ax == 2 ? 1 : 0);
         LAT_HIP(&c, hipGetLastError());
     }
-    LAT_HIP(&c, hipMemcpyAsync(grad2, acc, sizeof(double) * c.nvol, hipMemcpyDeviceToHost, c.stream));
-    return sync(c);
+    return copy_to_host(c, grad2, acc, sizeof(double) * c.nvol);
 }
 
 int lat_stencil_laplacian(lat_ctx *h, const double *f, double *lap)
@@ -937,10 +1101,9 @@ int lat_stencil_laplacian(lat_ctx *h, const double *f, double *lap)
     }
     int rc = ensure_io(c);
     if (rc) return rc;
-    LAT_HIP(&c, hipMemcpyAsync(c.io64, f, sizeof(double) * c.nvol, hipMemcpyHostToDevice, c.stream));
+    if ((rc = copy_to_device(c, c.io64, f, sizeof(double) * c.nvol))) return rc;
     if ((rc = launch_stencil_io(c, c.io64, c.io64 + c.nvol))) return rc;
-    LAT_HIP(&c, hipMemcpyAsync(lap, c.io64 + c.nvol, sizeof(double) * c.nvol, hipMemcpyDeviceToHost, c.stream));
-    return sync(c);
+    return copy_to_host(c, lap, c.io64 + c.nvol, sizeof(double) * c.nvol);
 }
 
 } // extern "C"
@@ -984,9 +1147,10 @@ int lat_spectrum_3d(lat_ctx *h, double *S, const double *f, double *Fk)
     const cpx<double> *F = (const cpx<double> *)c.Fk64;
     if ((rc = launch_bin<double>(c, F, F, 0)) < 0) return rc;
     std::vector<double> raw(2 * c.ns);
-    LAT_HIP(&c, hipMemcpyAsync(raw.data(), c.spec_out, sizeof(double) * 2 * c.ns, hipMemcpyDeviceToHost, c.stream));
+    if ((rc = spec_fetch(c, raw.size()))) return rc;
     if (Fk && (rc = fk_to_host(c, F, Fk))) return rc;
     if ((rc = sync(c))) return rc;
+    spec_read(c, raw);
     double *outs[1] = {S};
     finish_spectra(raw, c.ns, 1, outs);
     return 0;
@@ -1014,8 +1178,9 @@ int lat_spectrum_discrete(lat_ctx *h, const double *f, double *S, int kind)
     const cpx<double> *F = (const cpx<double> *)c.Fk64;
     if ((rc = launch_bin<double>(c, F, F, 0, ns, kind == 1 ? BIN_COUNTS : 0)) < 0) return rc;
     std::vector<double> raw(2 * (size_t)ns);
-    LAT_HIP(&c, hipMemcpyAsync(raw.data(), c.spec_out, sizeof(double) * 2 * ns, hipMemcpyDeviceToHost, c.stream));
+    if ((rc = spec_fetch(c, raw.size()))) return rc;
     if ((rc = sync(c))) return rc;
+    spec_read(c, raw);
     double *outs[1] = {S};
     // kind 0: S/W/n^6 (analysis.f90:113); kind 1: S/W (analysis.f90:50)
     const double n3 = (double)c.nvol;
@@ -1043,8 +1208,9 @@ int lat_spectrum_discrete_k(lat_ctx *h, const double *Fk, double *S, int kind)
     const int flags = kind == 0 ? BIN_HALF : (BIN_HALF | BIN_NO_NYQ | BIN_COUNTS);
     if ((rc = launch_bin<double>(c, F, F, 0, ns, flags)) < 0) return rc;
     std::vector<double> raw(2 * (size_t)ns);
-    LAT_HIP(&c, hipMemcpyAsync(raw.data(), c.spec_out, sizeof(double) * 2 * ns, hipMemcpyDeviceToHost, c.stream));
+    if ((rc = spec_fetch(c, raw.size()))) return rc;
     if ((rc = sync(c))) return rc;
+    spec_read(c, raw);
     double *outs[1] = {S};
     const double n3 = (double)c.nvol;
     finish_spectra(raw, ns, 1, outs, kind == 0 ? n3 * n3 : 1.0); // analysis.f90:146 / :82
@@ -1082,8 +1248,9 @@ int lat_crossspec_discrete_k(lat_ctx *h, const double *Fk1, const double *Fk2, d
     const int ns = lat_num_bins_discrete(c.nx);
     if ((rc = launch_bin<double>(c, F1, F2, 1, ns, BIN_HALF | BIN_NO_NYQ)) < 0) return rc;
     std::vector<double> raw(3 * (size_t)ns);
-    LAT_HIP(&c, hipMemcpyAsync(raw.data(), c.spec_out, sizeof(double) * 3 * ns, hipMemcpyDeviceToHost, c.stream));
+    if ((rc = spec_fetch(c, raw.size()))) return rc;
     if ((rc = sync(c))) return rc;
+    spec_read(c, raw);
     double *outs[2] = {S1, S2};
     finish_spectra(raw, ns, 2, outs); // analysis.f90:183-184, no n^6
     return 0;
@@ -1103,8 +1270,9 @@ int lat_crossspec_3d(lat_ctx *h, const double *Fk1, const double *Fk2, double *S
     if ((rc = fk_from_host(c, F2, Fk2))) return rc;
     if ((rc = launch_bin<double>(c, F1, F2, 1)) < 0) return rc;
     std::vector<double> raw(3 * c.ns);
-    LAT_HIP(&c, hipMemcpyAsync(raw.data(), c.spec_out, sizeof(double) * 3 * c.ns, hipMemcpyDeviceToHost, c.stream));
+    if ((rc = spec_fetch(c, raw.size()))) return rc;
     if ((rc = sync(c))) return rc;
+    spec_read(c, raw);
     double *outs[2] = {S_re, S_im};
     finish_spectra(raw, c.ns, 2, outs);
     return 0;
@@ -1131,14 +1299,15 @@ static int output_spectra_t(Ctx &c, int field, double *out)
     // crossspec_3d(Fk = pi^, Fk2 = phi^) as called at evolve_spectral.f90:534-538
     if ((rc = launch_bin<T>(c, Fpi, Fphi, 2)) < 0) return rc;
     std::vector<double> raw(5 * c.ns);
-    LAT_HIP(&c, hipMemcpyAsync(raw.data(), c.spec_out, sizeof(double) * 5 * c.ns, hipMemcpyDeviceToHost, c.stream));
-    cpx<T> f0[2];
+    if ((rc = spec_fetch(c, raw.size()))) return rc;
+    cpx<T> *const f0 = reinterpret_cast<cpx<T> *>(c.stage->small + HostStage::MODES);
     if (sizeof(T) == 4) {
         LAT_HIP(&c, hipMemcpyAsync(&f0[0], Fphi, sizeof(cpx<T>), hipMemcpyDeviceToHost, c.stream));
         LAT_HIP(&c, hipMemcpyAsync(&f0[1], Fpi, sizeof(cpx<T>), hipMemcpyDeviceToHost, c.stream));
         if ((rc = pull_scalars(c))) return rc;
     }
     if ((rc = sync(c))) return rc;
+    spec_read(c, raw);
     if (sizeof(T) == 4) {
         // Mixed form: the FP32 transform holds the fluctuations only.  Bin 0 is
         // the k = 0 mode alone (weight 1): the FP64 mean times the volume plus

@@ -1171,9 +1171,7 @@ int lat_corrector_infer(lat_corrector *h, lat_ctx *ctx, float *out)
     if (rc) return rc;
     pack(net, c, c.fld, c.fldp);
     forward(net, false);
-    LAT_HIP(&c, hipMemcpyAsync(out, net.y, sizeof(float) * 4 * c.nvol, hipMemcpyDeviceToHost, c.stream));
-    LAT_HIP(&c, hipStreamSynchronize(c.stream));
-    return 0;
+    return copy_to_host(c, out, net.y, sizeof(float) * 4 * c.nvol);
 }
 
 // Loss and gradients for the current state of ctx as input and `target`
@@ -1188,9 +1186,10 @@ int lat_corrector_gradients(lat_corrector *h, lat_ctx *ctx, const float *target,
     Ctx &c = ctx->c;
     int rc = check_ctx(net, c);
     if (rc) return rc;
-    LAT_HIP(&c, hipMemcpyAsync(net.tgt, target, sizeof(float) * 4 * c.nvol, hipMemcpyHostToDevice, c.stream));
+    // the network's forward pass runs while the target is staged
     pack(net, c, c.fld, c.fldp);
     forward(net, true);
+    if ((rc = copy_to_device(c, net.tgt, target, sizeof(float) * 4 * c.nvol))) return rc;
     backward(net);
     std::vector<float> lp(1024);
     LAT_HIP(&c, hipMemcpyAsync(lp.data(), net.lossp, sizeof(float) * 1024, hipMemcpyDeviceToHost, c.stream));

@@ -53,7 +53,7 @@ class Config(ctypes.Structure):
 
 EXPORTS = [
     "lat_create", "lat_destroy", "lat_last_error", "lat_synchronize",
-    "lat_laplacian_3d", "lat_gradient_squared_3d", "lat_fft_r2c_3d", "lat_fft_c2r_3d",
+    "lat_laplacian_3d", "lat_laplacian_3d_to", "lat_gradient_squared_3d", "lat_fft_r2c_3d", "lat_fft_c2r_3d",
     "lat_stencil_laplacian", "lat_num_bins", "lat_spectrum_3d", "lat_crossspec_3d",
     "lat_output_spectra", "lat_set_state", "lat_get_state", "lat_get_scalars",
     "lat_set_scalars", "lat_split", "lat_symp_o2step", "lat_symp", "lat_calc_metric",
@@ -247,11 +247,12 @@ class Lattice:
     # ---------------------------------------------------------------- module fftw3
     def laplacian_3d(self, f, dk=None):
         """laplacian_3d (fftw_mod.f90:177-207); returns a new array."""
-        f = self._field(f).copy()
+        f = self._field(f)
+        out = np.empty_like(f)
         dk = self.dk if dk is None else dk
-        self._check(lib().lat_laplacian_3d(self._h, self.nx, self.ny, self.nz, _p(f), ctypes.c_double(dk)),
-                    "laplacian_3d")
-        return f
+        self._check(lib().lat_laplacian_3d_to(self._h, self.nx, self.ny, self.nz, _p(f), _p(out),
+                                              ctypes.c_double(dk)), "laplacian_3d")
+        return out
 
     def gradient_squared_3d(self, f, dk=None):
         f = self._field(f)

@@ -234,3 +234,20 @@ def test_gradient_squared_matches_oracle(gpu):
         g = lat.gradient_squared_3d(f)
     r = O.gradient_squared_3d(f, 2 * np.pi / L)
     assert np.abs(g - r).max() <= 1e-12 * np.abs(r).max()
+
+
+@pytest.mark.parametrize("n", [32, 128])
+def test_laplacian_out_of_place_equals_in_place(gpu, n):
+    """laplacian_3d into another array (through one staging slot, and through
+    the slots of several threads) leaves its input alone and gives the in-place
+    entry's result."""
+    import ctypes
+
+    print("case laplacian out of place", n, flush=True)
+    f = np.random.default_rng(n).standard_normal((n, n, n))
+    keep = f.copy()
+    with _lat(gpu, (n, n, n)) as lat:
+        out = lat.laplacian_3d(f)
+        g = f.copy()
+        assert gpu.lib().lat_laplacian_3d(lat._h, n, n, n, gpu._p(g), ctypes.c_double(lat.dk)) == 0
+    assert np.array_equal(f, keep) and np.array_equal(out, g)
