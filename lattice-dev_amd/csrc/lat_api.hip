@@ -328,19 +328,42 @@ static int forward_state(Ctx &c, bool drift, int zmode, int layout = 0)
     const T *fldp = (const T *)c.fldp;
     cpx<T> *Fk = (cpx<T> *)c.Fk;
     int rc;
-    for (int l = 0; l < c.nfld; ++l) {
+    if (plane_fwd_ok(c)) {
         StageTimer st(c, LAT_ST_X_R2C);
-        rc = launch_x_r2c<T>(c, twx, fld + (size_t)l * c.nvol, fldp + (size_t)l * c.nvol, Fk + (size_t)l * c.nk,
-                             drift ? 1 : 0, l, layout);
-        if (rc) return rc;
-    }
-    {
+        if ((rc = launch_plane_fwd<T>(c, twx, fld, fldp, Fk, c.nfld, drift ? 1 : 0, 0))) return rc;
+    } else {
+        for (int l = 0; l < c.nfld; ++l) {
+            StageTimer st(c, LAT_ST_X_R2C);
+            rc = launch_x_r2c<T>(c, twx, fld + (size_t)l * c.nvol, fldp + (size_t)l * c.nvol, Fk + (size_t)l * c.nk,
+                                 drift ? 1 : 0, l, layout);
+            if (rc) return rc;
+        }
         StageTimer st(c, LAT_ST_Y_FWD);
         if ((rc = launch_col<T>(c, twy, Fk, 1, 0, c.nfld, layout))) return rc;
     }
     StageTimer st(c, LAT_ST_Z_LAP);
     if ((rc = launch_col<T>(c, twz, Fk, 2, zmode, c.nfld, layout))) return rc;
     return 0;
+}
+
+// y inverse and x C2R + epilogue of nf arrays; returns the number of
+// reduction partials.
+template <typename T>
+static int inverse_state(Ctx &c, cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp, int layout = 0)
+{
+    const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
+    const cpx<T> *twy = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twy64 : (void *)c.twy32);
+    if (plane_inv_ok(c, nf)) {
+        StageTimer st(c, LAT_ST_X_C2R);
+        return launch_plane_inv<T>(c, twx, Fk, nf, epi, fld, fldp);
+    }
+    {
+        StageTimer st(c, LAT_ST_Y_INV);
+        const int rc = launch_col<T>(c, twy, Fk, 1, 1, nf, layout);
+        if (rc) return rc;
+    }
+    StageTimer st(c, LAT_ST_X_C2R);
+    return launch_x_c2r<T>(c, twx, Fk, nf, epi, nullptr, fld, fldp, layout);
 }
 
 // Laplacian of the state into the C2R epilogue: EPI_KICK or EPI_REDUCE.
@@ -364,12 +387,17 @@ static int gw_kick(Ctx &c, bool drift)
     int rc;
     for (int c0 = 0; c0 < 6; c0 += 2) {
         if ((rc = launch_gw_source<T>(c, c0, 2, src))) return rc;
-        for (int q = 0; q < 2; ++q) {
+        if (plane_fwd_ok(c)) {
             StageTimer st(c, LAT_ST_X_R2C);
-            const size_t off = (size_t)(c0 + q) * c.nvol;
-            if ((rc = launch_x_r2c<T>(c, twx, u + off, p + off, Fk + (size_t)q * c.nk, drift ? 1 : 0, -1))) return rc;
-        }
-        {
+            const size_t off = (size_t)c0 * c.nvol;
+            if ((rc = launch_plane_fwd<T>(c, twx, u + off, p + off, Fk, 2, drift ? 1 : 0, -1))) return rc;
+        } else {
+            for (int q = 0; q < 2; ++q) {
+                StageTimer st(c, LAT_ST_X_R2C);
+                const size_t off = (size_t)(c0 + q) * c.nvol;
+                if ((rc = launch_x_r2c<T>(c, twx, u + off, p + off, Fk + (size_t)q * c.nk, drift ? 1 : 0, -1)))
+                    return rc;
+            }
             StageTimer st(c, LAT_ST_Y_FWD);
             if ((rc = launch_col<T>(c, twy, Fk, 1, 0, 2))) return rc;
         }
@@ -377,12 +405,7 @@ static int gw_kick(Ctx &c, bool drift)
             StageTimer st(c, LAT_ST_Z_LAP);
             if ((rc = launch_col<T>(c, twz, Fk, 2, 2, 2))) return rc;
         }
-        {
-            StageTimer st(c, LAT_ST_Y_INV);
-            if ((rc = launch_col<T>(c, twy, Fk, 1, 1, 2))) return rc;
-        }
-        StageTimer st(c, LAT_ST_X_C2R);
-        rc = launch_x_c2r<T>(c, twx, Fk, 2, EPI_GWKICK, nullptr, src, p + (size_t)c0 * c.nvol);
+        rc = inverse_state<T>(c, Fk, 2, EPI_GWKICK, src, p + (size_t)c0 * c.nvol);
         if (rc < 0) return rc;
     }
     return 0;
@@ -426,17 +449,7 @@ static int state_force(Ctx &c, bool drift, int epi)
     const int layout = kblk_active(c);
     int rc = forward_state<T>(c, drift, 2, layout);
     if (rc) return rc;
-    const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
-    const cpx<T> *twy = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twy64 : (void *)c.twy32);
-    {
-        StageTimer st(c, LAT_ST_Y_INV);
-        if ((rc = launch_col<T>(c, twy, (cpx<T> *)c.Fk, 1, 1, c.nfld, layout))) return rc;
-    }
-    int g;
-    {
-        StageTimer st(c, LAT_ST_X_C2R);
-        g = launch_x_c2r<T>(c, twx, (cpx<T> *)c.Fk, c.nfld, epi, nullptr, (const T *)c.fld, (T *)c.fldp, layout);
-    }
+    const int g = inverse_state<T>(c, (cpx<T> *)c.Fk, c.nfld, epi, (const T *)c.fld, (T *)c.fldp, layout);
     if (g < 0) return g;
     if (gw && (rc = gw_kick<T>(c, drift))) return rc;
     return g;
@@ -2362,12 +2375,9 @@ static int force_multi(std::vector<Ctx *> &cs, bool drift, std::vector<int> &npa
 {
     const int K = (int)cs.size(), nf = cs[0]->nfld;
     int rc;
-    for (int l = 0; l < nf; ++l)
-        if ((rc = launch_x_r2c_multi<T>(cs.data(), K, l, drift ? 1 : 0))) return rc;
-    if ((rc = launch_col_multi<T>(cs.data(), K, 1, 0, nf))) return rc;
+    if ((rc = launch_fwd_multi<T>(cs.data(), K, nf, drift ? 1 : 0))) return rc;
     if ((rc = launch_col_multi<T>(cs.data(), K, 2, 2, nf))) return rc;
-    if ((rc = launch_col_multi<T>(cs.data(), K, 1, 1, nf))) return rc;
-    return launch_x_c2r_multi<T>(cs.data(), K, nf, EPI_KICK, npart.data());
+    return launch_inv_multi<T>(cs.data(), K, nf, EPI_KICK, npart.data());
 }
 
 static int run_ops_multi(std::vector<Ctx *> &cs, const std::vector<std::vector<Op>> &ops)
@@ -2483,27 +2493,15 @@ static int ens_sweeps(lat_ensemble *e, bool single)
     const int K = (int)cs.size(), nf = cs[0]->nfld;
     int rc;
     if (single) {
-        for (int l = 0; l < nf; ++l)
-            if ((rc = launch_x_r2c_multi<T>(cs.data(), K, l, 0))) return rc;
-        if ((rc = launch_col_multi<T>(cs.data(), K, 1, 0, nf))) return rc;
+        if ((rc = launch_fwd_multi<T>(cs.data(), K, nf, 0))) return rc;
         if ((rc = launch_col_multi<T>(cs.data(), K, 2, 2, nf))) return rc;
-        if ((rc = launch_col_multi<T>(cs.data(), K, 1, 1, nf))) return rc;
         std::vector<int> np(K);
-        return launch_x_c2r_multi<T>(cs.data(), K, nf, EPI_REDUCE, np.data());
+        return launch_inv_multi<T>(cs.data(), K, nf, EPI_REDUCE, np.data());
     }
     for (Ctx *cp : cs) {
         Ctx &c = *cp;
-        const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
-        const cpx<T> *twy = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twy64 : (void *)c.twy32);
-        const cpx<T> *twz = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twz64 : (void *)c.twz32);
-        cpx<T> *Fk = (cpx<T> *)c.Fk;
-        for (int l = 0; l < nf; ++l)
-            if ((rc = launch_x_r2c<T>(c, twx, (T *)c.fld + (size_t)l * c.nvol, nullptr, Fk + (size_t)l * c.nk, 0, l)))
-                return rc;
-        if ((rc = launch_col<T>(c, twy, Fk, 1, 0, nf))) return rc;
-        if ((rc = launch_col<T>(c, twz, Fk, 2, 2, nf))) return rc;
-        if ((rc = launch_col<T>(c, twy, Fk, 1, 1, nf))) return rc;
-        const int g = launch_x_c2r<T>(c, twx, Fk, nf, EPI_REDUCE, nullptr, (const T *)c.fld, (T *)c.fldp);
+        if ((rc = forward_state<T>(c, false, 2))) return rc;
+        const int g = inverse_state<T>(c, (cpx<T> *)c.Fk, nf, EPI_REDUCE, (const T *)c.fld, (T *)c.fldp);
         if (g < 0) return g;
     }
     return 0;

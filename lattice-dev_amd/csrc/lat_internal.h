@@ -215,6 +215,16 @@ template <typename T>
 int launch_x_c2r(Ctx &c, const cpx<T> *tw, cpx<T> *Fk, int nf, int epi, T *out, const T *fld, T *fldp,
                  int layout = 0);
 
+// ---- plane sweeps of small cubic lattices (lat_plane.hip) ----
+// x R2C + y forward of nf arrays (drift and field as in launch_x_r2c, field0
+// the first one's index); y inverse + x C2R + epilogue (as launch_x_c2r).
+bool plane_fwd_ok(const Ctx &c);
+bool plane_inv_ok(const Ctx &c, int nf);
+template <typename T>
+int launch_plane_fwd(Ctx &c, const cpx<T> *tw, T *f, const T *pi, cpx<T> *Fk, int nf, int drift, int field0);
+template <typename T>
+int launch_plane_inv(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp);
+
 // ---- separable spectral Laplacian (lat_sep.hip), mixed form ----
 // Kick of all fields with the three-sweep Laplacian (x: drift + D_xx; y:
 // += D_yy; z: + D_zz, kick, reductions).  *npart = reduction partials per
@@ -229,13 +239,14 @@ int launch_sep_kick(Ctx &c, int drift, int *npart);
 // Returns 0, or <0 (unsupported class set / HIP error).
 constexpr int MULTI_MAXC = 4;
 bool multi_supported(int n);
+// forward x and y of nf fields, the z pass, inverse y and x + epilogue
 template <typename T>
-int launch_x_r2c_multi(Ctx *const *cs, int ncls, int field, int drift);
+int launch_fwd_multi(Ctx *const *cs, int ncls, int nf, int drift);
 template <typename T>
 int launch_col_multi(Ctx *const *cs, int ncls, int axis, int mode, int n_arrays);
 // EPI_KICK or EPI_REDUCE; npart[k] = reduction partials per member of class k
 template <typename T>
-int launch_x_c2r_multi(Ctx *const *cs, int ncls, int nf, int epi, int *npart);
+int launch_inv_multi(Ctx *const *cs, int ncls, int nf, int epi, int *npart);
 
 // ---- step kernels (lat_step.hip) ----
 template <typename T>

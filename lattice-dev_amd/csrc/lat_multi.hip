@@ -10,12 +10,20 @@
 // reduction-partial slot of the class's own launch, so every member's
 // arithmetic is bitwise that of the one-class launch.  The FFT bodies are
 // specialised on the line length, so the kernel switches on the class's
-// size; LDS is dynamic, sized for the largest class of the launch.
-#include "sweeps.h"
+// size; LDS is dynamic, sized for the largest class of the launch.  Classes that
+// take the plane sweeps (planes.h) share a launch per number of threads per
+// plane instead of the x and y launches; every class shares the z launch.
+#include "planes.h"
 
 namespace lat {
 
 #define LAT_FOR_MULTI_SIZES(X) X(16) X(32) X(48) X(64) X(96) X(128) X(192) X(256)
+
+// sizes that take the separate x and y sweeps: forward only above 128, inverse
+// at 128 too where two planes do not fit the LDS (FP64)
+#define LAT_FOR_MULTI_LARGE(X) X(128) X(192) X(256)
+template <typename T, int N, bool INV>
+constexpr bool multi_sweep() { return INV ? !plane_inv_fits<T, N, 2>() : !plane_fwd_fits<T, N>(); }
 
 bool multi_supported(int n)
 {
@@ -128,10 +136,10 @@ __global__ __launch_bounds__(TPB) void k_x_r2c_multi(R2CArgs<T> a)
     if (!multi_block(a.m, k, bk)) return;
     const R2CCls<T> c = pick(a.c, k);
     switch (c.sel) {
-#define CASE(NN)                                                   \
-    case 2 * NN: r2c_case<T, NN, 0, DRIFT>(c, a.field, bk, lds); break; \
-    case 2 * NN + 1: r2c_case<T, NN, 1, DRIFT>(c, a.field, bk, lds); break;
-        LAT_FOR_MULTI_SIZES(CASE)
+#define CASE(NN)                                                                                             \
+    case 2 * NN: if constexpr (multi_sweep<T, NN, false>()) r2c_case<T, NN, 0, DRIFT>(c, a.field, bk, lds); break; \
+    case 2 * NN + 1: if constexpr (multi_sweep<T, NN, false>()) r2c_case<T, NN, 1, DRIFT>(c, a.field, bk, lds); break;
+        LAT_FOR_MULTI_LARGE(CASE)
 #undef CASE
     default:
         break;
@@ -179,9 +187,9 @@ __global__ __launch_bounds__(COL_MULTI_NT) void k_col_multi(ColArgs<T> a)
     if (!multi_block(a.m, k, bk)) return;
     const ColCls<T> c = pick(a.c, k);
     switch (c.sel) {
-#define CASE(NN)                                            \
-    case 2 * NN: col_case<T, NN, 0, MODE>(c, bk, lds); break; \
-    case 2 * NN + 1: col_case<T, NN, 1, MODE>(c, bk, lds); break;
+#define CASE(NN)                                                                                              \
+    case 2 * NN: if constexpr (MODE == 2 || multi_sweep<T, NN, MODE == 1>()) col_case<T, NN, 0, MODE>(c, bk, lds); break; \
+    case 2 * NN + 1: if constexpr (MODE == 2 || multi_sweep<T, NN, MODE == 1>()) col_case<T, NN, 1, MODE>(c, bk, lds); break;
         LAT_FOR_MULTI_SIZES(CASE)
 #undef CASE
     default:
@@ -228,10 +236,86 @@ __global__ __launch_bounds__(TPB) void k_x_c2r_multi(C2RArgs<T> a)
     if (!multi_block(a.m, k, bk)) return;
     const C2RCls<T> c = pick(a.c, k);
     switch (c.sel) {
-#define CASE(NN)                                               \
-    case 2 * NN: c2r_case<T, NN, 0, EPI>(c, a.nf, bk, lds); break; \
-    case 2 * NN + 1: c2r_case<T, NN, 1, EPI>(c, a.nf, bk, lds); break;
-        LAT_FOR_MULTI_SIZES(CASE)
+#define CASE(NN)                                                                                         \
+    case 2 * NN: if constexpr (multi_sweep<T, NN, true>()) c2r_case<T, NN, 0, EPI>(c, a.nf, bk, lds); break; \
+    case 2 * NN + 1: if constexpr (multi_sweep<T, NN, true>()) c2r_case<T, NN, 1, EPI>(c, a.nf, bk, lds); break;
+        LAT_FOR_MULTI_LARGE(CASE)
+#undef CASE
+    default:
+        break;
+    }
+}
+
+// ---------------------------------------------------------------- planes
+// Blocks of a class: its planes, field by field in the forward sweep.
+template <typename T>
+struct PlaneCls {
+    T *f, *p;
+    cpx<T> *Fk;
+    const cpx<T> *tw;
+    const DevScalars *dsc;
+    double *partials;
+    ModelDev md;
+    MemberStride ms;
+    size_t nk, nvol;
+    int P, n;
+};
+template <typename T>
+struct PlaneArgs {
+    MultiMap m;
+    PlaneCls<T> c[MULTI_MAXC];
+};
+
+template <typename T, int N, int NT, bool DRIFT>
+__device__ __forceinline__ void plane_fwd_case(const PlaneCls<T> &c, const Blk &bk, cpx<T> *lds)
+{
+    if constexpr (plane_nt<N>() == NT && plane_fwd_fits<T, N>()) {
+        const int l = bk.x / N;
+        plane_fwd_body<T, N, NT, DRIFT>(c.f + l * c.nvol, c.p + l * c.nvol, c.Fk + l * c.nk, c.tw, c.P, c.dsc, l, c.ms,
+                                        Blk{bk.x - l * N, N, bk.y}, lds, lds + plane_fwd_buf<T, N>());
+    }
+}
+
+template <typename T, int NT, bool DRIFT>
+__global__ __launch_bounds__(NT) void k_plane_fwd_multi(PlaneArgs<T> a)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char lat_dyn_lds[];
+    cpx<T> *lds = reinterpret_cast<cpx<T> *>(lat_dyn_lds);
+    int k;
+    Blk bk;
+    if (!multi_block(a.m, k, bk)) return;
+    const PlaneCls<T> c = pick(a.c, k);
+    switch (c.n) {
+#define CASE(NN) \
+    case NN: plane_fwd_case<T, NN, NT, DRIFT>(c, bk, lds); break;
+        LAT_FOR_PLANE_SIZES(CASE)
+#undef CASE
+    default:
+        break;
+    }
+}
+
+template <typename T, int N, int NT, int NF, int EPI>
+__device__ __forceinline__ void plane_inv_case(const PlaneCls<T> &c, const Blk &bk, cpx<T> *lds)
+{
+    if constexpr (plane_nt<N>() == NT && plane_inv_fits<T, N, NF>())
+        plane_inv_body<T, N, NT, NF, EPI>(c.Fk, c.tw, c.P, c.nk, c.nvol, c.f, c.p, c.dsc, c.md, c.partials, c.ms, bk,
+                                          lds, lds + plane_inv_buf<T, N, NF>());
+}
+
+template <typename T, int NT, int NF, int EPI>
+__global__ __launch_bounds__(NT) void k_plane_inv_multi(PlaneArgs<T> a)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char lat_dyn_lds[];
+    cpx<T> *lds = reinterpret_cast<cpx<T> *>(lat_dyn_lds);
+    int k;
+    Blk bk;
+    if (!multi_block(a.m, k, bk)) return;
+    const PlaneCls<T> c = pick(a.c, k);
+    switch (c.n) {
+#define CASE(NN) \
+    case NN: plane_inv_case<T, NN, NT, NF, EPI>(c, bk, lds); break;
+        LAT_FOR_PLANE_SIZES(CASE)
 #undef CASE
     default:
         break;
@@ -324,7 +408,7 @@ static int allow_lds(Ctx &c, K kernel, size_t bytes)
 }
 
 template <typename T>
-int launch_x_r2c_multi(Ctx *const *cs, int ncls, int field, int drift)
+static int launch_x_r2c_multi(Ctx *const *cs, int ncls, int field, int drift)
 {
     int rc = check_classes(cs, ncls);
     if (rc) return rc;
@@ -405,7 +489,7 @@ int launch_col_multi(Ctx *const *cs, int ncls, int axis, int mode, int n_arrays)
 }
 
 template <typename T>
-int launch_x_c2r_multi(Ctx *const *cs, int ncls, int nf, int epi, int *npart)
+static int launch_x_c2r_multi(Ctx *const *cs, int ncls, int nf, int epi, int *npart)
 {
     int rc = check_classes(cs, ncls);
     if (rc) return rc;
@@ -439,11 +523,139 @@ int launch_x_c2r_multi(Ctx *const *cs, int ncls, int nf, int epi, int *npart)
     return 0;
 }
 
-template int launch_x_r2c_multi<double>(Ctx *const *, int, int, int);
-template int launch_x_r2c_multi<float>(Ctx *const *, int, int, int);
+static int plane_threads(int n)
+{
+    switch (n) {
+#define CASE(NN) \
+    case NN: return plane_nt<NN>();
+        LAT_FOR_PLANE_SIZES(CASE)
+#undef CASE
+    }
+    return 0;
+}
+
+// LDS bytes of a plane of size n, without the reduction's static part
+template <typename T>
+static size_t plane_lds(int n, int nf)
+{
+    switch (n) {
+#define CASE(NN)                                                                                    \
+    case NN: return sizeof(cpx<T>) * (size_t)(NN + (nf == 0   ? plane_fwd_buf<T, NN>()              \
+                                                    : nf == 1 ? plane_inv_buf<T, NN, 1>()           \
+                                                              : plane_inv_buf<T, NN, 2>()));
+        LAT_FOR_PLANE_SIZES(CASE)
+#undef CASE
+    }
+    return 0;
+}
+
+// The classes cs[0 .. ncls) that share NT threads per plane, in one launch
+// (nf = 0: forward with nfld fields).
+template <typename T>
+static void plane_classes(PlaneArgs<T> &a, Ctx *const *cs, int ncls, int per_member, std::vector<Geo> &geo, int nf)
+{
+    for (int k = 0; k < ncls; ++k) {
+        Ctx &c = *cs[k];
+        geo[k] = Geo{c.nz * per_member, plane_lds<T>(c.nx, nf)};
+        const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
+        a.c[k] = PlaneCls<T>{(T *)c.fld, (T *)c.fldp, (cpx<T> *)c.Fk, twx, c.dsc, c.partials,
+                             ModelDev{c.cfg.model, c.nfld, c.cfg.model_params[0], c.cfg.model_params[1], c.gw_coup},
+                             c.ms, c.nk, c.nvol, c.P, c.nx};
+    }
+}
+
+template <typename T, int NT>
+static int plane_fwd_group(Ctx *const *cs, int ncls, int nf, int drift)
+{
+    PlaneArgs<T> a{};
+    std::vector<Geo> geo(ncls);
+    plane_classes<T>(a, cs, ncls, nf, geo, 0);
+    const int blocks = map_classes(a.m, geo, cs, ncls);
+    const size_t lds = max_lds(geo);
+    Ctx &c0 = *cs[0];
+    int rc;
+    if (drift) {
+        if ((rc = allow_lds(c0, k_plane_fwd_multi<T, NT, true>, lds))) return rc;
+        hipLaunchKernelGGL((k_plane_fwd_multi<T, NT, true>), dim3(blocks), dim3(NT), lds, c0.stream, a);
+    } else {
+        if ((rc = allow_lds(c0, k_plane_fwd_multi<T, NT, false>, lds))) return rc;
+        hipLaunchKernelGGL((k_plane_fwd_multi<T, NT, false>), dim3(blocks), dim3(NT), lds, c0.stream, a);
+    }
+    LAT_HIP(&c0, hipGetLastError());
+    return 0;
+}
+
+template <typename T, int NT, int NF, int EPI>
+static int plane_inv_go(Ctx *const *cs, int ncls)
+{
+    PlaneArgs<T> a{};
+    std::vector<Geo> geo(ncls);
+    plane_classes<T>(a, cs, ncls, 1, geo, NF);
+    const int blocks = map_classes(a.m, geo, cs, ncls);
+    const size_t lds = max_lds(geo);
+    Ctx &c0 = *cs[0];
+    const int rc = allow_lds(c0, k_plane_inv_multi<T, NT, NF, EPI>, lds);
+    if (rc) return rc;
+    hipLaunchKernelGGL((k_plane_inv_multi<T, NT, NF, EPI>), dim3(blocks), dim3(NT), lds, c0.stream, a);
+    LAT_HIP(&c0, hipGetLastError());
+    return 0;
+}
+
+template <typename T, int NT>
+static int plane_inv_group(Ctx *const *cs, int ncls, int nf, int epi)
+{
+    if (nf == 1)
+        return epi == EPI_KICK ? plane_inv_go<T, NT, 1, EPI_KICK>(cs, ncls) : plane_inv_go<T, NT, 1, EPI_REDUCE>(cs, ncls);
+    return epi == EPI_KICK ? plane_inv_go<T, NT, 2, EPI_KICK>(cs, ncls) : plane_inv_go<T, NT, 2, EPI_REDUCE>(cs, ncls);
+}
+
+template <typename T>
+int launch_fwd_multi(Ctx *const *cs, int ncls, int nf, int drift)
+{
+    int rc = check_classes(cs, ncls);
+    if (rc) return rc;
+    std::vector<Ctx *> sw, p256, p512;
+    for (int k = 0; k < ncls; ++k)
+        (!plane_fwd_ok(*cs[k]) ? sw : plane_threads(cs[k]->nx) == 256 ? p256 : p512).push_back(cs[k]);
+    if (!p256.empty() && (rc = plane_fwd_group<T, 256>(p256.data(), (int)p256.size(), nf, drift))) return rc;
+    if (!p512.empty() && (rc = plane_fwd_group<T, 512>(p512.data(), (int)p512.size(), nf, drift))) return rc;
+    if (sw.empty()) return 0;
+    for (int l = 0; l < nf; ++l)
+        if ((rc = launch_x_r2c_multi<T>(sw.data(), (int)sw.size(), l, drift))) return rc;
+    return launch_col_multi<T>(sw.data(), (int)sw.size(), 1, 0, nf);
+}
+
+template <typename T>
+int launch_inv_multi(Ctx *const *cs, int ncls, int nf, int epi, int *npart)
+{
+    int rc = check_classes(cs, ncls);
+    if (rc) return rc;
+    if (nf < 1 || nf > 2 || (epi != EPI_KICK && epi != EPI_REDUCE)) return -1;
+    std::vector<Ctx *> sw, p256, p512;
+    std::vector<int> at, np(ncls);
+    for (int k = 0; k < ncls; ++k) {
+        npart[k] = cs[k]->nz;
+        if (!plane_inv_ok(*cs[k], nf)) {
+            sw.push_back(cs[k]);
+            at.push_back(k);
+        } else {
+            (plane_threads(cs[k]->nx) == 256 ? p256 : p512).push_back(cs[k]);
+        }
+    }
+    if (!p256.empty() && (rc = plane_inv_group<T, 256>(p256.data(), (int)p256.size(), nf, epi))) return rc;
+    if (!p512.empty() && (rc = plane_inv_group<T, 512>(p512.data(), (int)p512.size(), nf, epi))) return rc;
+    if (sw.empty()) return 0;
+    if ((rc = launch_col_multi<T>(sw.data(), (int)sw.size(), 1, 1, nf))) return rc;
+    if ((rc = launch_x_c2r_multi<T>(sw.data(), (int)sw.size(), nf, epi, np.data()))) return rc;
+    for (size_t q = 0; q < sw.size(); ++q) npart[at[q]] = np[q];
+    return 0;
+}
+
+template int launch_fwd_multi<double>(Ctx *const *, int, int, int);
+template int launch_fwd_multi<float>(Ctx *const *, int, int, int);
+template int launch_inv_multi<double>(Ctx *const *, int, int, int, int *);
+template int launch_inv_multi<float>(Ctx *const *, int, int, int, int *);
 template int launch_col_multi<double>(Ctx *const *, int, int, int, int);
 template int launch_col_multi<float>(Ctx *const *, int, int, int, int);
-template int launch_x_c2r_multi<double>(Ctx *const *, int, int, int, int *);
-template int launch_x_c2r_multi<float>(Ctx *const *, int, int, int, int *);
 
 } // namespace lat

@@ -80,10 +80,10 @@ __device__ __forceinline__ int kspace_row(int row)
 }
 
 // ---------------------------------------------------------------- block reduction
-template <int NCH>
+template <int NCH, int NT = TPB>
 __device__ __forceinline__ void block_reduce_store(double (&v)[NCH], double *out)
 {
-    __shared__ double red[NCH][TPB / 64];
+    __shared__ double red[NCH][NT / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
@@ -96,10 +96,89 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NCH], double *out
     if (threadIdx.x < NCH) {
         double s = 0.0;
 #pragma unroll
-        for (int w = 0; w < TPB / 64; ++w) s += red[threadIdx.x][w];
+        for (int w = 0; w < NT / 64; ++w) s += red[threadIdx.x][w];
         out[threadIdx.x] = s;
     }
 }
+
+// ---------------------------------------------------------------- kick epilogue
+// Per-site work of the kick, reduce and tensor-kick epilogues on a vector of
+// sites (x_c2r_body, plane_inv_body).
+template <typename T, int EPI>
+struct EpiEnv {
+    static constexpr int MAXF = 2, VW = 16 / sizeof(T);
+    ModelDev md;
+    T hA = 0, hB = 0;
+    float pb32[MAXF] = {0, 0};
+    double pb64[MAXF] = {0, 0};
+    T mu[MAXF] = {0, 0};
+    __device__ __forceinline__ EpiEnv(const DevScalars *__restrict__ dsc, const ModelDev &m) : md(m)
+    {
+        md.p0 = dsc->mp[0];
+        md.p1 = dsc->mp[1];
+        md.p2 = dsc->mp[2];
+        if constexpr (EPI == EPI_KICK || EPI == EPI_GWKICK) {
+            hA = T(dsc->hA);
+            hB = T(dsc->hB);
+        }
+        if constexpr (sizeof(T) == 4 && (EPI == EPI_KICK || EPI == EPI_REDUCE)) {
+            for (int fi = 0; fi < MAXF; ++fi) {
+                pb64[fi] = dsc->mean_phi[fi];
+                pb32[fi] = float(pb64[fi]);
+                if constexpr (EPI == EPI_KICK) mu[fi] = T(dsc->mu[fi]);
+            }
+        }
+    }
+    // lap, phi (GW: the source S) and pi of nf fields (components) at VW
+    // sites; pi is updated, the reductions go to acc (RedChan order).  Field
+    // loops are unrolled over MAXF with an nf guard so that every register
+    // array is indexed by compile-time constants.
+    __device__ __forceinline__ void sites(int nf, const Vec16<T> (&lap)[MAXF], const Vec16<T> (&ph)[MAXF],
+                                          Vec16<T> (&pv)[MAXF], double (&acc)[NRED]) const
+    {
+        if constexpr (EPI == EPI_GWKICK) {
+            const T gwc = T(md.gwc);
+#pragma unroll
+            for (int fi = 0; fi < MAXF; ++fi) {
+                if (fi >= nf) break;
+#pragma unroll
+                for (int v = 0; v < VW; ++v)
+                    pv[fi].e[v] = pv[fi].e[v] + hA * (lap[fi].e[v] + gwc * ph[fi].e[v]);
+            }
+        } else {
+#pragma unroll
+            for (int v = 0; v < VW; ++v) {
+                T phi[MAXF] = {0, 0}, dv[MAXF] = {0, 0};
+#pragma unroll
+                for (int fi = 0; fi < MAXF; ++fi)
+                    if (fi < nf) phi[fi] = ph[fi].e[v];
+                if constexpr (sizeof(T) == 4) {
+                    // mixed form: phi, p hold fluctuations; V' and V as differences
+                    if constexpr (EPI == EPI_KICK) model_ddv(md, pb32, phi, dv);
+                    acc[RC_PE] += model_dvv(md, pb64, phi);
+                } else {
+                    if constexpr (EPI == EPI_KICK) model_dv(md, phi, dv);
+                    acc[RC_PE] += model_v(md, phi);
+                }
+                acc[RC_M1] += double(phi[0]);
+                acc[RC_M2] += double(phi[1]);
+#pragma unroll
+                for (int fi = 0; fi < MAXF; ++fi) {
+                    if (fi >= nf) break;
+                    T p = pv[fi].e[v];
+                    if constexpr (EPI == EPI_KICK) {
+                        p = p + (hA * lap[fi].e[v] - hB * dv[fi]);
+                        if constexpr (sizeof(T) == 4) p = p - mu[fi];
+                        pv[fi].e[v] = p;
+                    }
+                    acc[RC_GE] -= double(phi[fi]) * double(lap[fi].e[v]);
+                    acc[RC_KE] += double(p) * double(p);
+                    acc[RC_S1 + fi] += double(p);
+                }
+            }
+        }
+    }
+};
 
 // ---------------------------------------------------------------- x R2C
 // With DRIFT: phi += dc0*pi (+ dc1*pi) first, written back (mixed form: on
@@ -409,25 +488,8 @@ __device__ __forceinline__ void x_c2r_body(const cpx<T> *__restrict__ Fk, const 
     if (fldp) fldp += bk.y * ms.f;
     dsc += bk.y;
     partials += (size_t)bk.y * MAX_GRID * NRED;
-    md.p0 = dsc->mp[0];
-    md.p1 = dsc->mp[1];
-    md.p2 = dsc->mp[2];
+    const EpiEnv<T, EPI> env(dsc, md);
     double acc[NRED] = {0, 0, 0, 0, 0, 0, 0, 0}; // RedChan order
-    T hA = 0, hB = 0;
-    if constexpr (EPI == EPI_KICK || EPI == EPI_GWKICK) {
-        hA = T(dsc->hA);
-        hB = T(dsc->hB);
-    }
-    float pb32[MAXF] = {0, 0};
-    double pb64[MAXF] = {0, 0};
-    T mu[MAXF] = {0, 0};
-    if constexpr (sizeof(T) == 4 && (EPI == EPI_KICK || EPI == EPI_REDUCE)) {
-        for (int fi = 0; fi < MAXF; ++fi) {
-            pb64[fi] = dsc->mean_phi[fi];
-            pb32[fi] = float(pb64[fi]);
-            if constexpr (EPI == EPI_KICK) mu[fi] = T(dsc->mu[fi]);
-        }
-    }
     constexpr int VW = 16 / sizeof(T); // reals per 16-byte lane access
     using VT = Vec16<T>;
     // k-space units of 16 bytes per row: complex pairs in FP32 (the odd last
@@ -529,9 +591,7 @@ __device__ __forceinline__ void x_c2r_body(const cpx<T> *__restrict__ Fk, const 
         if (nf == 2) lds_fft_range<T, M, +1, 2 * L, TPB, false, 2, 0, num_passes(M, MR), MR>(buf, LS, 1, twp);
         else lds_fft_range<T, M, +1, L, TPB, false, 2, 0, num_passes(M, MR), MR>(buf, LS, 1, twp);
         // 4. epilogue: VW consecutive sites per thread, every global access a
-        //    16-byte vector per lane (4 sites in FP32, 2 in FP64).  Field loops
-        //    are unrolled over MAXF with an nf guard so that every register
-        //    array is indexed by compile-time constants.
+        //    16-byte vector per lane (4 sites in FP32, 2 in FP64)
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int idx = threadIdx.x + it * TPB;
@@ -549,51 +609,10 @@ __device__ __forceinline__ void x_c2r_body(const cpx<T> *__restrict__ Fk, const 
 #pragma unroll
                 for (int fi = 0; fi < MAXF; ++fi)
                     if (fi < nf) *reinterpret_cast<VT *>(out + (size_t)fi * nvol + site) = lap[fi];
-            } else if constexpr (EPI == EPI_GWKICK) {
-                // tensor components: phv holds the source S, pv the momenta pi_u
-                if constexpr (!PRE) load_state(it);
-                const T gwc = T(md.gwc);
-#pragma unroll
-                for (int fi = 0; fi < MAXF; ++fi) {
-                    if (fi >= nf) break;
-#pragma unroll
-                    for (int v = 0; v < VW; ++v)
-                        pv[it][fi].e[v] = pv[it][fi].e[v] + hA * (lap[fi].e[v] + gwc * phv[it][fi].e[v]);
-                    *reinterpret_cast<VT *>(fldp + (size_t)fi * nvol + site) = pv[it][fi];
-                }
             } else {
                 if constexpr (!PRE) load_state(it);
-#pragma unroll
-                for (int v = 0; v < VW; ++v) {
-                    T phi[MAXF] = {0, 0}, dv[MAXF] = {0, 0};
-#pragma unroll
-                    for (int fi = 0; fi < MAXF; ++fi)
-                        if (fi < nf) phi[fi] = phv[it][fi].e[v];
-                    if constexpr (sizeof(T) == 4) {
-                        // mixed form: phi, p hold fluctuations; V' and V as differences
-                        if constexpr (EPI == EPI_KICK) model_ddv(md, pb32, phi, dv);
-                        acc[RC_PE] += model_dvv(md, pb64, phi);
-                    } else {
-                        if constexpr (EPI == EPI_KICK) model_dv(md, phi, dv);
-                        acc[RC_PE] += model_v(md, phi);
-                    }
-                    acc[RC_M1] += double(phi[0]);
-                    acc[RC_M2] += double(phi[1]);
-#pragma unroll
-                    for (int fi = 0; fi < MAXF; ++fi) {
-                        if (fi >= nf) break;
-                        T p = pv[it][fi].e[v];
-                        if constexpr (EPI == EPI_KICK) {
-                            p = p + (hA * lap[fi].e[v] - hB * dv[fi]);
-                            if constexpr (sizeof(T) == 4) p = p - mu[fi];
-                            pv[it][fi].e[v] = p;
-                        }
-                        acc[RC_GE] -= double(phi[fi]) * double(lap[fi].e[v]);
-                        acc[RC_KE] += double(p) * double(p);
-                        acc[RC_S1 + fi] += double(p);
-                    }
-                }
-                if constexpr (EPI == EPI_KICK) {
+                env.sites(nf, lap, phv[it], pv[it], acc);
+                if constexpr (EPI != EPI_REDUCE) {
 #pragma unroll
                     for (int fi = 0; fi < MAXF; ++fi)
                         if (fi < nf) *reinterpret_cast<VT *>(fldp + (size_t)fi * nvol + site) = pv[it][fi];

@@ -108,6 +108,28 @@ def test_single_splits_match_oracle(gpu, case):
     assert abs(g[3] - o[3]) < 1e-12 * abs(o[3])
 
 
+@pytest.mark.parametrize("shape", [(16, 16, 8), (32, 32, 64), (48, 48, 16), (64, 64, 32), (96, 96, 8), (128, 128, 16)])
+@pytest.mark.parametrize("nfld", [1, 2])
+def test_plane_sweeps_match_oracle(gpu, shape, nfld):
+    """Spectral steps of lattices with nx = ny (the plane sweeps; at 128 per
+    side FP64 takes the inverse one with one field only) and nz of its own."""
+    print("case planes", shape, nfld, flush=True)
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx + nz)
+    fld = 1e-3 * rng.standard_normal((nfld, nz, ny, nx))
+    fldp = 1e-3 * rng.standard_normal((nfld, nz, ny, nx))
+    fld[0] += 1.0
+    fldp[0] -= 0.6
+    phi4 = nfld == 1
+    g, o = run_pair(gpu, shape, 0.05 * nx, nfld, O.CONFORMAL if phi4 else O.COSMIC,
+                    O.MODEL_PHI4 if phi4 else O.MODEL_TWOFIELD, (1.0,) if phi4 else (1.0, 2.5e5), O.LAP_SPECTRAL,
+                    (-6, 1, 0, 0, 1), fld, fldp, [("symp", (4, 1e-3, 2)), ("Hamiltonian_Split", (1e-3, 3))])
+    assert rel(g[0], o[0]) < 1e-12 and rel(g[1], o[1]) < 1e-12
+    assert abs(g[2] - o[2]) < 1e-13 * abs(o[2]) and abs(g[3] - o[3]) < 1e-11 * abs(o[3])
+    for k in ("rho", "ke", "pe", "ge"):
+        assert abs(g[4][k] - o[4][k]) <= 1e-11 * abs(o[4][k]), k
+
+
 FD_SHAPES = [(8, 8, 64), (16, 48, 8), (96, 32, 8), (192, 8, 16), (64, 192, 8), (128, 16, 96)]
 
 
