@@ -100,12 +100,15 @@ int  lat_member(lat_ctx *batch, int member, lat_ctx **view);
  * context's stream; *gbps = 2 * bytes * reps / time. */
 int  lat_copy_bandwidth(lat_ctx *ctx, size_t bytes, int reps, double *gbps);
 
-/* Autotuner (no reference counterpart): for lattices of up to 256 per axis,
+/* Autotuner (no reference counterpart): for lattices of up to 512 per axis,
  * times two launch shapes of each sweep of the spectral Laplacian (x R2C and
  * x C2R rows per workgroup, y and z columns per tile) on the context's arrays
  * and keeps the faster; fields are not modified.  Ensembles tune every size
- * class at creation.  lat_tuning reports the choices (0 = default shape):
- * out[4] = {x R2C, y, z, x C2R}. */
+ * class at creation.  lat_tuning reports the shapes in use (0 or 1 each; a
+ * context starts with those measured faster for its size):
+ * out[4] = {x R2C, y, z, x C2R}.  Lattices with nx = ny up to 128 take the x and
+ * y passes of a force evaluation plane by plane: there the x and y shapes
+ * serve the output transforms only. */
 /* Form of the spectral Laplacian in the field kicks (no reference
  * counterpart; the reference has the 3-D form only): 0 = five HBM sweeps
  * (x R2C, y, z * -k^2, y, x C2R + kick), 1 = the same operator as the sum of

@@ -134,9 +134,17 @@ __global__ __launch_bounds__(256) void k_stage(uint4 *__restrict__ dst, const ui
 static int stage_copy(Ctx &c, bool to_host, char *dev, size_t dpitch, char *host, size_t width, size_t rows)
 {
     if (!width || !rows) return 0;
+    HostStage &h = *c.stage;
+    if (!h.ring && width * rows < (size_t)256 << 10) {
+        // a small lattice: not worth the ring's allocation (70 us)
+        if (to_host)
+            LAT_HIP(&c, hipMemcpy2DAsync(host, width, dev, dpitch, width, rows, hipMemcpyDeviceToHost, c.stream));
+        else
+            LAT_HIP(&c, hipMemcpy2DAsync(dev, dpitch, host, width, width, rows, hipMemcpyHostToDevice, c.stream));
+        return sync(c);
+    }
     int rc = stage_ring(c);
     if (rc) return rc;
-    HostStage &h = *c.stage;
     const Chunks ck(width, rows);
     // a thread costs about 20 us to start: from 8 chunks on
     const size_t T = ck.count >= 8 ? HostStage::THREADS : 1;
@@ -799,6 +807,26 @@ extern "C" {
 
 } // extern "C"
 
+// Launch shapes of a new context.  The second shape of the x and y sweeps
+// (half the rows, half the columns per workgroup: fewer registers and less
+// LDS, so more waves per SIMD) is the faster one, but for the x C2R of
+// 512-site rows in FP64; so is that of the z pass on lines of 128 and 256, and of
+// 96 and 192 in FP64 (in FP32 their half tile is 16 or 32 columns, from 42 or
+// 64).  Per kick of two fields, one lattice / three in turn, first shapes
+// against these: 256^3 mixed 440 -> 390 / 435 -> 412 us, FP64 838 -> 829 / 881 ->
+// 894; 192^3 mixed 240 -> 212 / 205 -> 192, FP64 418 -> 334 / 373 -> 351;
+// 256 x 192 x 128 mixed 211 -> 165 / 171 -> 147; 512 x 512 x 256 mixed 1815 ->
+// 1654 / 1761 -> 1658, and at 512^3 the z pass's second shape costs 3 %.
+static Ctx::Tune default_tune(const Ctx &c)
+{
+    const bool f64 = c.prec == LAT_F64;
+    Ctx::Tune t;
+    t.r2c = t.coly = 1;
+    t.c2r = !(f64 && c.nx == 512);
+    t.colz = c.nz == 128 || c.nz == 256 || (f64 && (c.nz == 96 || c.nz == 192));
+    return t;
+}
+
 // B realisations of one configuration; mparams (B x 4, nullable) overrides
 // lat_config.model_params per member.
 static int create_ctx(const lat_config *cfg, int B, const double *mparams, lat_ctx **out)
@@ -838,6 +866,7 @@ static int create_ctx(const lat_config *cfg, int B, const double *mparams, lat_c
         const int nd = lat_num_bins_discrete(nmax);
         c.spec_cap = c.ns > nd ? c.ns : nd;
     }
+    c.tune = default_tune(c);
     c.B = B;
     c.mvalid.assign(B, 0);
     c.ms.f = (size_t)c.nfld * c.nvol;

@@ -680,8 +680,9 @@ struct ColCfg {
 
 #define LAT_FOR_SIZES(X) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(48) X(96) X(192)
 
-// Sizes up to 256 carry a second launch shape per sweep that the autotuner
-// (lat_autotune) may pick: half the rows per workgroup for the x sweeps; for
+// Sizes up to 512 carry a second launch shape per sweep, which contexts start
+// with where it is the faster one (default_tune) and the autotuner (lat_autotune)
+// may pick: half the rows per workgroup for the x sweeps; for
 // the y/z sweeps the largest power-of-two column count up to half the
 // default (whole 8-byte-multiple row segments: 192^3 takes 16, not 21), run
 // by exactly the threads of its first pass, rounded to whole waves (the
@@ -689,7 +690,7 @@ struct ColCfg {
 // 0.418 -> 0.357 ms and fused z pass 0.546 -> 0.402 ms (32 columns, 256
 // threads), 192^3 y pass 0.462 -> 0.398 ms (16 columns, 192 threads).
 template <int N>
-constexpr bool tunable() { return N <= 256; }
+constexpr bool tunable() { return N <= 512; }
 constexpr int pow2_floor(int v) { return v >= 2 ? 2 * pow2_floor(v / 2) : 1; }
 template <typename T, int N>
 constexpr int col_tc(int mode, int v)
