@@ -324,6 +324,20 @@ static int kblk_active(const Ctx &c)
     return c.kblk && c.nx == c.ny && c.nx == c.nz && (c.nx == 256 || c.nx == 1024) ? 1 : 0;
 }
 
+// x R2C and y forward of nf arrays (nvol apart) into Fk (nk apart), no drift.
+template <typename T>
+static int forward_xy(Ctx &c, T *f, cpx<T> *Fk, int nf)
+{
+    const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
+    const cpx<T> *twy = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twy64 : (void *)c.twy32);
+    if (plane_fwd_ok<T>(c)) return launch_plane_fwd<T>(c, twx, f, nullptr, Fk, nf, 0, -1);
+    for (int l = 0; l < nf; ++l) {
+        const int rc = launch_x_r2c<T>(c, twx, f + (size_t)l * c.nvol, nullptr, Fk + (size_t)l * c.nk, 0, -1);
+        if (rc) return rc;
+    }
+    return launch_col<T>(c, twy, Fk, 1, 0, nf);
+}
+
 // Forward R2C (x, y, z) of the nfld state fields into Fk; drift fused if asked.
 // layout 1: the blocked order (zmode 2 only: the transforms stay internal).
 template <typename T>
@@ -336,7 +350,7 @@ static int forward_state(Ctx &c, bool drift, int zmode, int layout = 0)
     const T *fldp = (const T *)c.fldp;
     cpx<T> *Fk = (cpx<T> *)c.Fk;
     int rc;
-    if (plane_fwd_ok(c)) {
+    if (plane_fwd_ok<T>(c)) {
         StageTimer st(c, LAT_ST_X_R2C);
         if ((rc = launch_plane_fwd<T>(c, twx, fld, fldp, Fk, c.nfld, drift ? 1 : 0, 0))) return rc;
     } else {
@@ -357,13 +371,13 @@ static int forward_state(Ctx &c, bool drift, int zmode, int layout = 0)
 // y inverse and x C2R + epilogue of nf arrays; returns the number of
 // reduction partials.
 template <typename T>
-static int inverse_state(Ctx &c, cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp, int layout = 0)
+static int inverse_state(Ctx &c, cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp, int layout = 0, int gwc0 = 0)
 {
     const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
     const cpx<T> *twy = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twy64 : (void *)c.twy32);
-    if (plane_inv_ok(c, nf)) {
+    if (plane_inv_ok<T>(c, nf)) {
         StageTimer st(c, LAT_ST_X_C2R);
-        return launch_plane_inv<T>(c, twx, Fk, nf, epi, fld, fldp);
+        return launch_plane_inv<T>(c, twx, Fk, nf, epi, fld, fldp, gwc0);
     }
     {
         StageTimer st(c, LAT_ST_Y_INV);
@@ -371,15 +385,15 @@ static int inverse_state(Ctx &c, cpx<T> *Fk, int nf, int epi, const T *fld, T *f
         if (rc) return rc;
     }
     StageTimer st(c, LAT_ST_X_C2R);
-    return launch_x_c2r<T>(c, twx, Fk, nf, epi, nullptr, fld, fldp, layout);
+    return launch_x_c2r<T>(c, twx, Fk, nf, epi, nullptr, fld, fldp, layout, gwc0);
 }
 
 // Laplacian of the state into the C2R epilogue: EPI_KICK or EPI_REDUCE.
 // Returns the number of reduction partials (>0) or an error (<0).
 // Kick of the metric perturbations after the field kick of the same step (the
 // fields hold the drifted phi the source needs).  Spectral: three pairs of
-// components, each S_ij pair -> x R2C (pending drift of u fused) -> y -> z lap
-// -> y -> x C2R with pi_u += hA (lap + gw_coup S).  FD: one stencil sweep.
+// components, each x R2C (pending drift of u fused) -> y -> z lap -> y -> x C2R
+// with pi_u += hA (lap + gw_coup S), S formed there.  FD: one stencil sweep.
 template <typename T>
 static int gw_kick(Ctx &c, bool drift)
 {
@@ -390,12 +404,11 @@ static int gw_kick(Ctx &c, bool drift)
     const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
     const cpx<T> *twy = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twy64 : (void *)c.twy32);
     const cpx<T> *twz = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twz64 : (void *)c.twz32);
-    T *u = (T *)c.gwu, *p = (T *)c.gwp, *src = (T *)c.gwsrc;
+    T *u = (T *)c.gwu, *p = (T *)c.gwp;
     cpx<T> *Fk = (cpx<T> *)c.Fk;
     int rc;
     for (int c0 = 0; c0 < 6; c0 += 2) {
-        if ((rc = launch_gw_source<T>(c, c0, 2, src))) return rc;
-        if (plane_fwd_ok(c)) {
+        if (plane_fwd_ok<T>(c)) {
             StageTimer st(c, LAT_ST_X_R2C);
             const size_t off = (size_t)c0 * c.nvol;
             if ((rc = launch_plane_fwd<T>(c, twx, u + off, p + off, Fk, 2, drift ? 1 : 0, -1))) return rc;
@@ -413,7 +426,7 @@ static int gw_kick(Ctx &c, bool drift)
             StageTimer st(c, LAT_ST_Z_LAP);
             if ((rc = launch_col<T>(c, twz, Fk, 2, 2, 2))) return rc;
         }
-        rc = inverse_state<T>(c, Fk, 2, EPI_GWKICK, src, p + (size_t)c0 * c.nvol);
+        rc = inverse_state<T>(c, Fk, 2, EPI_GWKICK, (const T *)c.fld, p + (size_t)c0 * c.nvol, 0, c0);
         if (rc < 0) return rc;
     }
     return 0;
@@ -721,8 +734,7 @@ static int host_r2c(Ctx &c, const double *f_host)
     if (rc) return rc;
     if ((rc = copy_to_device(c, c.io64, f_host, sizeof(double) * c.nvol))) return rc;
     cpx<double> *F = (cpx<double> *)c.Fk64;
-    if ((rc = launch_x_r2c<double>(c, c.twx64, c.io64, nullptr, F, 0))) return rc;
-    if ((rc = launch_col<double>(c, c.twy64, F, 1, 0, 1))) return rc;
+    if ((rc = forward_xy<double>(c, c.io64, F, 1))) return rc;
     return launch_col<double>(c, c.twz64, F, 2, 0, 1);
 }
 
@@ -889,7 +901,6 @@ static int create_ctx(const lat_config *cfg, int B, const double *mparams, lat_c
     if (c.gw) {
         rc |= ensure(c, &c.gwu, es * 6 * c.nvol, "hipMalloc gwu");
         rc |= ensure(c, &c.gwp, es * 6 * c.nvol, "hipMalloc gwp");
-        if (cfg->laplacian == LAT_LAP_SPECTRAL) rc |= ensure(c, &c.gwsrc, es * 2 * c.nvol, "hipMalloc gwsrc");
     }
     if (cfg->laplacian == LAT_LAP_STENCIL && !c.gw) {
         // second state arrays of the fused drift + kick sweep, where they
@@ -1094,8 +1105,7 @@ int lat_laplacian_3d_to(lat_ctx *h, int n1, int n2, int n3, const double *f, dou
     if (rc) return rc;
     cpx<double> *F = (cpx<double> *)c.Fk64;
     if ((rc = copy_to_device(c, c.io64, f, sizeof(double) * c.nvol))) return rc;
-    if ((rc = launch_x_r2c<double>(c, c.twx64, c.io64, nullptr, F, 0))) return rc;
-    if ((rc = launch_col<double>(c, c.twy64, F, 1, 0, 1))) return rc;
+    if ((rc = forward_xy<double>(c, c.io64, F, 1))) return rc;
     const double saved = c.dk;
     c.dk = dk;
     rc = launch_col<double>(c, c.twz64, F, 2, 2, 1);
@@ -1334,9 +1344,14 @@ static int output_spectra_t(Ctx &c, int field, double *out)
     cpx<T> *Fpi = Fphi + c.nk;
     T *fld = (T *)c.fld + (size_t)field * c.nvol;
     T *fldp = (T *)c.fldp + (size_t)field * c.nvol;
-    if ((rc = launch_x_r2c<T>(c, twx, fld, nullptr, Fphi, 0))) return rc;
-    if ((rc = launch_x_r2c<T>(c, twx, fldp, nullptr, Fpi, 0))) return rc;
-    if ((rc = launch_col<T>(c, twy, Fphi, 1, 0, 2))) return rc;
+    if (plane_fwd_ok<T>(c)) {
+        if ((rc = forward_xy<T>(c, fld, Fphi, 1))) return rc;
+        if ((rc = forward_xy<T>(c, fldp, Fpi, 1))) return rc;
+    } else {
+        if ((rc = launch_x_r2c<T>(c, twx, fld, nullptr, Fphi, 0))) return rc;
+        if ((rc = launch_x_r2c<T>(c, twx, fldp, nullptr, Fpi, 0))) return rc;
+        if ((rc = launch_col<T>(c, twy, Fphi, 1, 0, 2))) return rc;
+    }
     if ((rc = launch_col<T>(c, twz, Fphi, 2, 0, 2))) return rc;
     // crossspec_3d(Fk = pi^, Fk2 = phi^) as called at evolve_spectral.f90:534-538
     if ((rc = launch_bin<T>(c, Fpi, Fphi, 2)) < 0) return rc;
@@ -1393,8 +1408,6 @@ static int gw_comp(int a, int b)
 template <typename T>
 static int gw_spectrum_t(Ctx &c, double *out)
 {
-    const cpx<T> *twx = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twx64 : (void *)c.twx32);
-    const cpx<T> *twy = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twy64 : (void *)c.twy32);
     const cpx<T> *twz = (const cpx<T> *)(sizeof(T) == 8 ? (void *)c.twz64 : (void *)c.twz32);
     int rc = ensure(c, &c.gwk, 6 * sizeof(cpx<T>) * c.nk, "hipMalloc gwk");
     if (rc) return rc;
@@ -1403,10 +1416,7 @@ static int gw_spectrum_t(Ctx &c, double *out)
     std::vector<double> raw(2 * (size_t)ns);
     for (int ch = 0; ch < 2; ++ch) {
         T *arr = (T *)(ch == 0 ? c.gwp : c.gwu);
-        for (int q = 0; q < 6; ++q)
-            if ((rc = launch_x_r2c<T>(c, twx, arr + (size_t)q * c.nvol, nullptr, K + (size_t)q * c.nk, 0, -1)))
-                return rc;
-        if ((rc = launch_col<T>(c, twy, K, 1, 0, 6))) return rc;
+        if ((rc = forward_xy<T>(c, arr, K, 6))) return rc;
         if ((rc = launch_col<T>(c, twz, K, 2, 0, 6))) return rc;
         if ((rc = launch_bin<T>(c, K, nullptr, 3)) < 0) return rc;
         LAT_HIP(&c, hipMemcpyAsync(raw.data(), c.spec_out, sizeof(double) * 2 * ns, hipMemcpyDeviceToHost, c.stream));

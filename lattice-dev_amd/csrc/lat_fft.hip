@@ -237,10 +237,25 @@ static int c2r_size(Ctx &c, const cpx<T> *tw, cpx<T> *Fk, int nf, int epi, T *ou
     return c2r_shape<T, N, 0>(c, tw, Fk, nf, epi, out, fld, fldp, md);
 }
 
-template <typename T>
-int launch_x_c2r(Ctx &c, const cpx<T> *tw, cpx<T> *Fk, int nf, int epi, T *out, const T *fld, T *fldp, int layout)
+ModelDev model_dev(const Ctx &c, int gwc0)
 {
     ModelDev md{c.cfg.model, c.nfld, c.cfg.model_params[0], c.cfg.model_params[1], c.gw_coup};
+    md.gc0 = gwc0;
+    md.gny = c.ny;
+    md.gnz = c.nz;
+    md.gr = 0.5 / c.dx;
+    return md;
+}
+
+template <typename T>
+int launch_x_c2r(Ctx &c, const cpx<T> *tw, cpx<T> *Fk, int nf, int epi, T *out, const T *fld, T *fldp, int layout,
+                 int gwc0)
+{
+    const ModelDev md = model_dev(c, gwc0);
+    if (epi == EPI_GWKICK && nf != 2) {
+        c.last_error = "tensor components come in pairs";
+        return -1;
+    }
     if (nf < 1 || nf > 2) {
         c.last_error = "nf must be 1 or 2";
         return -1;
@@ -267,8 +282,8 @@ template int launch_x_r2c<float>(Ctx &, const cpx<float> *, float *, const float
 template int launch_col<double>(Ctx &, const cpx<double> *, cpx<double> *, int, int, int, int);
 template int launch_col<float>(Ctx &, const cpx<float> *, cpx<float> *, int, int, int, int);
 template int launch_x_c2r<double>(Ctx &, const cpx<double> *, cpx<double> *, int, int, double *, const double *,
-                                  double *, int);
+                                  double *, int, int);
 template int launch_x_c2r<float>(Ctx &, const cpx<float> *, cpx<float> *, int, int, float *, const float *, float *,
-                                 int);
+                                 int, int);
 
 } // namespace lat

@@ -86,6 +86,9 @@ struct ModelDev {
     double p0, p1; // phi4: lambda; twofield: m2, g2
     double gwc;    // u_ij source coefficient 2 / M_p^2 (EPI_GWKICK only)
     double p2;     // twofield: m_chi^2 (0 unless lat_config.model_params[2] sets it)
+    // EPI_GWKICK: the source of components gc0, gc0 + 1 from the fields
+    int gc0 = 0, gny = 0, gnz = 0;
+    double gr = 0.0; // 1 / (2 dx)
 };
 
 // Per-stage HIP-event accounting (lat_profile / lat_profile_read).
@@ -208,22 +211,26 @@ int launch_col(Ctx &c, const cpx<T> *tw, cpx<T> *Fk, int axis, int mode, int n_a
 //   EPI_STORE:  write the real rows into out (one array per field)
 //   EPI_KICK:   kick pi with the device coefficients; reduce GE, PE, KE'
 //   EPI_REDUCE: reduce GE, PE, KE (no state change)
-//   EPI_GWKICK: pi_u += hA (lap + gw_coup S) for nf tensor components, with
-//               fld = S and fldp = pi_u of those components; no reductions
+//   EPI_GWKICK: pi_u += hA (lap + gw_coup S) for the two tensor components
+//               gwc0, gwc0 + 1, with fld = the fields, from which S is formed,
+//               and fldp = pi_u of those components; no reductions
 enum { EPI_STORE = 0, EPI_KICK = 1, EPI_REDUCE = 2, EPI_GWKICK = 3 };
 template <typename T>
 int launch_x_c2r(Ctx &c, const cpx<T> *tw, cpx<T> *Fk, int nf, int epi, T *out, const T *fld, T *fldp,
-                 int layout = 0);
+                 int layout = 0, int gwc0 = 0);
+ModelDev model_dev(const Ctx &c, int gwc0 = 0);
 
 // ---- plane sweeps of small cubic lattices (lat_plane.hip) ----
 // x R2C + y forward of nf arrays (drift and field as in launch_x_r2c, field0
 // the first one's index); y inverse + x C2R + epilogue (as launch_x_c2r).
+template <typename T>
 bool plane_fwd_ok(const Ctx &c);
+template <typename T>
 bool plane_inv_ok(const Ctx &c, int nf);
 template <typename T>
 int launch_plane_fwd(Ctx &c, const cpx<T> *tw, T *f, const T *pi, cpx<T> *Fk, int nf, int drift, int field0);
 template <typename T>
-int launch_plane_inv(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp);
+int launch_plane_inv(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp, int gwc0 = 0);
 
 // ---- separable spectral Laplacian (lat_sep.hip), mixed form ----
 // Kick of all fields with the three-sweep Laplacian (x: drift + D_xx; y:

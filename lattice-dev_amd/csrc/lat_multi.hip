@@ -616,7 +616,7 @@ int launch_fwd_multi(Ctx *const *cs, int ncls, int nf, int drift)
     if (rc) return rc;
     std::vector<Ctx *> sw, p256, p512;
     for (int k = 0; k < ncls; ++k)
-        (!plane_fwd_ok(*cs[k]) ? sw : plane_threads(cs[k]->nx) == 256 ? p256 : p512).push_back(cs[k]);
+        (!plane_fwd_ok<T>(*cs[k]) ? sw : plane_threads(cs[k]->nx) == 256 ? p256 : p512).push_back(cs[k]);
     if (!p256.empty() && (rc = plane_fwd_group<T, 256>(p256.data(), (int)p256.size(), nf, drift))) return rc;
     if (!p512.empty() && (rc = plane_fwd_group<T, 512>(p512.data(), (int)p512.size(), nf, drift))) return rc;
     if (sw.empty()) return 0;
@@ -635,7 +635,7 @@ int launch_inv_multi(Ctx *const *cs, int ncls, int nf, int epi, int *npart)
     std::vector<int> at, np(ncls);
     for (int k = 0; k < ncls; ++k) {
         npart[k] = cs[k]->nz;
-        if (!plane_inv_ok(*cs[k], nf)) {
+        if (!plane_inv_ok<T>(*cs[k], nf)) {
             sw.push_back(cs[k]);
             at.push_back(k);
         } else {

@@ -33,26 +33,26 @@ __global__ __launch_bounds__(plane_nt<N>()) void k_plane_inv(const cpx<T> *__res
                                                  twl);
 }
 
+template <typename T>
 bool plane_fwd_ok(const Ctx &c)
 {
     if (c.nx != c.ny) return false;
     switch (c.nx) {
 #define CASE(NN) \
-    case NN: return c.prec == LAT_F64 ? plane_fwd_fits<double, NN>() : plane_fwd_fits<float, NN>();
+    case NN: return plane_fwd_fits<T, NN>();
         LAT_FOR_PLANE_SIZES(CASE)
 #undef CASE
     }
     return false;
 }
 
+template <typename T>
 bool plane_inv_ok(const Ctx &c, int nf)
 {
     if (c.nx != c.ny || nf < 1 || nf > 2) return false;
     switch (c.nx) {
-#define CASE(NN)                                                                                           \
-    case NN:                                                                                               \
-        if (c.prec == LAT_F64) return nf == 1 ? plane_inv_fits<double, NN, 1>() : plane_inv_fits<double, NN, 2>(); \
-        return nf == 1 ? plane_inv_fits<float, NN, 1>() : plane_inv_fits<float, NN, 2>();
+#define CASE(NN) \
+    case NN: return nf == 1 ? plane_inv_fits<T, NN, 1>() : plane_inv_fits<T, NN, 2>();
         LAT_FOR_PLANE_SIZES(CASE)
 #undef CASE
     }
@@ -92,10 +92,10 @@ int launch_plane_fwd(Ctx &c, const cpx<T> *tw, T *f, const T *pi, cpx<T> *Fk, in
 }
 
 template <typename T, int N, int NF>
-static int inv_go(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int epi, const T *fld, T *fldp)
+static int inv_go(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int epi, const T *fld, T *fldp, int gwc0)
 {
     if constexpr (plane_inv_fits<T, N, NF>()) {
-        const ModelDev md{c.cfg.model, c.nfld, c.cfg.model_params[0], c.cfg.model_params[1], c.gw_coup};
+        const ModelDev md = model_dev(c, gwc0);
         const dim3 grid(c.nz, c.B), blk(plane_nt<N>());
         if (epi == EPI_KICK)
             hipLaunchKernelGGL((k_plane_inv<T, N, NF, EPI_KICK>), grid, blk, 0, c.stream, Fk, tw, c.P, c.nk, c.nvol,
@@ -103,8 +103,8 @@ static int inv_go(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int epi, const T *
         else if (epi == EPI_REDUCE)
             hipLaunchKernelGGL((k_plane_inv<T, N, NF, EPI_REDUCE>), grid, blk, 0, c.stream, Fk, tw, c.P, c.nk, c.nvol,
                                fld, fldp, c.dsc, md, c.partials, c.ms);
-        else
-            hipLaunchKernelGGL((k_plane_inv<T, N, NF, EPI_GWKICK>), grid, blk, 0, c.stream, Fk, tw, c.P, c.nk, c.nvol,
+        else if constexpr (NF == 2)
+            hipLaunchKernelGGL((k_plane_inv<T, N, 2, EPI_GWKICK>), grid, blk, 0, c.stream, Fk, tw, c.P, c.nk, c.nvol,
                                fld, fldp, c.dsc, md, c.partials, c.ms);
         LAT_HIP(&c, hipGetLastError());
         return c.nz;
@@ -115,11 +115,11 @@ static int inv_go(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int epi, const T *
 }
 
 template <typename T>
-int launch_plane_inv(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp)
+int launch_plane_inv(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int nf, int epi, const T *fld, T *fldp, int gwc0)
 {
     switch (c.nx) {
 #define CASE(NN) \
-    case NN: return nf == 1 ? inv_go<T, NN, 1>(c, tw, Fk, epi, fld, fldp) : inv_go<T, NN, 2>(c, tw, Fk, epi, fld, fldp);
+    case NN: return nf == 1 ? inv_go<T, NN, 1>(c, tw, Fk, epi, fld, fldp, gwc0) : inv_go<T, NN, 2>(c, tw, Fk, epi, fld, fldp, gwc0);
         LAT_FOR_PLANE_SIZES(CASE)
 #undef CASE
     }
@@ -127,11 +127,16 @@ int launch_plane_inv(Ctx &c, const cpx<T> *tw, const cpx<T> *Fk, int nf, int epi
     return -2;
 }
 
+template bool plane_fwd_ok<double>(const Ctx &);
+template bool plane_fwd_ok<float>(const Ctx &);
+template bool plane_inv_ok<double>(const Ctx &, int);
+template bool plane_inv_ok<float>(const Ctx &, int);
 template int launch_plane_fwd<double>(Ctx &, const cpx<double> *, double *, const double *, cpx<double> *, int, int,
                                       int);
 template int launch_plane_fwd<float>(Ctx &, const cpx<float> *, float *, const float *, cpx<float> *, int, int, int);
 template int launch_plane_inv<double>(Ctx &, const cpx<double> *, const cpx<double> *, int, int, const double *,
-                                      double *);
-template int launch_plane_inv<float>(Ctx &, const cpx<float> *, const cpx<float> *, int, int, const float *, float *);
+                                      double *, int);
+template int launch_plane_inv<float>(Ctx &, const cpx<float> *, const cpx<float> *, int, int, const float *, float *,
+                                     int);
 
 } // namespace lat

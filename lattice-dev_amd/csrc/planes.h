@@ -222,7 +222,7 @@ __device__ __forceinline__ void plane_inv_body(const cpx<T> *__restrict__ Fk, co
             for (int fi = 0; fi < NF; ++fi) {
                 if (!WHOLE && i0 + u * NT >= NV) continue;
                 const size_t site = fi * nvol + (size_t)bk.x * N * N + (size_t)(i0 + u * NT) * VW;
-                ph[u][fi] = *reinterpret_cast<const VT *>(fld + site);
+                if constexpr (EPI != EPI_GWKICK) ph[u][fi] = *reinterpret_cast<const VT *>(fld + site);
                 pv[u][fi] = *reinterpret_cast<const VT *>(fldp + site);
             }
 #pragma unroll
@@ -234,6 +234,7 @@ __device__ __forceinline__ void plane_inv_body(const cpx<T> *__restrict__ Fk, co
 #pragma unroll
             for (int fi = 0; fi < NF; ++fi)
                 lap[fi] = *reinterpret_cast<const VT *>(reinterpret_cast<const T *>(buf + (fi * N + line) * LS) + e0);
+            if constexpr (EPI == EPI_GWKICK) gw_source_vec<T>(fld, md, nvol, N, line, bk.x, e0, ph[u]);
             env.sites(NF, lap, ph[u], pv[u], acc);
             if constexpr (EPI == EPI_KICK || EPI == EPI_GWKICK) {
 #pragma unroll
