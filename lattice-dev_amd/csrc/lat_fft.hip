@@ -37,14 +37,14 @@ __global__ __launch_bounds__(TPB) void k_x_r2c(T *__restrict__ f, const T *__res
 
 template <typename T, int N, int TC, int MODE, int MR = 16, bool PF = true, int MINW = 1, int NT = TPB,
           bool TWL = false, bool FUSE = false, bool PP = false, int BLK = 0>
-__global__ __launch_bounds__(NT, MINW) void k_col(cpx<T> *__restrict__ Fk, const cpx<T> *__restrict__ tw, int nxh,
+__global__ __launch_bounds__(NT, MINW) void k_col(cpx<T> *__restrict__ Fk, const cpx<T> *__restrict__ tw, int P,
                                              int n_other, size_t s_axis, size_t s_other, size_t s_arr,
                                              int n_arr, int ny, double kfac, size_t ms_k, size_t s_blk)
 {
     __shared__ cpx<T> twl[tw_lds<T, N, TWL>()];
     __shared__ __attribute__((aligned(16))) cpx<T> buf[col_buf<T, N, TC>()];
     __shared__ __attribute__((aligned(16))) cpx<T> buf2[PP ? col_buf<T, N, TC>() : 1];
-    col_body<T, N, TC, MODE, MR, PF, MINW, NT, TWL, FUSE, PP, BLK>(Fk, tw, nxh, n_other, s_axis, s_other, s_arr,
+    col_body<T, N, TC, MODE, MR, PF, MINW, NT, TWL, FUSE, PP, BLK>(Fk, tw, P, n_other, s_axis, s_other, s_arr,
                                                                    n_arr, ny, kfac, ms_k, hw_blk(), buf, buf2, twl,
                                                                    s_blk);
 }
@@ -121,9 +121,9 @@ static void col_go(Ctx &c, const cpx<T> *tw, cpx<T> *Fk, int n_other, size_t s_a
 {
     using C = ColCfg<T, N, MODE == 2 ? 2 : 0>;
     constexpr int NT = col_nt<T, N, MODE, TC>();
-    const int g = grid_for(((c.nxh + TC - 1) / TC) * n_other * n_arrays, C::GRID);
+    const int g = grid_for(col_tiles<T, N>(c.P, n_other, TC) * n_arrays, C::GRID);
     hipLaunchKernelGGL((k_col<T, N, TC, MODE, C::MR, C::PF, 1, NT, true, C::FUSE, C::PP, BLK>), dim3(g, c.B),
-                       dim3(NT), 0, c.stream, Fk, tw, c.nxh, n_other, s_axis, s_other, c.nk, n_arrays, c.ny, kfac,
+                       dim3(NT), 0, c.stream, Fk, tw, c.P, n_other, s_axis, s_other, c.nk, n_arrays, c.ny, kfac,
                        c.ms.k, s_blk);
 }
 

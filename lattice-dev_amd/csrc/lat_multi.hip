@@ -153,7 +153,7 @@ struct ColCls {
     const cpx<T> *tw;
     size_t s_axis, s_other, s_arr, ms_k;
     double kfac;
-    int nxh, n_other, n_arr, ny, sel;
+    int P, n_other, n_arr, ny, sel;
 };
 template <typename T>
 struct ColArgs {
@@ -173,7 +173,7 @@ __device__ __forceinline__ void col_case(const ColCls<T> &c, const Blk &bk, cpx<
     constexpr int TC = col_TC<T, N, MODE, V>();
     constexpr int B = col_buf<T, N, TC>();
     col_body<T, N, TC, MODE, C::MR, C::PF, 1, COL_MULTI_NT, true, C::FUSE, C::PP>(
-        c.Fk, c.tw, c.nxh, c.n_other, c.s_axis, c.s_other, c.s_arr, c.n_arr, c.ny, c.kfac, c.ms_k, bk, lds, lds + B,
+        c.Fk, c.tw, c.P, c.n_other, c.s_axis, c.s_other, c.s_arr, c.n_arr, c.ny, c.kfac, c.ms_k, bk, lds, lds + B,
         lds + (C::PP ? 2 * B : B));
 }
 
@@ -340,7 +340,7 @@ static Geo col_geo(const Ctx &c, int n_other, int n_arr)
 {
     using C = ColCfg<T, N, MODE == 2 ? 2 : 0>;
     constexpr int TC = col_TC<T, N, MODE, V>();
-    return {grid_for(((c.nxh + TC - 1) / TC) * n_other * n_arr, C::GRID),
+    return {grid_for(col_tiles<T, N>(c.P, n_other, TC) * n_arr, C::GRID),
             sizeof(cpx<T>) * col_lds<T, N, TC, C::PP, true>()};
 }
 template <typename T, int N, int V>
@@ -461,7 +461,7 @@ static int col_multi_mode(Ctx *const *cs, int ncls, int axis, int n_arrays)
                            c.nk,
                            c.ms.k,
                            c.dk * c.dk / (double)c.nvol,
-                           c.nxh,
+                           c.P,
                            n_other,
                            n_arrays,
                            c.ny,

@@ -386,9 +386,27 @@ __device__ __forceinline__ void x_r2c_body(T *__restrict__ f, const T *__restric
 //      (o % KBLK) s_other (s_other = P), lines along ky with s_axis = KBLK P;
 //   2: z pass on the blocked order: kz = n at (n / KBLK) s_blk + (n % KBLK)
 //      s_axis (s_axis = P), tiles along ky with s_other = KBLK P.
+// Tiles.  A half-complex row is nx/2 + 1 columns and padded to P (a multiple of
+// 8), so tiles cut row by row leave a tile of one column at the end of every row:
+// 1 of 9 at nx = 256, 1 of 3 at 128 (32 columns), 1 of 2 at 64.  The tiles therefore
+// run on over the ends of the rows (flat_tiles: an array is one run of n_other P
+// columns), and the padding is transformed along: whole 64-byte pieces are
+// written, never one element of one.  Per kick, three lattices in turn: 256^3 FP64
+// 889 -> 843 us, 192^3 mixed 181 -> 175, 128^3 mixed 37.9 -> 37.0, 256^3 mixed 415 -> 411,
+// 512^3 FP64 6.87 -> 6.33 ms (one).  In longer columns a tile over two planes costs what
+// the short tile did, and tiles stay within their rows, with the padding: 1024^3
+// mixed 27.1 -> 26.5 ms (27.2 across rows), 512^3 mixed 3.40 -> 3.33 (3.43).
+template <typename T, int N>
+constexpr bool flat_tiles() { return N <= 256 || (N == 512 && sizeof(T) == 8); }
+// tiles of TC columns per array of n_other rows of pitch P
+template <typename T, int N>
+constexpr int col_tiles(int P, int n_other, int TC)
+{
+    return flat_tiles<T, N>() ? (P * n_other + TC - 1) / TC : (P + TC - 1) / TC * n_other;
+}
 template <typename T, int N, int TC, int MODE, int MR = 16, bool PF = true, int MINW = 1, int NT = TPB,
           bool TWL = false, bool FUSE = false, bool PP = false, int BLK = 0>
-__device__ __forceinline__ void col_body(cpx<T> *__restrict__ Fk, const cpx<T> *__restrict__ tw, int nxh, int n_other,
+__device__ __forceinline__ void col_body(cpx<T> *__restrict__ Fk, const cpx<T> *__restrict__ tw, int P, int n_other,
                                          size_t s_axis, size_t s_other, size_t s_arr, int n_arr, int ny, double kfac,
                                          size_t ms_k, const Blk bk, cpx<T> *__restrict__ buf,
                                          cpx<T> *__restrict__ buf2, cpx<T> *__restrict__ twl, size_t s_blk = 0)
@@ -415,37 +433,51 @@ __device__ __forceinline__ void col_body(cpx<T> *__restrict__ Fk, const cpx<T> *
     constexpr int NR0 = N / R0;
     constexpr int TOT0 = TC * NR0;
     constexpr int B0 = cdiv(TOT0, NT);
-    const int nct = (nxh + TC - 1) / TC;
+    constexpr bool FLAT = flat_tiles<T, N>();
+    // columns of a run of tiles (FLAT: an array, else a row) and tiles of it
+    const int ncol = FLAT ? n_other * P : P, nct = (ncol + TC - 1) / TC;
     int t0, t1, ts;
-    tile_range(nct * n_other * n_arr, bk, t0, t1, ts);
-    cpx<T> v[B0][R0];
-    auto tile_base = [&](int t, int &ncol, int &ct, int &o) -> cpx<T> * {
-        ct = t % nct;
-        const int rest = t / nct;
-        o = rest % n_other;
-        const int arr = rest / n_other;
-        ncol = min(TC, nxh - ct * TC);
-        return Fk + (size_t)arr * s_arr + tile_off(o) + (size_t)ct * TC;
+    tile_range(FLAT ? nct * n_arr : nct * n_other * n_arr, bk, t0, t1, ts);
+    // column `line` of tile t: element offset, |k|^2 of its kx and ky (MODE 2)
+    struct Col {
+        size_t off;
+        int k2;
+        bool ok;
     };
+    auto col_at = [&](int t, int line) -> Col {
+        const unsigned c = (unsigned)((t % nct) * TC + line);
+        int o, kx, arr = t / nct;
+        if constexpr (FLAT) {
+            o = (int)(c / (unsigned)P);
+            kx = (int)(c - (unsigned)o * (unsigned)P);
+        } else {
+            o = arr % n_other;
+            arr /= n_other;
+            kx = (int)c;
+        }
+        const int ky = MODE == 2 ? wmag(o, ny) : 0;
+        return {(size_t)arr * s_arr + tile_off(o) + kx, kx * kx + ky * ky, c < (unsigned)ncol};
+    };
+    constexpr bool ONE = NT % TC == 0; // a thread's butterflies belong to one column
+    cpx<T> v[B0][R0];
     auto load = [&](int t) {
-        int ncol, ct, o;
-        const cpx<T> *base = tile_base(t, ncol, ct, o);
+        Col col{};
+        if constexpr (ONE) col = col_at(t, threadIdx.x % TC);
 #pragma unroll
         for (int b = 0; b < B0; ++b) {
             const int g = threadIdx.x + b * NT;
             const int line = g % TC, j = g / TC;
+            if constexpr (!ONE) col = col_at(t, line);
 #pragma unroll
             for (int q = 0; q < R0; ++q) {
                 cpx<T> a = {0, 0};
-                if ((TOT0 % NT == 0 || g < TOT0) && line < ncol) a = base[line_off(j + q * NR0) + line];
+                if ((TOT0 % NT == 0 || g < TOT0) && col.ok) a = Fk[col.off + line_off(j + q * NR0)];
                 v[b][q] = a;
             }
         }
     };
     if (PF && t0 < t1) load(t0);
     for (int t = t0; t < t1; t += ts) {
-        int ncol, ct, o;
-        cpx<T> *base = tile_base(t, ncol, ct, o);
         if (!PF) load(t);
 #pragma unroll
         for (int b = 0; b < B0; ++b) {
@@ -459,58 +491,43 @@ __device__ __forceinline__ void col_body(cpx<T> *__restrict__ Fk, const cpx<T> *
         }
         if (PF && t + ts < t1) load(t + ts);
         lds_sync();
+        Col cur{};
+        if constexpr (ONE) cur = col_at(t, threadIdx.x % TC);
+        auto col_of = [&](int line) -> Col {
+            if constexpr (ONE) return cur;
+            else return col_at(t, line);
+        };
         auto store = [&](int line, int pos, cpx<T> a) {
-            if (line < ncol) base[line_off(pos) + line] = a;
+            const Col c = col_of(line);
+            if (c.ok) Fk[c.off + line_off(pos)] = a;
+        };
+        // -|k|^2 kfac; |k|^2 in lattice units is an integer below 2^24
+        // (N <= 1024): exact in FP32, one rounding in the product
+        const float kf = float(kfac);
+        auto mul = [&](int line, int n) -> T {
+            const int kk = wmag(n, N);
+            const int k2 = col_of(line).k2 + kk * kk;
+            if constexpr (sizeof(T) == 4) return -float(k2) * kf;
+            else return T(-double(k2) * kfac);
         };
         if constexpr (MODE == 2 && FUSE && PP && NP >= 2) {
             // pass 0 left the tile in buf; forward passes 1 .. NP-2, fused,
             // inverse passes 1 .. NP-2 alternate buffers; the data ends in buf2
             lds_fft_range_pp<T, N, -1, TC, NT, 1, NP - 1, MR, false, 0>(buf, buf2, twp);
             constexpr int FB = (NP - 2) & 1; // buffer holding the forward result
-            const int jj = wmag(o, ny);
-            const float kf = float(kfac);
-            auto mul = [&](int c, int n) -> T {
-                const int ii = ct * TC + c;
-                const int kk = wmag(n, N);
-                if constexpr (sizeof(T) == 4) {
-                    return -float(ii * ii + jj * jj + kk * kk) * kf;
-                } else {
-                    const double rad2 = double(ii * ii) + double(jj * jj) + double(kk * kk);
-                    return T(-rad2 * kfac);
-                }
-            };
             fused_last_first_pp<T, N, TC, NT, MR>(FB ? buf2 : buf, FB ? buf : buf2, twp, mul);
             lds_fft_range_pp<T, N, +1, TC, NT, 1, NP - 1, MR, true, FB ^ 1>(buf, buf2, twp);
             static_assert(((FB ^ 1) ^ ((NP - 2) & 1)) == 1, "inverse result in buf2");
             stockham_pass_out<T, N, NP - 1, +1, TC, NT, true, 1, MR, true>(buf2, 1, TC, twp, store);
         } else if constexpr (MODE == 2 && FUSE && NP >= 2) {
             lds_fft_range<T, N, -1, TC, NT, true, 1, 1, NP - 1, MR>(buf, 1, TC, twp);
-            const int jj = wmag(o, ny);
-            const float kf = float(kfac);
-            auto mul = [&](int c, int n) -> T {
-                const int ii = ct * TC + c;
-                const int kk = wmag(n, N);
-                if constexpr (sizeof(T) == 4) {
-                    // |k|^2 in lattice units is an integer below 2^24 (N <= 1024):
-                    // exact in FP32, one rounding in the product
-                    return -float(ii * ii + jj * jj + kk * kk) * kf;
-                } else {
-                    const double rad2 = double(ii * ii) + double(jj * jj) + double(kk * kk);
-                    return T(-rad2 * kfac);
-                }
-            };
             fused_last_first<T, N, TC, NT, MR>(buf, twp, mul);
             lds_fft_range<T, N, +1, TC, NT, true, 1, 1, NP - 1, MR, true>(buf, 1, TC, twp);
             stockham_pass_out<T, N, NP - 1, +1, TC, NT, true, 1, MR, true>(buf, 1, TC, twp, store);
         } else if constexpr (MODE == 2) {
             lds_fft_range<T, N, -1, TC, NT, true, 1, 1, NP, MR>(buf, 1, TC, twp);
-            const int jj = wmag(o, ny);
             for (int idx = threadIdx.x; idx < TC * N; idx += NT) {
-                const int c = idx % TC, n = idx / TC;
-                const int ii = ct * TC + c;
-                const int kk = wmag(n, N);
-                const double rad2 = double(ii * ii) + double(jj * jj) + double(kk * kk);
-                const T m = T(-rad2 * kfac);
+                const T m = mul(idx % TC, idx / TC);
                 cpx<T> a = buf[idx];
                 buf[idx] = {a.x * m, a.y * m};
             }
