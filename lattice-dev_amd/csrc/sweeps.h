@@ -257,6 +257,34 @@ struct EpiEnv {
         twp = twl_;                                                               \
     }
 
+// The same copy in two halves: issue() puts the table's loads in flight, put()
+// stores them to LDS ahead of a barrier that the caller has anyway.
+template <typename T, int NTW, int NTH, bool TWL>
+struct TwFill {
+    static constexpr int C = TWL ? (NTW + NTH - 1) / NTH : 1;
+    cpx<T> r[C];
+    __device__ __forceinline__ void issue(const cpx<T> *__restrict__ tw)
+    {
+        if constexpr (TWL) {
+#pragma unroll
+            for (int i = 0; i < C; ++i) {
+                const int k = threadIdx.x + i * NTH;
+                if (NTW % NTH == 0 || k < NTW) r[i] = tw[k];
+            }
+        }
+    }
+    __device__ __forceinline__ void put(cpx<T> *__restrict__ twl) const
+    {
+        if constexpr (TWL) {
+#pragma unroll
+            for (int i = 0; i < C; ++i) {
+                const int k = threadIdx.x + i * NTH;
+                if (NTW % NTH == 0 || k < NTW) twl[k] = r[i];
+            }
+        }
+    }
+};
+
 // LDS of each body in complex elements: the transform buffer(s) and the
 // twiddle table (when TWL), passed to the bodies as separate restrict
 // pointers so that buffer stores and table loads are known not to alias.
@@ -283,7 +311,22 @@ __device__ __forceinline__ void x_r2c_body(T *__restrict__ f, const T *__restric
 {
     constexpr int M = N / 2;
     constexpr int LS = M + 1;
-    LAT_TWIDDLES_TO_LDS(N, TPB, twl)
+    // AHEAD: a thread's vectors of phi and pi all in flight before the first is used,
+    // the twiddle table's loads ahead of them, so that a workgroup starts with one
+    // memory latency instead of one for the table and one per vector.  FP32, per
+    // kick: 1024^3 27.0 -> 26.3 ms (one lattice), 25.5 -> 25.1 (three in turn);
+    // 256^3 398 -> 385 us, 414 -> 411.  FP64 has twice the vectors per thread in
+    // flight anyway and loses 1 % (192^3 334 -> 339 us, 256x192x128 293 -> 297).
+    constexpr bool AHEAD = sizeof(T) == 4;
+    TwFill<T, N, TPB, TWL> twf;
+    if constexpr (AHEAD) {
+        twf.issue(tw);
+    } else {
+        twf.issue(tw);
+        twf.put(twl);
+        lds_sync();
+    }
+    const cpx<T> *twp = TWL ? twl : tw;
     assume_blk(bk);
     f += bk.y * ms.f;
     if (pi) pi += bk.y * ms.f;
@@ -301,31 +344,61 @@ __device__ __forceinline__ void x_r2c_body(T *__restrict__ f, const T *__restric
     tile_range((rows + L - 1) / L, bk, t0, t1, ts);
     constexpr int VW = 16 / sizeof(T); // reals per 16-byte lane access
     using VT = Vec16<T>;
+    constexpr int NV = L * N / VW, U = (NV + TPB - 1) / TPB; // vectors of a tile, of a thread
+    auto drift = [&](VT &v, const VT &p) {
+#pragma unroll
+        for (int e = 0; e < VW; ++e) {
+            T x = v.e[e] + dc0 * p.e[e];
+            if (nd > 1) x = x + dc1 * p.e[e];
+            if constexpr (sizeof(T) == 4) x = x - nu;
+            v.e[e] = x;
+        }
+    };
     for (int t = t0; t < t1; t += ts) {
         const int r0 = t * L;
-        for (int idx = threadIdx.x; idx < L * N / VW; idx += TPB) {
-            const int line = idx / (N / VW), i0 = (idx - line * (N / VW)) * VW;
-            const int row = r0 + line;
-            VT v{};
-            if (row < rows) {
-                VT *src = reinterpret_cast<VT *>(f + (size_t)row * N + i0);
-                v = *src;
-                if constexpr (DRIFT) {
-                    if (nd > 0) {
-                        const VT p = *reinterpret_cast<const VT *>(pi + (size_t)row * N + i0);
+        if constexpr (AHEAD) {
+            VT v[U], p[U];
 #pragma unroll
-                        for (int e = 0; e < VW; ++e) {
-                            T x = v.e[e] + dc0 * p.e[e];
-                            if (nd > 1) x = x + dc1 * p.e[e];
-                            if constexpr (sizeof(T) == 4) x = x - nu;
-                            v.e[e] = x;
-                        }
-                        *src = v;
-                    }
+            for (int u = 0; u < U; ++u) {
+                const int idx = threadIdx.x + u * TPB;
+                v[u] = p[u] = VT{};
+                if ((NV % TPB == 0 || idx < NV) && r0 + idx / (N / VW) < rows) {
+                    v[u] = *reinterpret_cast<const VT *>(f + (size_t)r0 * N + (size_t)idx * VW);
+                    if constexpr (DRIFT) p[u] = *reinterpret_cast<const VT *>(pi + (size_t)r0 * N + (size_t)idx * VW);
                 }
             }
 #pragma unroll
-            for (int e = 0; e < VW; e += 2) buf[line * LS + (i0 + e) / 2] = cpx<T>{v.e[e], v.e[e + 1]};
+            for (int u = 0; u < U; ++u) {
+                const int idx = threadIdx.x + u * TPB;
+                if (NV % TPB != 0 && idx >= NV) continue;
+                const int line = idx / (N / VW), i0 = (idx - line * (N / VW)) * VW;
+                if constexpr (DRIFT) {
+                    if (nd > 0 && r0 + line < rows) {
+                        drift(v[u], p[u]);
+                        *reinterpret_cast<VT *>(f + (size_t)r0 * N + (size_t)idx * VW) = v[u];
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < VW; e += 2) buf[line * LS + (i0 + e) / 2] = cpx<T>{v[u].e[e], v[u].e[e + 1]};
+            }
+            twf.put(twl);
+        } else {
+            for (int idx = threadIdx.x; idx < NV; idx += TPB) {
+                const int line = idx / (N / VW), i0 = (idx - line * (N / VW)) * VW;
+                VT v{};
+                if (r0 + line < rows) {
+                    VT *src = reinterpret_cast<VT *>(f + (size_t)r0 * N + (size_t)idx * VW);
+                    v = *src;
+                    if constexpr (DRIFT) {
+                        if (nd > 0) {
+                            drift(v, *reinterpret_cast<const VT *>(pi + (size_t)r0 * N + (size_t)idx * VW));
+                            *src = v;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < VW; e += 2) buf[line * LS + (i0 + e) / 2] = cpx<T>{v.e[e], v.e[e + 1]};
+            }
         }
         lds_sync();
         lds_fft_range<T, M, -1, L, TPB, false, 2, 0, num_passes(M, MR), MR>(buf, LS, 1, twp);
