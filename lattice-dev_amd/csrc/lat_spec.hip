@@ -29,19 +29,28 @@
 
 namespace lat {
 
-// TT projection of a symmetric tensor at wavevector kv (signed integers):
-// sum_ab |(Lambda U)_ab|^2 with Lambda_ab,lm = P_al P_bm - P_ab P_lm / 2,
-// P = 1 - k k^T / k^2 (gw-projectors.f90:13-26 is a stub); 0 at k = 0.
-// U holds the components xx, xy, xz, yy, yz, zz.
-__device__ __forceinline__ double tt_norm2(const double kv[3], const double ur[6], const double ui[6])
+// Projector P = 1 - k k^T / k^2 at the wavevector kv (signed integers; zero at
+// k = 0), components xx, xy, xz, yy, yz, zz.
+__device__ __forceinline__ void tt_projector(const double kv[3], double P[6])
 {
     const double k2 = kv[0] * kv[0] + kv[1] * kv[1] + kv[2] * kv[2];
-    if (k2 == 0.0) return 0.0;
-    double P[3][3];
+    const bool z = k2 == 0.0;
+    const double d = z ? 1.0 : k2;
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+    for (int a = 0, c = 0; a < 3; ++a)
 #pragma unroll
-        for (int b = 0; b < 3; ++b) P[a][b] = (a == b ? 1.0 : 0.0) - kv[a] * kv[b] / k2;
+        for (int b = a; b < 3; ++b, ++c) P[c] = z ? 0.0 : (a == b ? 1.0 : 0.0) - kv[a] * kv[b] / d;
+}
+
+// TT projection of a symmetric tensor: sum_ab |(Lambda U)_ab|^2 with
+// Lambda_ab,lm = P_al P_bm - P_ab P_lm / 2 (gw-projectors.f90:13-26 is a stub).
+// U holds the components xx, xy, xz, yy, yz, zz; sy, sz: the signs of ky and kz
+// against those of the projector p.
+__device__ __forceinline__ double tt_norm2(const double p[6], double sy, double sz, const double ur[6],
+                                           const double ui[6])
+{
+    const double pxy = sy * p[1], pxz = sz * p[2], pyz = sy * sz * p[4];
+    const double P[3][3] = {{p[0], pxy, pxz}, {pxy, p[3], pyz}, {pxz, pyz, p[5]}};
     const int ix[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
     double mr[3][3], mi[3][3]; // M = P U
 #pragma unroll
@@ -244,21 +253,36 @@ __global__ __launch_bounds__(64) void k_bin(const cpx<T> *__restrict__ F1, const
         auto values = [&](int i, const cpx<T> (&a_)[4], const cpx<T> (&b_)[4], double (&val)[NV]) {
 #pragma unroll
             for (int ch = 0; ch < NV; ++ch) val[ch] = 0.0;
+            // tensor modes: the members' six components all in flight (absent
+            // members read member 0), and one projector for the four, whose
+            // wavevectors differ in the signs of ky and kz.  Taken member by
+            // member (a load latency and six divides each) the kernel took 182 us
+            // at 256^3 mixed, now 157; the GW spectra call 1589 -> 1425 us, FP64
+            // 3122 -> 2965, 128^3 mixed 273 -> 211, 64^3 FP64 158 -> 127.
+            cpx<T> w[MODE == 3 ? 4 : 1][6];
+            double proj[6];
+            if constexpr (MODE == 3) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    const int mm = m < c.nm ? m : 0;
+                    const size_t id = ((size_t)c.mk[mm] * ny + c.mj[mm]) * P + i;
+#pragma unroll
+                    for (int c6 = 0; c6 < 6; ++c6) w[m][c6] = F1[(size_t)c6 * nk + id];
+                }
+                const double kv[3] = {double(i), double(c.jj), double(c.kk)};
+                tt_projector(kv, proj);
+            }
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 if (m >= c.nm) break;
                 if constexpr (MODE == 3) {
-                    const size_t id = ((size_t)c.mk[m] * ny + c.mj[m]) * P + i;
-                    const double kv[3] = {double(i), double(c.mj[m] <= ny / 2 ? c.mj[m] : c.mj[m] - ny),
-                                          double(c.mk[m] <= nz / 2 ? c.mk[m] : c.mk[m] - nz)};
                     double ur[6], ui[6];
 #pragma unroll
                     for (int c6 = 0; c6 < 6; ++c6) {
-                        const cpx<T> w = F1[(size_t)c6 * nk + id];
-                        ur[c6] = double(w.x);
-                        ui[c6] = double(w.y);
+                        ur[c6] = double(w[m][c6].x);
+                        ui[c6] = double(w[m][c6].y);
                     }
-                    val[0] += tt_norm2(kv, ur, ui);
+                    val[0] += tt_norm2(proj, 2 * c.mj[m] > ny ? -1.0 : 1.0, 2 * c.mk[m] > nz ? -1.0 : 1.0, ur, ui);
                 } else if constexpr (MODE <= 2) {
                     const cpx<T> x = a_[m], y = b_[m];
                     if constexpr (MODE == 0) {
@@ -421,8 +445,19 @@ __global__ __launch_bounds__(256) void k_bin_reduce(const double *__restrict__ p
     const int g = blockIdx.y;
     if (q >= nq) return;
     const int b0 = g * group, b1 = min(nblk, b0 + group);
+    // a chain of up to 64 loads and adds per thread: sixteen loads in flight, added in
+    // order (one load at a time: 18-22 us a launch, now 5)
+    constexpr int U = 16;
     double s = 0.0;
-    for (int b = b0; b < b1; ++b) s += part[(size_t)b * nq + q];
+    int b = b0;
+    for (; b + U <= b1; b += U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = part[(size_t)(b + u) * nq + q];
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += v[u];
+    }
+    for (; b < b1; ++b) s += part[(size_t)b * nq + q];
     out[(size_t)g * nq + q] = s;
 }
 

@@ -231,3 +231,20 @@ def test_gw_mixed_form_tracks_f64_at_128(gpu):
     print("gw mixed 128: spectra (pi_u, u)", errs, "u, pi_u fields", fu, flush=True)
     assert max(errs) < 1e-4
     assert max(fu) < 1e-4
+
+
+@pytest.mark.parametrize("shape", [(8, 8, 8), (16, 48, 32), (64, 16, 48), (128, 8, 96)], ids=lambda s: "x".join(map(str, s)))
+def test_gw_spectrum_row_classes_match_oracle(gpu, shape):
+    """Row classes of one, two and four rows, and histograms of 25 to 425 blocks
+    (the sums' groups of 64 and batches of 16 with remainders)."""
+    print("case gw row classes", shape, flush=True)
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx + 3 * ny)
+    pu = rng.standard_normal((6, nz, ny, nx))
+    with gpu.Lattice(shape, nfld=2, length=7.0, gw=True) as lat:
+        lat.set_gw(0.5 * pu, pu)
+        S = lat.gw_spectrum()
+    Uk = np.stack([O.r2c_3d(pu[q]) for q in range(6)])
+    ref = O.gw_spectrum(O.tt_project(Uk, nx), nx)
+    assert np.allclose(S[0], ref, rtol=1e-11, atol=1e-13 * np.abs(ref).max())
+    assert np.allclose(S[1], 0.25 * ref, rtol=1e-11, atol=1e-13 * np.abs(ref).max())
