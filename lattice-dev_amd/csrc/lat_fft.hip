@@ -10,6 +10,7 @@
 //   4. y: inverse;
 //   5. x: C2R of every field's rows, then the kick of all fields at each site
 //      (V' needs all fields) with the GE/PE/KE reductions fused in.
+// Lattices with nx = ny <= 128 run 1 + 2 and 4 + 5 as one sweep each (lat_plane.hip).
 // Every 1-D transform is LDS-resident (fft_core.h).  The k-space array is
 // FFTW's half-complex layout with the row pitch padded to P >= nx/2+1.
 #include "sweeps.h"

@@ -156,7 +156,7 @@ struct Ctx {
     bool gw;
     double gw_coup;         // 2 / M_p^2
     void *gwu, *gwp;        // 6 * nvol of T
-    void *gwsrc;            // 2 * nvol of T: S_ij of the component pair being kicked
+    void *gwsrc;            // 2 * nvol of T: S_ij of a component pair (lat_gw_source, allocated there)
     void *gwk;              // 6 * nk of cpx<T>: transforms for the GW spectra
     // separable form of the spectral Laplacian (lat_sep.hip): lap holds the
     // running sum D_xx + D_yy of every field between the x and z sweeps

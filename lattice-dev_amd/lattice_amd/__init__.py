@@ -153,7 +153,7 @@ class Lattice:
         self.ns = num_bins(self.nx, self.ny, self.nz)
 
     def autotune(self):
-        """Pick the faster launch shape of each sweep (sizes up to 256)."""
+        """Pick the faster launch shape of each sweep (sizes up to 512)."""
         self._check(lib().lat_autotune(self._h), "lat_autotune")
         return self.tuning()
 
