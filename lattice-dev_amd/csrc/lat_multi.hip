@@ -19,11 +19,33 @@ namespace lat {
 
 #define LAT_FOR_MULTI_SIZES(X) X(16) X(32) X(48) X(64) X(96) X(128) X(192) X(256)
 
-// sizes that take the separate x and y sweeps: forward only above 128, inverse
-// at 128 too where two planes do not fit the LDS (FP64)
+// Sizes with separate x and y sweeps: what the plane sweeps do not take (192 and
+// 256; the inverse at 128 too where two planes do not fit the LDS, FP64).
+// multi_sweep is what these kernels compile; the launchers send them the
+// classes that plane_fwd_ok and plane_inv_ok, the same predicate, turn down.
 #define LAT_FOR_MULTI_LARGE(X) X(128) X(192) X(256)
 template <typename T, int N, bool INV>
 constexpr bool multi_sweep() { return INV ? !plane_inv_fits<T, N, 2>() : !plane_fwd_fits<T, N>(); }
+template <int N>
+constexpr bool multi_sweep_any()
+{
+    return multi_sweep<float, N, false>() || multi_sweep<float, N, true>() || multi_sweep<double, N, false>() ||
+           multi_sweep<double, N, true>();
+}
+constexpr bool multi_large(int n)
+{
+    switch (n) {
+#define CASE(NN) case NN:
+        LAT_FOR_MULTI_LARGE(CASE)
+#undef CASE
+        return true;
+    default:
+        return false;
+    }
+}
+#define CASE(NN) static_assert(!multi_sweep_any<NN>() || multi_large(NN), "a class without a sweep");
+LAT_FOR_MULTI_SIZES(CASE)
+#undef CASE
 
 bool multi_supported(int n)
 {

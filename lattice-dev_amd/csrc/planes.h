@@ -28,6 +28,17 @@ constexpr int plane_nt() { return N >= 48 ? 512 : 256; }
 constexpr int PLANE_MRX = 8, PLANE_MRY = 16;
 
 constexpr int PLANE_LDS = 160 * 1024;
+constexpr bool plane_size(int n)
+{
+    switch (n) {
+#define CASE(NN) case NN:
+        LAT_FOR_PLANE_SIZES(CASE)
+#undef CASE
+        return true;
+    default:
+        return false;
+    }
+}
 template <typename T, int N>
 constexpr int plane_fwd_buf() { return N * (N / 2 + 1); }
 template <typename T, int N, int NF>
@@ -37,10 +48,13 @@ template <typename T, int N>
 constexpr int plane_fwd_lds() { return (int)sizeof(cpx<T>) * (plane_fwd_buf<T, N>() + N); }
 template <typename T, int N, int NF>
 constexpr int plane_inv_lds() { return (int)sizeof(cpx<T>) * (plane_inv_buf<T, N, NF>() + N) + 1024; } // + reduction
+// Which sizes take the plane sweeps, for the host's choice (plane_fwd_ok,
+// plane_inv_ok) and for what the shared launches compile alike: the size has
+// plane kernels and its planes fit.  (The bytes alone would admit FP32 192, 147 KB.)
 template <typename T, int N>
-constexpr bool plane_fwd_fits() { return plane_fwd_lds<T, N>() <= PLANE_LDS; }
+constexpr bool plane_fwd_fits() { return plane_size(N) && plane_fwd_lds<T, N>() <= PLANE_LDS; }
 template <typename T, int N, int NF>
-constexpr bool plane_inv_fits() { return plane_inv_lds<T, N, NF>() <= PLANE_LDS; }
+constexpr bool plane_inv_fits() { return plane_size(N) && plane_inv_lds<T, N, NF>() <= PLANE_LDS; }
 
 // ---------------------------------------------------------------- x R2C + y forward
 // Plane bk.x of the lattice, member bk.y; f, pi, Fk: the field's arrays.

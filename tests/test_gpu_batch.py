@@ -189,6 +189,47 @@ def test_ensemble_single_launch_matches_per_class_launches(gpu, precision):
         assert ens.single_launch(True) is False
 
 
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+@pytest.mark.parametrize("sizes", [(64, 128, 192), (128, 192, 256)], ids=lambda s: "-".join(map(str, s)))
+@pytest.mark.parametrize("nfld", [1, 2])
+def test_single_launch_of_large_classes_matches_per_class_launches(gpu, nfld, sizes, precision):
+    """Shared launches of classes on both sides of the plane sweeps' limit (the
+    separate x and y sweeps carry 192, 256, and the FP64 two-field inverse at
+    128): bitwise the per-class launches, eagerly and through the graph."""
+    print("case ensemble single launch, large", nfld, sizes, precision, flush=True)
+    counts = (2, 1, 1)
+    classes = [(n, c, 10.0 * n / 256) for n, c in zip(sizes, counts)]
+    dts = [2e-4, 1e-4, 3e-4]
+    kw = dict(nfld=nfld, precision=gpu.F64 if precision == "f64" else gpu.MIXED,
+              model=gpu.MODEL_TWOFIELD if nfld == 2 else gpu.MODEL_PHI4,
+              members=[(1.0, 1e4 * (m + 1)) if nfld == 2 else (0.5 * (m + 1),) for m in range(sum(counts))])
+    shapes = [(1, 1, 1, 1), (0, 1, 0, 1), (1, 0, 1, 0)]
+    out = {}
+    for single, graph in ((False, False), (True, False), (True, True)):
+        with gpu.Ensemble(classes, **kw) as ens:
+            assert ens.single_launch(single) is single  # these classes allow both
+            for k, sh in enumerate(shapes):
+                ens.set_tuning(k, sh)
+            ens.use_graph(graph)
+            views = [ens.member(i) for i in range(ens.size)]
+            for i, v in enumerate(views):
+                for q in range(2 * nfld):
+                    v.sample_field(q // 2, q % 2, (PHI0, DPHI0, 0.0, 0.0)[q], (-0.25, 0.25)[q % 2], 1.0, 2e5, 60 + i, q)
+                v.set_scalars(1.0, 0.0)
+                v.calc_metric()
+            for nsteps in (1, 1):  # the second call replays the first's graph
+                ens.symp(4, dts, nsteps)
+            ens.synchronize()
+            out[(single, graph)] = [v.get_state() for v in views]
+            for v in views:
+                v.close()
+    ref = out[(False, False)]
+    for key in ((True, False), (True, True)):
+        for i in range(sum(counts)):
+            for a, b in zip(out[key][i], ref[i]):
+                assert np.array_equal(np.asarray(a), np.asarray(b)), (key, i)
+
+
 @pytest.mark.parametrize("n", [32, 64, 128, 192])
 @pytest.mark.parametrize("precision", ["f64", "mixed"])
 def test_tuned_launch_shapes_match_oracle(gpu, n, precision):
