@@ -7,6 +7,9 @@
  * message via lat_last_error).  An opaque lat_ctx owns all device memory,
  * FFT twiddle tables and one HIP stream.  Host pointers are borrowed for the
  * duration of a call only.  A context is not thread-safe; use one per thread.
+ * Views of one batch (lat_member) may have a thread each for their state,
+ * scalars and steps; spectra and host transforms run in scratch that the views
+ * of a batch share, so one thread at a time calls those.
  *
  * Layout at this boundary is the reference's: Fortran column-major, x
  * fastest.  A real field f(nx,ny,nz) is f[i + nx*(j + ny*k)].  A half-complex

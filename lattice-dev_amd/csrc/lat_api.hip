@@ -135,6 +135,7 @@ static int stage_copy(Ctx &c, bool to_host, char *dev, size_t dpitch, char *host
 {
     if (!width || !rows) return 0;
     HostStage &h = *c.stage;
+    const std::lock_guard<std::mutex> hold(h.ring_lock);
     if (!h.ring && width * rows < (size_t)256 << 10) {
         // a small lattice: not worth the ring's allocation (70 us)
         if (to_host)
@@ -239,6 +240,7 @@ static void spec_read(Ctx &c, std::vector<double> &raw)
 
 static int pull_scalars(Ctx &c)
 {
+    const std::lock_guard<std::mutex> hold(c.stage->scalars_lock);
     LAT_HIP(&c, hipMemcpyAsync(c.stage->small, c.dsc, sizeof(DevScalars), hipMemcpyDeviceToHost, c.stream));
     int rc = sync(c);
     if (!rc) memcpy(&c.host_sc, c.stage->small, sizeof(DevScalars));
@@ -247,6 +249,7 @@ static int pull_scalars(Ctx &c)
 
 static int push_scalars(Ctx &c)
 {
+    const std::lock_guard<std::mutex> hold(c.stage->scalars_lock);
     memcpy(c.stage->small, &c.host_sc, sizeof(DevScalars));
     LAT_HIP(&c, hipMemcpyAsync(c.dsc, c.stage->small, sizeof(DevScalars), hipMemcpyHostToDevice, c.stream));
     return sync(c);

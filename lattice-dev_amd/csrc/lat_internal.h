@@ -4,6 +4,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -106,14 +107,19 @@ struct Prof {
 // copies of 16.8 MB run at 17 GB/s to pageable memory and 36 GB/s from it;
 // between the device and pinned memory they run at 55 GB/s, and one CPU thread
 // drains the ring at about 30 GB/s, so large arrays take several.  @STAGE_FIGS@
+//
+// Views of a batch may be driven by a host thread each, as far as they do not
+// share device scratch (scalars, state, steps): the scalars' place and the
+// ring are therefore taken under a lock, from the first write to the last read.
 struct HostStage {
+    std::mutex scalars_lock, ring_lock;
     static constexpr size_t SMALL = 64 << 10, SLOT = 1 << 20;
     static constexpr size_t MODES = 1024, SPEC = 2048; // small: scalars, k = 0 modes, binned channels
     static constexpr int THREADS = 4, SLOTS = 2 * THREADS; // two slots per copying thread
     char *small = nullptr;
     char *ring = nullptr;
     hipEvent_t ev[SLOTS] = {};
-    bool used[SLOTS] = {}; // an H2D copy from the slot has been recorded
+    bool used[SLOTS] = {}; // a copy of the slot, either way, that nobody has waited for yet
 };
 
 struct Ctx {

@@ -2,6 +2,8 @@
 lattice size advanced by batched launches must reproduce, member by member,
 single-context runs with the same initial conditions and couplings, and the
 oracle."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -334,3 +336,41 @@ def test_member_views_free_their_scratch(gpu):
         free1 = torch.cuda.mem_get_info()[0]
     nk_bytes = 2 * 8 * (n // 2 + 8) * n * n  # one view's two complex FP32 arrays
     assert free0 - free1 < nk_bytes, (free0, free1, nk_bytes)
+
+
+def test_member_views_on_threads_keep_their_own_values(gpu):
+    """A host thread per member view: scalars and states that the threads set
+    and read back at the same time, through staging memory that the views of a
+    batch share (arrays of 64 KB and of 4 MB, without and with the copy ring)."""
+    print("case views on threads", flush=True)
+    for n, rounds in ((16, 200), (64, 12)):
+        with gpu.Lattice(n, nfld=2, length=10.0, members=[(1.0, 1e4)] * 4) as batch:
+            views = [batch.member(m) for m in range(4)]
+            rngs = [np.random.default_rng(m) for m in range(4)]
+            bad = []
+
+            def work(m):
+                try:
+                    v = views[m]
+                    for r in range(rounds):
+                        fld, fldp = rngs[m].standard_normal((2, 2, n, n, n))
+                        v.set_state(fld, fldp, 1.0 + m + r, -2.0 - m - r)
+                        for q in range(20):
+                            y, p = 10.0 * m + q + 0.5, -(3.0 * m + r)
+                            v.set_scalars(y, p)
+                            if v.scalars != (y, p):
+                                bad.append((n, m, r, q, "scalars"))
+                        gf, gp, gy, gpy = v.get_state()
+                        if not (np.array_equal(gf, fld) and np.array_equal(gp, fldp) and (gy, gpy) == (y, p)):
+                            bad.append((n, m, r, "state"))
+                except Exception as e:
+                    bad.append((n, m, repr(e)))
+
+            threads = [threading.Thread(target=work, args=(m,)) for m in range(4)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join()
+            for v in views:
+                v.close()
+        assert not bad, bad[:4]
