@@ -574,14 +574,18 @@ __device__ __forceinline__ void col_body(cpx<T> *__restrict__ Fk, const cpx<T> *
             const Col c = col_of(line);
             if (c.ok) Fk[c.off + line_off(pos)] = a;
         };
-        // -|k|^2 kfac; |k|^2 in lattice units is an integer below 2^24
-        // (N <= 1024): exact in FP32, one rounding in the product
+        // -|k|^2 kfac; |k|^2 in lattice units is an integer below 2^24 (N <= 1024),
+        // exact in FP32.  The fused passes, with a factor per register, round
+        // kfac and the product in FP32; the pass over LDS of the short lines
+        // (8 and 16) rounds the FP64 product once.
         const float kf = float(kfac);
-        auto mul = [&](int line, int n) -> T {
+        auto k2_at = [&](int line, int n) -> int {
             const int kk = wmag(n, N);
-            const int k2 = col_of(line).k2 + kk * kk;
-            if constexpr (sizeof(T) == 4) return -float(k2) * kf;
-            else return T(-double(k2) * kfac);
+            return col_of(line).k2 + kk * kk;
+        };
+        auto mul = [&](int line, int n) -> T {
+            if constexpr (sizeof(T) == 4) return -float(k2_at(line, n)) * kf;
+            else return T(-double(k2_at(line, n)) * kfac);
         };
         if constexpr (MODE == 2 && FUSE && PP && NP >= 2) {
             // pass 0 left the tile in buf; forward passes 1 .. NP-2, fused,
@@ -600,7 +604,7 @@ __device__ __forceinline__ void col_body(cpx<T> *__restrict__ Fk, const cpx<T> *
         } else if constexpr (MODE == 2) {
             lds_fft_range<T, N, -1, TC, NT, true, 1, 1, NP, MR>(buf, 1, TC, twp);
             for (int idx = threadIdx.x; idx < TC * N; idx += NT) {
-                const T m = mul(idx % TC, idx / TC);
+                const T m = T(-double(k2_at(idx % TC, idx / TC)) * kfac);
                 cpx<T> a = buf[idx];
                 buf[idx] = {a.x * m, a.y * m};
             }

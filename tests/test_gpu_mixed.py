@@ -208,3 +208,37 @@ def test_mixed_tracks_fp64_at_1024(gpu):
     err3 = spec_err(sm, sd, 1e-3)
     print("1024 mixed spectrum max rel err (floor 1e-3)", err3, flush=True)
     assert err3 < 1e-5
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 16), (64, 64, 8), (64, 48, 16), (48, 64, 8)], ids=lambda s: "x".join(map(str, s)))
+def test_short_line_multiplier_is_rounded_once(gpu, shape):
+    """z lines of 8 and 16 sites, mixed form: the factor -k^2 dk^2 / n^3 is formed
+    in FP64 and rounded once, so it has no error common to all modes.  Measured
+    as the least-squares factor of a kick against the FP64 Laplacian, at a box
+    side whose dk^2 / n^3 is half a step of FP32 off (1.05 and a half times
+    2^-23, relative 5.7e-8) against one where it is a power of two; the rest
+    (rounded twiddles) is the same in both.  Bound: a third of that error; what
+    remains is noise, 1e-7 / sqrt(sites) of the transforms and 2.4e-8 / sqrt(150)
+    of the single rounding over the values of k^2 that carry the sum: 2e-9."""
+    print("case short lines", shape, flush=True)
+    nx, ny, nz = shape
+    nv, h = nx * ny * nz, 2.0 ** -6
+    phi = np.float32(np.random.default_rng(nx + nz).standard_normal((nz, ny, nx))).astype(np.float64)
+    phi -= phi.mean()
+    kx = np.arange(nx // 2 + 1)
+    ky, kz = (np.minimum(np.arange(n), n - np.arange(n)) for n in (ny, nz))
+    k2 = kx[None, None, :] ** 2 + ky[None, :, None] ** 2 + kz[:, None, None] ** 2
+    lap1 = np.fft.irfftn(-k2 * np.fft.rfftn(np.float64(np.float32(phi))), s=phi.shape, axes=(0, 1, 2))
+    fac = []
+    for mant in (1.0 + (int(0.05 * 2**23) + 0.49) * 2.0**-23, 1.0):
+        dk = np.sqrt(mant * 2.0**-14 * nv)
+        with gpu.Lattice(shape, nfld=1, length=2.0 * np.pi / dk, precision=gpu.MIXED, model=gpu.MODEL_PHI4,
+                         model_params=(0.0,)) as lat:
+            lat.set_state(phi[None], np.zeros_like(phi)[None], 1.0, 0.0)
+            lat.Hamiltonian_Split(h, 3)
+            pi = lat.get_state()[1][0]
+        ref = h * dk * dk * lap1
+        fac.append(float((pi * ref).sum() / (ref * ref).sum()))
+    print("factors - 1:", fac[0] - 1.0, fac[1] - 1.0, flush=True)
+    assert abs(fac[1] - 1.0) < 1e-6
+    assert abs(fac[0] - fac[1]) < 1.9e-8
