@@ -2112,19 +2112,26 @@ static int autotune(Ctx &c, int reps)
 // allocations in one process, ran 3.07, 3.21, 3.49 and 3.55 ms per launch,
 // each allocation keeping its own figure on every later call.  The tuner
 // allocates further sets of these arrays (with the metric perturbations,
-// their momenta and source scratch where the context has them), times one
+// their momenta and source scratch, or the second state arrays of the
+// finite-difference sweeps, where the context has them), times one
 // force evaluation's sweeps on each (one pending drift of size zero, so that
-// the x R2C reads the momenta as it does in a step; kick coefficients zero),
+// the x R2C reads the momenta as it does in a step; kick coefficients zero;
+// with second state arrays the fused drift + kick sweep, there and back),
 // keeps the fastest set holding the state unchanged and frees the others.
 struct Placement {
     void *fld = nullptr, *fldp = nullptr, *Fk = nullptr;
+    void *fld2 = nullptr, *fldp2 = nullptr; // contexts with second state arrays
     void *gwu = nullptr, *gwp = nullptr, *gwsrc = nullptr; // contexts with the metric perturbations
 };
 
 template <typename T>
 static int place_time(Ctx &c, int reps, float *ms)
 {
+    // (after an odd number of fused sweeps the state is in both pairs of arrays:
+    // drift and kick are zero)
+    FdHome home(c);
     auto run = [&]() -> int {
+        c.fd_fuse = c.fld2 != nullptr;
         const int g = state_force<T>(c, true, EPI_KICK);
         return g < 0 ? g : 0;
     };
@@ -2149,27 +2156,30 @@ static int place_tune(Ctx &c, int cand, int reps)
     const size_t es = elem_size(c), B = (size_t)c.B;
     const size_t bf = es * B * c.ms.f, bk = c.Fk ? 2 * es * B * c.ms.k : 0;
     const size_t bg = c.gw ? es * 6 * c.nvol : 0, bs = c.gwsrc ? es * 2 * c.nvol : 0;
+    const size_t b2 = c.fld2 ? bf : 0;
     std::vector<Placement> pl(1);
-    pl[0] = {c.fld, c.fldp, c.Fk, c.gwu, c.gwp, c.gwsrc};
+    pl[0] = {c.fld, c.fldp, c.Fk, c.fld2, c.fldp2, c.gwu, c.gwp, c.gwsrc};
     // Set k puts a spacer of its own size between its field and momentum
-    // arrays (and between the metric perturbations and their momenta), so
-    // that even where consecutive allocations are consecutive in memory each
-    // set has the two at another distance (a spacer of 66 MB or 1026 MB made
-    // the 1024^3 mixed x R2C 3.20 ms per launch, none or 130 MB 3.49 ms, in
-    // each of several processes).
+    // arrays, first and second ones (and between the metric perturbations and
+    // their momenta), so that even where consecutive allocations are
+    // consecutive in memory each set has the two at another distance (a spacer
+    // of 66 MB or 1026 MB made the 1024^3 mixed x R2C 3.20 ms per launch, none
+    // or 130 MB 3.49 ms, in each of several processes).
     static const size_t spacer_mb[7] = {66, 1026, 34, 258, 18, 514, 2050};
     for (int k = 1; k < cand; ++k) {
         const size_t sp = spacer_mb[(k - 1) % 7] << 20;
         // a further set only while it leaves 8 GiB of device memory free
         size_t fr = 0, tot = 0;
-        if (hipMemGetInfo(&fr, &tot) != hipSuccess || fr < 2 * bf + bk + 2 * bg + bs + sp + (size_t(8) << 30)) {
+        if (hipMemGetInfo(&fr, &tot) != hipSuccess ||
+            fr < 2 * bf + bk + 2 * b2 + 2 * bg + bs + sp + (size_t(8) << 30)) {
             (void)hipGetLastError();
             break;
         }
         Placement q;
         void *spacer = nullptr, *spacer2 = nullptr;
-        bool ok = hipMalloc(&q.fld, bf) == hipSuccess && hipMalloc(&spacer, sp) == hipSuccess &&
-                  hipMalloc(&q.fldp, bf) == hipSuccess && (!bk || hipMalloc(&q.Fk, bk) == hipSuccess);
+        bool ok = hipMalloc(&q.fld, bf) == hipSuccess && (!b2 || hipMalloc(&q.fld2, b2) == hipSuccess) &&
+                  hipMalloc(&spacer, sp) == hipSuccess && hipMalloc(&q.fldp, bf) == hipSuccess &&
+                  (!b2 || hipMalloc(&q.fldp2, b2) == hipSuccess) && (!bk || hipMalloc(&q.Fk, bk) == hipSuccess);
         if (ok && bg)
             ok = hipMalloc(&q.gwu, bg) == hipSuccess && hipMalloc(&spacer2, sp) == hipSuccess &&
                  hipMalloc(&q.gwp, bg) == hipSuccess && (!bs || hipMalloc(&q.gwsrc, bs) == hipSuccess);
@@ -2177,7 +2187,7 @@ static int place_tune(Ctx &c, int cand, int reps)
             if (p) (void)hipFree(p);
         if (!ok) {
             (void)hipGetLastError(); // out of memory: tune over the sets allocated so far
-            for (void *p : {q.fld, q.fldp, q.Fk, q.gwu, q.gwp, q.gwsrc})
+            for (void *p : {q.fld, q.fldp, q.Fk, q.fld2, q.fldp2, q.gwu, q.gwp, q.gwsrc})
                 if (p) (void)hipFree(p);
             break;
         }
@@ -2194,6 +2204,8 @@ static int place_tune(Ctx &c, int cand, int reps)
         c.fld = q.fld;
         c.fldp = q.fldp;
         c.Fk = q.Fk;
+        c.fld2 = q.fld2;
+        c.fldp2 = q.fldp2;
         if (Fk64_0 && Fk64_0 == pl[0].Fk) c.Fk64 = q.Fk; // the FP64 context's Fk64 is its Fk
         c.gwu = q.gwu;
         c.gwp = q.gwp;
@@ -2262,7 +2274,8 @@ static int place_tune(Ctx &c, int cand, int reps)
         (void)hipStreamSynchronize(c.stream);
         for (int k = 0; k < K; ++k) {
             if (k == w) continue;
-            for (void *p : {pl[k].fld, pl[k].fldp, pl[k].Fk, pl[k].gwu, pl[k].gwp, pl[k].gwsrc})
+            for (void *p : {pl[k].fld, pl[k].fldp, pl[k].Fk, pl[k].fld2, pl[k].fldp2, pl[k].gwu, pl[k].gwp,
+                            pl[k].gwsrc})
                 if (p) (void)hipFree(p);
         }
         c.place_ms.resize(K);
@@ -2680,8 +2693,10 @@ int lat_ensemble_create(const lat_config *base, int nclass, const int *n, const 
         c.stream = e->stream;
         c.owns_stream = false;
         // launch shapes, then the fastest of eight placements of the class's
-        // arrays (before any graph or member view holds their addresses)
-        if (autotune(c, 3) || place_tune(c, 8, 3)) {
+        // arrays (before any graph or member view holds their addresses); four
+        // with second state arrays, which take as long to allocate as eight
+        // without (16 x 64^3 + 8 x 128^3 mixed 7-point, eight of them: 22 -> 30 ms)
+        if (autotune(c, 3) || place_tune(c, c.fld2 ? 4 : 8, 3)) {
             e->last_error = c.last_error;
             lat_destroy(h);
             lat_ensemble_destroy(e);
