@@ -108,10 +108,12 @@ int  lat_copy_bandwidth(lat_ctx *ctx, size_t bytes, int reps, double *gbps);
  * x C2R rows per workgroup, y and z columns per tile) on the context's arrays
  * and keeps the faster; fields are not modified.  Ensembles tune every size
  * class at creation.  lat_tuning reports the shapes in use (0 or 1 each; a
- * context starts with those measured faster for its size):
+ * context starts with those measured faster for its size, and an axis longer
+ * than 512 has shape 0 only, whatever is set):
  * out[4] = {x R2C, y, z, x C2R}.  Lattices with nx = ny up to 128 take the x and
- * y passes of a force evaluation plane by plane: there the x and y shapes
- * serve the output transforms only. */
+ * y passes of a force evaluation and of the forward transforms plane by
+ * plane: there the x and y shapes serve the inverse host transforms only (and
+ * the inverse sweeps of two FP64 fields at 128). */
 /* Form of the spectral Laplacian in the field kicks (no reference
  * counterpart; the reference has the 3-D form only): 0 = five HBM sweeps
  * (x R2C, y, z * -k^2, y, x C2R + kick), 1 = the same operator as the sum of

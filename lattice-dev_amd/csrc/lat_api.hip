@@ -836,8 +836,9 @@ static Ctx::Tune default_tune(const Ctx &c)
 {
     const bool f64 = c.prec == LAT_F64;
     Ctx::Tune t;
-    t.r2c = t.coly = 1;
-    t.c2r = !(f64 && c.nx == 512);
+    t.r2c = c.nx <= SHAPES_MAX;
+    t.coly = c.ny <= SHAPES_MAX;
+    t.c2r = c.nx <= SHAPES_MAX && !(f64 && c.nx == 512);
     t.colz = c.nz == 128 || c.nz == 256 || (f64 && (c.nz == 96 || c.nz == 192));
     return t;
 }
@@ -2379,10 +2380,11 @@ int lat_tuning(lat_ctx *h, int *out)
 {
     CTX_OR_FAIL(h);
     if (!out) return -1;
-    out[0] = c.tune.r2c;
-    out[1] = c.tune.coly;
-    out[2] = c.tune.colz;
-    out[3] = c.tune.c2r;
+    // an axis without a second shape runs its one shape whatever was set
+    out[0] = c.nx <= SHAPES_MAX && c.tune.r2c;
+    out[1] = c.ny <= SHAPES_MAX && c.tune.coly;
+    out[2] = c.nz <= SHAPES_MAX && c.tune.colz;
+    out[3] = c.nx <= SHAPES_MAX && c.tune.c2r;
     return 0;
 }
 

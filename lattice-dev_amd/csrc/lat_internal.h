@@ -18,6 +18,7 @@ constexpr int TPB = 256;       // threads per workgroup for all lattice kernels
 constexpr int MAX_GRID = 8192; // most reduction partials (blocks) per member of a launch
 constexpr int GRID_CAP = 4096; // default cap of grid-stride launches
 constexpr int NRED = 8;        // reduction channels per partial
+constexpr int SHAPES_MAX = 512; // longest axis whose sweeps have a second launch shape
 
 // 16-byte vector of reals (4 floats or 2 doubles) for vector loads/stores.
 template <typename T>

@@ -848,7 +848,7 @@ struct ColCfg {
 // 0.418 -> 0.357 ms and fused z pass 0.546 -> 0.402 ms (32 columns, 256
 // threads), 192^3 y pass 0.462 -> 0.398 ms (16 columns, 192 threads).
 template <int N>
-constexpr bool tunable() { return N <= 512; }
+constexpr bool tunable() { return N <= SHAPES_MAX; }
 constexpr int pow2_floor(int v) { return v >= 2 ? 2 * pow2_floor(v / 2) : 1; }
 template <typename T, int N>
 constexpr int col_tc(int mode, int v)

@@ -268,6 +268,26 @@ def test_tuned_launch_shapes_match_oracle(gpu, n, precision):
         assert set(t.values()) <= {0, 1}
 
 
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("size", [512, 1024])
+def test_tuning_reports_the_shapes_in_use(gpu, size, axis):
+    """A 1024 axis has one launch shape per sweep: 0 is reported for the sweeps
+    along it, at creation, after asking for shape 1 and after autotuning; a 512
+    axis has two."""
+    print("case tuning report", size, axis, flush=True)
+    shape = [8, 8, 8]
+    shape[axis] = size
+    knobs = ((0, 3), (1,), (2,))[axis]  # x R2C and x C2R, y, z
+    with gpu.Lattice(tuple(shape), nfld=1, length=1.0, model=gpu.MODEL_PHI4, model_params=(1.0,)) as lat:
+        start = list(lat.tuning().values())
+        lat.set_tuning(1, 1, 1, 1)
+        asked = list(lat.tuning().values())
+        tuned = list(lat.autotune().values())
+    assert asked == [0 if size == 1024 and k in knobs else 1 for k in range(4)]
+    if size == 1024:
+        assert not any(start[k] or tuned[k] for k in knobs)
+
+
 def test_ensemble_96_members_match_oracle(gpu):
     """The 96-realisation ensemble (32 x 64^3 + 48 x 128^3 + 16 x 192^3, fixed
     L = 10, g^2/m^2 log-uniform in [1e4, 1e6]), autotuned launch mode and
