@@ -131,6 +131,46 @@ def test_gw_evolution_matches_oracle(gpu, case, order):
     assert rel(gpu_, sim.gwp) < 1e-11
 
 
+@pytest.mark.parametrize("shape", [(16, 48, 32), (48, 16, 8), (8, 32, 64), (192, 192, 8), (32, 32, 8), (64, 64, 16),
+                                   (128, 128, 8)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("nfld", [1, 2])
+def test_gw_evolution_of_boxes_matches_oracle(gpu, shape, nfld):
+    """The tensor kick's source in both of its epilogues: rows of separate x
+    sweeps (nx != ny, 192, and FP64 at 128) and planes (nx = ny up to 128, here
+    with nz of its own).  FP64 as the cubic cases; the mixed form to the level of
+    the FP32 fields against FP64."""
+    print("case gw boxes", shape, nfld, flush=True)
+    c = CASES["cosmic_twofield_spectral" if nfld == 2 else "conformal_phi4_spectral"]
+    nx, ny, nz = shape
+    L, dt, nsteps = 10.0 * nx / 16, 0.01, 4
+    rng = np.random.default_rng(nx + 3 * ny + 5 * nz)
+    fld = 0.05 * rng.standard_normal((nfld, nz, ny, nx))
+    fldp = 0.05 * rng.standard_normal((nfld, nz, ny, nx))
+    fld[0] += 1.0
+    u, pu = 1e-3 * rng.standard_normal((2, 6, nz, ny, nx))
+    got = {}
+    for prec in (gpu.F64, gpu.MIXED):
+        lat, sim = make_pair(gpu, c, shape, L, gw_mpl=0.5, precision=prec)
+        with lat:
+            lat.set_state(fld, fldp, 1.0, 0.0)
+            lat.set_gw(u, pu)
+            lat.calc_metric()
+            lat.symp(4, dt, nsteps)
+            got[prec] = lat.get_gw()
+    sim.set_state(fld, fldp, 1.0, 0.0)
+    sim.gwu[...] = u
+    sim.gwp[...] = pu
+    sim.calc_metric()
+    sim.symp(4, dt, nsteps)
+    assert rel(sim.gwp, pu) > 1e-3  # the sourced part is visible
+    for a, b in zip(got[gpu.F64], (sim.gwu, sim.gwp)):
+        for q in range(6):
+            assert rel(a[q], b[q]) < 1e-11, q
+    for a, b in zip(got[gpu.MIXED], (sim.gwu, sim.gwp)):
+        for q in range(6):
+            assert rel(a[q], b[q]) < 1e-5, q
+
+
 @pytest.mark.parametrize("lap", ["spectral", "fd7"])
 def test_gw_split_pieces_match_oracle(gpu, lap):
     """Single split calls (drift, grav, kick) and symp_o2step with u_ij."""
