@@ -154,6 +154,81 @@ def test_fd_tiles_match_oracle(gpu, shape, stencil):
         assert abs(g[4][k] - o[4][k]) <= 1e-11 * abs(o[4][k]), k
 
 
+@pytest.mark.parametrize("shape", [(512, 256, 48), (512, 512, 16)])
+@pytest.mark.parametrize("stencil", [(-6.0, 1.0, 0.0, 0.0, 1.0), (-128.0, 14.0, 3.0, 1.0, 30.0)])
+@pytest.mark.parametrize("nfld", [1, 2])
+def test_fd_partial_chunks_match_oracle(gpu, shape, stencil, nfld):
+    """Finite-difference kicks in chunks of 32 planes (boxes with enough tiles for
+    them) whose last chunk is shorter: 16 of 48 planes, and the only one 16 of
+    16.  A drift sweep with a kick in place, and fused sweeps."""
+    print("case fd partial chunks", shape, stencil, nfld, flush=True)
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nfld + nz)
+    fld = 1e-3 * rng.standard_normal((nfld, nz, ny, nx))
+    fldp = 1e-3 * rng.standard_normal((nfld, nz, ny, nx))
+    fld[0] += PHI0_C
+    fldp[0] += DPHI0_C
+    tv, model, par = (O.COSMIC, O.MODEL_TWOFIELD, (1.0, 2.5e5)) if nfld == 2 else (O.CONFORMAL, O.MODEL_PHI4, (1.0,))
+    plan = [("symp", (2, 1e-3, 2)), ("symp", (2, 1e-3, 1))]
+    g, o = run_pair(gpu, shape, 0.05 * nx, nfld, tv, model, par, O.LAP_STENCIL, stencil, fld, fldp, plan)
+    assert rel(g[0], o[0]) < 1e-12 and rel(g[1], o[1]) < 1e-12
+    for k in ("rho", "ke", "pe", "ge"):
+        assert abs(g[4][k] - o[4][k]) <= 1e-11 * abs(o[4][k]), k
+
+
+class _Device:
+    """n reals at a device address, for torch.as_tensor."""
+
+    def __init__(self, ptr, shape, dtype):
+        self.__cuda_array_interface__ = dict(data=(ptr, False), shape=shape, typestr=np.dtype(dtype).str, version=3)
+
+
+@pytest.mark.parametrize("precision,shape,n", [("f64", (1024, 1024, 192), 64), ("mixed", (1024, 512, 1024), 64),
+                                               ("f64", (512, 512, 48), 16), ("mixed", (512, 512, 48), 16)])
+@pytest.mark.parametrize("stencil", [(-6.0, 1.0, 0.0, 0.0, 1.0), (-128.0, 14.0, 3.0, 1.0, 30.0)])
+def test_fd_large_lattices_match_their_period(gpu, precision, shape, n, stencil):
+    """A state with the period of an n^3 lattice against that lattice, three
+    leapfrog steps (an unfused and two fused kicks): lattices with more tiles and
+    chunks than the 8192 blocks of a kick, so that blocks take a second item,
+    and chunks of 32 planes of which the last is half full.  Sites see the same
+    operations with background coefficients from sums in another order: a few
+    roundings of the largest value."""
+    import torch
+
+    print("case fd period", precision, shape, n, stencil, flush=True)
+    tile = {"f64": 64 * 8 * 32, "mixed": 64 * 16 * 32}[precision]  # sites of an item
+    assert n == 16 or shape[0] * shape[1] * shape[2] // tile > 8192
+    dtype = np.float64 if precision == "f64" else np.float32
+    kw = dict(nfld=1, precision=gpu.F64 if precision == "f64" else gpu.MIXED, model=gpu.MODEL_PHI4,
+              model_params=(0.7,), laplacian=gpu.LAP_STENCIL, stencil=stencil)
+    rng = np.random.default_rng(8)
+    init = [torch.from_numpy(rng.standard_normal((n, n, n)).astype(dtype)).cuda() for _ in range(2)]
+    reps = tuple(shape[2 - d] // n for d in range(3))
+
+    def view(lat):
+        return [torch.as_tensor(_Device(ptr, (lat.nz, lat.ny, lat.nx), dtype), device="cuda")
+                for ptr in lat.device_state()]
+
+    with gpu.Lattice(n, length=0.125 * n, **kw) as small, gpu.Lattice(shape, length=0.125 * shape[0], **kw) as big:
+        for lat in (small, big):
+            lat.set_scalars(1.0, 0.0)
+            for v, x in zip(view(lat), init):
+                v.copy_(x if lat is small else x.repeat(reps))
+            torch.cuda.synchronize()
+            lat.calc_metric()
+            lat.symp2(2e-3, 3)
+            lat.synchronize()
+        eps = float(np.finfo(dtype).eps)
+        y = [lat.scalars for lat in (small, big)]
+        assert abs(y[0][0] - y[1][0]) <= 1e-13 * abs(y[0][0]) and abs(y[0][1] - y[1][1]) <= 1e-12 * abs(y[0][1])
+        for a, b in zip(view(small), view(big)):
+            top, worst = float(a.abs().max()), 0.0
+            for k in range(0, shape[2], n):
+                worst = max(worst, float((b[k:k + n] - a.repeat(1, reps[1], reps[2])).abs().max()))
+            print("largest difference", worst, "of", top, flush=True)
+            assert worst <= 16 * eps * top
+
+
 @pytest.mark.parametrize("shape", [(8, 16, 32), (16, 8, 48), (48, 32, 8), (64, 16, 96), (32, 192, 16), (192, 48, 8),
                                    (16, 256, 8), (256, 8, 16), (8, 8, 512), (16, 512, 8)])
 @pytest.mark.parametrize("nfld", [1, 2])
