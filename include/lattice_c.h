@@ -78,7 +78,14 @@ typedef struct lat_config {
     int reserved[4];
 } lat_config;
 
-/* ---- lifetime ---- */
+/* ---- lifetime ----
+ * A context takes its device memory at creation: the state, and for the
+ * spectral Laplacian (and FP64) the k-space arrays.  Finite-difference contexts
+ * without metric perturbations also take second state arrays of the same size,
+ * for drift and kick in one sweep, if more than half of the device's memory is
+ * free after them; else the drift is a sweep of its own.  64 KB of pinned host memory
+ * per context, and 8 MB at the first host array of 256 KB or more, carry
+ * transfers; lat_destroy gives all of it back. */
 int  lat_create(const lat_config *cfg, lat_ctx **out);
 void lat_destroy(lat_ctx *ctx);
 
@@ -138,8 +145,8 @@ int  lat_set_tuning(lat_ctx *ctx, const int *in);   /* in[4] of 0/1, as lat_tuni
  * x R2C of a 1024^3 mixed state ran 3.07-3.55 ms per launch over four
  * allocations in one process, each keeping its figure; the distance between
  * the field and momentum arrays sets it).  Allocates candidates - 1 further
- * sets of these arrays (fewer if memory runs out), each with a spacer of its
- * own size between its field and momentum arrays, times the sweeps of one
+ * sets of these arrays (with a finite-difference context's second state
+ * arrays; fewer sets if memory runs out), each with a spacer of its own size between its field and momentum arrays, times the sweeps of one
  * force evaluation on each and on the context's own (on copies of the
  * state), keeps the fastest set holding the state unchanged and frees the
  * others.  candidates in 1..8; ms_out (nullable) receives `candidates`
@@ -157,15 +164,17 @@ int  lat_place_tune(lat_ctx *ctx, int candidates, float *ms_out);
  * lat_ensemble_symp advances every member of class k by nsteps steps of
  * dt[k]: the first call with given (order, nsteps, dt) is captured into a
  * hipGraph, later calls replay it.  Two launch modes: every FFT sweep of a
- * force evaluation as ONE launch covering all classes in lockstep (up to 4
- * classes of spectral, cubic lattices of 16, 32, 48, 64, 96, 128, 192 or 256
+ * force evaluation as ONE launch covering all classes in lockstep (x and y as
+ * one for each kind of sweep: planes of up to 32 and of 48 to 128 per side,
+ * separate x and y sweeps above; up to 4 classes of spectral, cubic lattices of 16, 32, 48, 64, 96, 128, 192 or 256
  * sites per side), or one launch per sweep per class.  At creation the
  * autotuner times both and keeps the faster, and each class's arrays are
  * put on the fastest of eight HBM placements (as lat_place_tune does for a
- * single context).  lat_ensemble_single_launch(ens,
- * 1 or 0) forces a mode, (ens, -1) only queries; it returns 1 when the single
- * launch is in use (0 if not, or if the classes do not allow it).  Members
- * are addressed class-major through lat_ensemble_member views. */
+ * single context; four for classes with second state arrays).
+ * lat_ensemble_single_launch(ens, 1 or 0) forces a mode, (ens, -1) only
+ * queries; it returns 1 when the single launch is in use (0 if not, or if the
+ * classes do not allow it).  Members are addressed class-major through
+ * lat_ensemble_member views. */
 typedef struct lat_ensemble lat_ensemble;
 int  lat_ensemble_create(const lat_config *base, int nclass, const int *n, const int *count,
                          const double *len, const double *model_params, lat_ensemble **out);

@@ -107,7 +107,8 @@ struct Prof {
 // a ring for whole arrays, allocated at the first such copy.  The runtime's own
 // copies of 16.8 MB run at 17 GB/s to pageable memory and 36 GB/s from it;
 // between the device and pinned memory they run at 55 GB/s, and one CPU thread
-// drains the ring at about 30 GB/s, so large arrays take several.  @STAGE_FIGS@
+// drains the ring at about 30 GB/s, so large arrays take several: the host
+// Laplacian of 128^3 (16.8 MB each way) 2.22 -> 1.00 ms.
 //
 // Views of a batch may be driven by a host thread each, as far as they do not
 // share device scratch (scalars, state, steps): the scalars' place and the

@@ -700,10 +700,11 @@ __global__ __launch_bounds__(TPB) void k_fd_kick(const T *f, const T *p, T *fo, 
 // (neighbouring lanes read neighbouring vectors; a row's tiles are equal, so no
 // lane is masked along x); as many rows as 256 threads hold, spread evenly
 // over ny; planes per chunk: 32 (two of 34 loaded planes are halo), halved down
-// to 4 until there are 2 blocks per CU (256^3 mixed, per kick with three lattices
-// in turn: 139 us; until 1 / 4 / 8 per CU: 140, 147,
-// 161 us; 192 x 96 x 128 FP64 27-point: 48 us, 45, 56, 56).  The shape depends on the lattice only,
-// so batch members run exactly as single contexts.
+// to 4 until there are 2 blocks per CU.  Per kick with three lattices in turn, until
+// 1 / 2 / 4 / 8 blocks per CU: 256^3 mixed 140, 139, 147, 161 us; 192 x 96 x 128 FP64
+// 27-point 45, 48, 56, 56: more than 2 lose to the chunks' halo planes, 1 against
+// 2 is open (the box gains 6 % with 1).  The shape depends on the lattice only, so
+// batch members run exactly as single contexts.
 struct FdShape {
     int LX, TY, KC, items;
     size_t lds;

@@ -12,7 +12,10 @@
 // fields 41.5 -> 18.5 / 27.8 -> 15.9 us, 48^3 73 -> 28 / 27 -> 16, 64^3 FP64 one field
 // 38.5 -> 27.3 / 21.9 -> 16.0, 96^3 mixed 83 -> 50 / 35 -> 23, 128^3 mixed 90 -> 66 /
 // 57 -> 41, 128^3 FP64 one field 86 -> 70 / 56 -> 37, two fields (forward only)
-// 137 -> 115 / 102 -> 91.
+// 137 -> 115 / 102 -> 91.  One workgroup per plane leaves CUs idle where nz is small, and
+// is still the faster way: of the boxes nx = ny = 16 .. 128, nz = 8 .. 256, mixed and
+// FP64, one and two fields, the least gain is 128 x 128 x 8 FP64 one field, 56.3 ->
+// 47.2 / 26.1 -> 19.6 us; 128 x 128 x 256 mixed 154 -> 91 / 108 -> 75.
 #pragma once
 #include "sweeps.h"
 

@@ -314,8 +314,8 @@ __device__ __forceinline__ void x_r2c_body(T *__restrict__ f, const T *__restric
     // AHEAD: a thread's vectors of phi and pi all in flight before the first is used,
     // the twiddle table's loads ahead of them, so that a workgroup starts with one
     // memory latency instead of one for the table and one per vector.  FP32, per
-    // kick: 1024^3 27.0 -> 26.3 ms (one lattice), 25.5 -> 25.1 (three in turn);
-    // 256^3 398 -> 385 us, 414 -> 411.  FP64 has twice the vectors per thread in
+    // kick: 1024^3 25.5 -> 25.1 ms (three lattices in turn); 256^3 398 -> 385 us (one
+    // lattice), 414 -> 411.  FP64 has twice the vectors per thread in
     // flight anyway and loses 1 % (192^3 334 -> 339 us, 256x192x128 293 -> 297).
     constexpr bool AHEAD = sizeof(T) == 4;
     TwFill<T, N, TPB, TWL> twf;
@@ -467,8 +467,10 @@ __device__ __forceinline__ void x_r2c_body(T *__restrict__ f, const T *__restric
 // written, never one element of one.  Per kick, three lattices in turn: 256^3 FP64
 // 889 -> 843 us, 192^3 mixed 181 -> 175, 128^3 mixed 37.9 -> 37.0, 256^3 mixed 415 -> 411,
 // 512^3 FP64 6.87 -> 6.33 ms (one).  In longer columns a tile over two planes costs what
-// the short tile did, and tiles stay within their rows, with the padding: 1024^3
-// mixed 27.1 -> 26.5 ms (27.2 across rows), 512^3 mixed 3.40 -> 3.33 (3.43).
+// the short tile did, and tiles stay within their rows, with the padding: 512^3
+// mixed 3.40 -> 3.33 ms (3.43 across rows), 1024^3 mixed 27.2 across rows, 26.5 within.
+// A 1024^3 mixed step, timed in turn before this and the loads ahead of the x R2C
+// and after both: 82.3 -> 81.4 ms.
 template <typename T, int N>
 constexpr bool flat_tiles() { return N <= 256 || (N == 512 && sizeof(T) == 8); }
 // tiles of TC columns per array of n_other rows of pitch P
