@@ -166,9 +166,9 @@ int  lat_place_tune(lat_ctx *ctx, int candidates, float *ms_out);
  * hipGraph, later calls replay it.  Two launch modes: every FFT sweep of a
  * force evaluation as ONE launch covering all classes in lockstep (x and y as
  * one for each kind of sweep: planes of up to 32 and of 48 to 128 per side,
- * separate x and y sweeps above; up to 4 classes of spectral, cubic lattices of 16, 32, 48, 64, 96, 128, 192 or 256
- * sites per side), or one launch per sweep per class.  At creation the
- * autotuner times both and keeps the faster, and each class's arrays are
+ * separate x and y sweeps above; up to 4 classes of spectral, cubic lattices
+ * of 16, 32, 48, 64, 96, 128, 192 or 256 sites per side), or one launch per
+ * sweep per class.  At creation the autotuner times both and keeps the faster, and each class's arrays are
  * put on the fastest of eight HBM placements (as lat_place_tune does for a
  * single context; four for classes with second state arrays).
  * lat_ensemble_single_launch(ens, 1 or 0) forces a mode, (ens, -1) only
