@@ -123,6 +123,8 @@ def roofline(prof, n, nf, w):
         b = algorithmic_bytes(stage, n, nf, w)
         if b is None or cnt == 0:
             continue
+        if stage == "x_r2c" and prof["y_fwd"][1] == 0:
+            b *= nf  # plane sweeps (up to 128 per side): all fields and their y pass in one launch
         if best is None or ms > best[1]:
             best = (stage, ms, cnt, b)
     if best is None:

@@ -425,15 +425,17 @@ int  lat_device_state(lat_ctx *ctx, void **fld, void **fldp);
  *      wall-clock times at evolve_spectral.f90:79,99) ---- */
 enum lat_stage {
     LAT_ST_X_R2C = 0, /* x-direction R2C (drift fused)            */
-    LAT_ST_Y_FWD,     /* y forward column FFT                      */
+    LAT_ST_Y_FWD,     /* y forward column FFT (plane sweeps, nx = ny up to
+                         128: within X_R2C, one launch for all fields)  */
     LAT_ST_Z_LAP,     /* z forward * -k^2 * z inverse              */
-    LAT_ST_Y_INV,     /* y inverse column FFT                      */
+    LAT_ST_Y_INV,     /* y inverse column FFT (plane sweeps: within X_C2R) */
     LAT_ST_X_C2R,     /* x-direction C2R + kick + reductions       */
     LAT_ST_SCALAR,    /* background scalar update                  */
     LAT_ST_DRIFT,     /* standalone drift sweep                    */
-    LAT_ST_STENCIL,   /* FD stencil + kick                         */
+    LAT_ST_STENCIL,   /* FD stencil + kick (fused: with the drift) */
     LAT_ST_REDUCE,    /* state reductions                          */
-    LAT_ST_GW_SRC,    /* u_ij source S_ij = sum d_i phi d_j phi     */
+    LAT_ST_GW_SRC,    /* u_ij source S_ij = sum d_i phi d_j phi of
+                         lat_gw_source (spectral kicks: within X_C2R)   */
     LAT_ST_SEP_X,     /* separable Laplacian: drift + D_xx          */
     LAT_ST_SEP_Y,     /* separable Laplacian: lap += D_yy           */
     LAT_ST_SEP_Z,     /* separable Laplacian: D_zz + kick + reductions */

@@ -34,3 +34,20 @@ def test_algorithmic_bytes_match_the_array_sizes():
             assert bench.algorithmic_bytes("x_c2r", n, nf, w) == nf * (half + 3 * real)
     # the figure quoted for the mixed 1024^3 x R2C launch
     assert bench.algorithmic_bytes("x_r2c", 1024, nf, 4) == 17188257792
+
+
+def test_roofline_counts_all_fields_of_a_plane_sweep():
+    """Lattices that take the x and y passes plane by plane time no y stage, and
+    one forward launch carries every field."""
+    sys.path.insert(0, ROOT)
+    import bench
+
+    n, nf, w = 128, 2, 4
+    real, half = n ** 3 * w, n * n * (n // 2 + 1) * 2 * w
+    none = (0.0, 0)
+    planes = {"x_r2c": (6.0, 3), "y_fwd": none, "z_lap": (2.0, 3), "y_inv": none, "x_c2r": (5.0, 3)}
+    r = bench.roofline(planes, n, nf, w)
+    assert r["kernel"] == "x_r2c" and r["algorithmic_bytes_per_launch"] == nf * (3 * real + half)
+    sweeps = dict(planes, x_r2c=(6.0, 6), y_fwd=(2.0, 3), y_inv=(2.0, 3))
+    r = bench.roofline(sweeps, n, nf, w)
+    assert r["kernel"] == "x_r2c" and r["algorithmic_bytes_per_launch"] == 3 * real + half
