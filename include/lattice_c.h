@@ -85,7 +85,8 @@ typedef struct lat_config {
  * for drift and kick in one sweep, if more than half of the device's memory is
  * free after them; else the drift is a sweep of its own.  64 KB of pinned host memory
  * per context, and 8 MB at the first host array of 256 KB or more, carry
- * transfers; lat_destroy gives all of it back. */
+ * transfers (where pinned memory is refused, the runtime's own copies do);
+ * lat_destroy gives all of it back. */
 int  lat_create(const lat_config *cfg, lat_ctx **out);
 void lat_destroy(lat_ctx *ctx);
 

@@ -67,20 +67,38 @@ static int sync(Ctx &c)
 }
 
 // ---------------------------------------------------------------- host copies
-static int stage_ring(Ctx &c)
+// Pinned memory may not be had (a limit on locked memory): the small area is
+// then ordinary memory, and whole arrays go through the runtime's own copies.
+static bool stage_ring(HostStage &h)
 {
-    HostStage &h = *c.stage;
-    if (h.ring) return 0;
-    for (hipEvent_t &e : h.ev)
-        if (!e) LAT_HIP(&c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    LAT_HIP(&c, hipHostMalloc((void **)&h.ring, HostStage::SLOT * HostStage::SLOTS, hipHostMallocDefault));
-    return 0;
+    if (h.ring || h.no_ring) return h.ring != nullptr;
+    bool ok = true;
+    for (hipEvent_t &e : h.ev) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+    if (ok && hipHostMalloc((void **)&h.ring, HostStage::SLOT * HostStage::SLOTS, hipHostMallocDefault) != hipSuccess)
+        h.ring = nullptr;
+    if (!h.ring) {
+        (void)hipGetLastError();
+        h.no_ring = true;
+    }
+    return h.ring != nullptr;
+}
+
+static HostStage *stage_new()
+{
+    HostStage *h = new HostStage();
+    h->pinned = hipHostMalloc((void **)&h->small, HostStage::SMALL, hipHostMallocDefault) == hipSuccess;
+    if (!h->pinned) {
+        (void)hipGetLastError();
+        h->small = new char[HostStage::SMALL];
+    }
+    return h;
 }
 
 static void stage_free(HostStage *h)
 {
     if (!h) return;
-    if (h->small) (void)hipHostFree(h->small);
+    if (h->pinned) (void)hipHostFree(h->small);
+    else delete[] h->small;
     if (h->ring) (void)hipHostFree(h->ring);
     for (hipEvent_t e : h->ev)
         if (e) (void)hipEventDestroy(e);
@@ -136,16 +154,17 @@ static int stage_copy(Ctx &c, bool to_host, char *dev, size_t dpitch, char *host
     if (!width || !rows) return 0;
     HostStage &h = *c.stage;
     const std::lock_guard<std::mutex> hold(h.ring_lock);
-    if (!h.ring && width * rows < (size_t)256 << 10) {
+    if ((!h.ring && width * rows < (size_t)256 << 10) || !stage_ring(h)) {
         // a small lattice: not worth the ring's allocation (70 us)
-        if (to_host)
+        if (rows == 1 || width == dpitch) // (a pitch is below 2 GiB)
+            LAT_HIP(&c, hipMemcpyAsync(to_host ? host : dev, to_host ? dev : host, width * rows,
+                                       to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, c.stream));
+        else if (to_host)
             LAT_HIP(&c, hipMemcpy2DAsync(host, width, dev, dpitch, width, rows, hipMemcpyDeviceToHost, c.stream));
         else
             LAT_HIP(&c, hipMemcpy2DAsync(dev, dpitch, host, width, width, rows, hipMemcpyHostToDevice, c.stream));
         return sync(c);
     }
-    int rc = stage_ring(c);
-    if (rc) return rc;
     const Chunks ck(width, rows);
     // a thread costs about 20 us to start: from 8 chunks on
     const size_t T = ck.count >= 8 ? HostStage::THREADS : 1;
@@ -890,11 +909,7 @@ static int create_ctx(const lat_config *cfg, int B, const double *mparams, lat_c
     int rc = 0;
     hipError_t e = hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking);
     if (e != hipSuccess) { delete h; return -3; }
-    c.stage = new HostStage();
-    if (hipHostMalloc((void **)&c.stage->small, HostStage::SMALL, hipHostMallocDefault) != hipSuccess) {
-        lat_destroy(h);
-        return -3;
-    }
+    c.stage = stage_new();
     const size_t es = elem_size(c);
     rc |= ensure(c, &c.fld, es * B * c.ms.f, "hipMalloc fld");
     rc |= ensure(c, &c.fldp, es * B * c.ms.f, "hipMalloc fldp");

@@ -120,6 +120,8 @@ struct HostStage {
     static constexpr int THREADS = 4, SLOTS = 2 * THREADS; // two slots per copying thread
     char *small = nullptr;
     char *ring = nullptr;
+    bool pinned = false;  // the small area is pinned memory
+    bool no_ring = false; // pinned memory for the ring was refused
     hipEvent_t ev[SLOTS] = {};
     bool used[SLOTS] = {}; // a copy of the slot, either way, that nobody has waited for yet
 };

@@ -1,5 +1,9 @@
 """GPU parity of the single operators (FFT, Laplacians, spectra) against the
 CPU oracle and numpy.  Calls go through the C ABI (lattice_amd -> liblattice_amd.so)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -251,3 +255,63 @@ def test_laplacian_out_of_place_equals_in_place(gpu, n):
         g = f.copy()
         assert gpu.lib().lat_laplacian_3d(lat._h, n, n, n, gpu._p(g), ctypes.c_double(lat.dk)) == 0
     assert np.array_equal(f, keep) and np.array_equal(out, g)
+
+
+_NO_PINNED = r"""
+import ctypes, sys
+import numpy as np
+shim, pkg, out, granted = sys.argv[1:]
+if shim:
+    S = ctypes.CDLL(shim, mode=ctypes.RTLD_GLOBAL)
+    S.grant(int(granted))
+sys.path.insert(0, pkg)
+import lattice_amd as la
+rng = np.random.default_rng(4)
+f, p = rng.standard_normal((2, 2, 48, 64, 32))
+res = []
+for prec in (la.F64, la.MIXED):
+    with la.Lattice((32, 64, 48), nfld=2, length=3.0, precision=prec) as lat:
+        lat.set_state(f, p, 1.0, 0.0)
+        lat.calc_metric()
+        lat.symp4(1e-4, 1)
+        st = lat.get_state()
+        res += [st[0], st[1], np.array(st[2:]), lat.output_spectra(0), lat.laplacian_3d(f[0]), lat.fft_r2c_3d(p[0])]
+if shim:
+    print("refused", S.refused())
+np.savez(out, *res)
+"""
+
+
+@pytest.mark.parametrize("granted", [0, 1])
+def test_host_calls_without_pinned_memory(gpu, tmp_path, granted):
+    """Where the runtime refuses pinned memory (all of it; all but the first
+    piece, so that the copy ring is refused), host arrays, scalars and spectra go
+    through ordinary copies with the same results.  The refusal comes from a
+    hipHostMalloc that a process of its own loads before the library."""
+    print("case no pinned memory", granted, flush=True)
+    shim = tmp_path / "refuse.so"
+    src = tmp_path / "refuse.c"
+    src.write_text(
+        "#include <dlfcn.h>\n#include <stddef.h>\n"
+        "static int left, refused_;\n"
+        "void grant(int n) { left = n; }\nint refused(void) { return refused_; }\n"
+        "int hipHostMalloc(void **p, size_t n, unsigned f)\n{\n"
+        "    static int (*next)(void **, size_t, unsigned);\n"
+        "    if (left-- <= 0) { ++refused_; *p = NULL; return 2; }\n"  # hipErrorOutOfMemory
+        "    if (!next) next = (int (*)(void **, size_t, unsigned))dlsym(dlopen(\"libamdhip64.so.7\", RTLD_NOW), "
+        "\"hipHostMalloc\");\n"
+        "    return next(p, n, f);\n}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(shim), str(src), "-ldl"], check=True)
+    pkg = os.path.dirname(os.path.dirname(gpu.__file__))
+    out = []
+    for s in (str(shim), ""):
+        path = tmp_path / ("shim.npz" if s else "plain.npz")
+        r = subprocess.run([sys.executable, "-c", _NO_PINNED, s, pkg, str(path), str(granted)], capture_output=True,
+                           text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        if s:
+            assert int(r.stdout.split()[-1]) > 0  # the library did ask
+        out.append(np.load(path))
+    assert out[0].files == out[1].files and len(out[0].files) == 12
+    for k in out[0].files:
+        assert np.array_equal(out[0][k], out[1][k]), k
